@@ -184,7 +184,7 @@ __global__ void kb_set_mask_bit(uint8_t* __restrict__ flags, const T* __restrict
 // range of its pages) with the single-grid kernels' walk and per-point
 // bodies, called with the item's grid.
 template <int R, typename T, int S = IFACE_WENO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves<T>()))) kb_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) kb_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                        const T* __restrict__ fn, const uint8_t* __restrict__ flags,
                                                        IList il, BatchView B, int stage, int* __restrict__ over,
                                                        int* __restrict__ over_count, int seq, int niface)
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(256) kb_reinit_deferred(T* __restrict__ out, c
 // interface list (three lanes per point), the others take the z-march work
 // items; see k_extend_stage
 template <int R, typename T, int S = IFACE_WENO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves<T>()))) kb_extend_stage(T* __restrict__ out, const T* __restrict__ cs,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) kb_extend_stage(T* __restrict__ out, const T* __restrict__ cs,
                                                        const T* __restrict__ cn, const T* __restrict__ vx,
                                                        const T* __restrict__ vy, const T* __restrict__ vz,
                                                        IList il, const double* __restrict__ lcp,
@@ -494,7 +494,7 @@ __global__ void __launch_bounds__(256) kb_list_interp(double* __restrict__ cp, I
 // the same values line7 reads).  Each point reads cn only at itself, so out
 // may be cn.
 template <int R>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves<double>())))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves)))
 kb_eno2_extend_stage(double* __restrict__ out, const double* __restrict__ cs, const double* __restrict__ cn,
                      const double* __restrict__ vx, const double* __restrict__ vy, const double* __restrict__ vz,
                      const uint8_t* __restrict__ flags, IList il, const double* __restrict__ lcp, BatchView B,

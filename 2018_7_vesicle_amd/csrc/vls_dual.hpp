@@ -5,7 +5,7 @@
 // and its value part equals the double result bit for bit; the derivative
 // parts are the exact derivatives of that formula with the branches frozen.
 #pragma once
-#include <hip/hip_runtime.h>
+#include "vls_device.hpp"
 
 namespace vls {
 // own namespace: the double code of namespace vls keeps finding ::fma and
@@ -93,6 +93,17 @@ __device__ __forceinline__ Dual<N> operator/(const Dual<N>& a, const Dual<N>& b)
     const double ib = 1.0 / b.v;
 #pragma unroll
     for (int k = 0; k < N; ++k) r.d[k] = (a.d[k] - r.v * b.d[k]) * ib;
+    return r;
+}
+// quotients in the forms of vls_device.hpp
+template <int N>
+__device__ __forceinline__ Dual<N> quot(const Dual<N>& a, const Dual<N>& b)
+{
+    const RecipT<double> ib = recip(b.v);
+    Dual<N> r;
+    r.v = vls::quot(a.v, ib);
+#pragma unroll
+    for (int k = 0; k < N; ++k) r.d[k] = (a.d[k] - r.v * b.d[k]) * ib.y;
     return r;
 }
 // mixed forms with a constant
@@ -207,4 +218,27 @@ __device__ __forceinline__ Dual<N> sq(const Dual<N>& a)
 
 }  // namespace ad
 using ad::Dual;
+
+// a dual denominator and the reciprocal of its value
+template <int N>
+struct RecipT<Dual<N>> {
+    Dual<N> b;
+    double y;
+};
+namespace ad {
+template <int N>
+__device__ __forceinline__ RecipT<Dual<N>> recip(const Dual<N>& b)
+{
+    return RecipT<Dual<N>>{b, vls::recip(b.v).y};
+}
+template <int N>
+__device__ __forceinline__ Dual<N> quot(const Dual<N>& a, const RecipT<Dual<N>>& i)
+{
+    Dual<N> r;
+    r.v = vls::quot(a.v, RecipT<double>{i.b.v, i.y});
+#pragma unroll
+    for (int k = 0; k < N; ++k) r.d[k] = (a.d[k] - r.v * i.b.d[k]) * i.y;
+    return r;
+}
+}  // namespace ad
 }  // namespace vls

@@ -341,7 +341,7 @@ __global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, cons
 // other slot is cleared here for the next stage.  FP32 evaluates such a
 // point in the bulk (defers_crossings) and has no launch 2.
 template <int R, typename T, int S = IFACE_WENO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves<T>()))) k_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                       const T* __restrict__ fn, const uint8_t* __restrict__ flags,
                                                       IList il, Box b, Inv invs, int stage, int* __restrict__ over,
                                                       int* __restrict__ over_count, int seq, int depth, int niface)
@@ -726,7 +726,7 @@ __global__ void __launch_bounds__(256) k_extend_step(double* __restrict__ step, 
 // chains (the nonuniform WENO divides ~30 times) then run beside the bulk
 // blocks instead of after them.  The two sets of points are disjoint.
 template <int R, typename T, int S = IFACE_WENO>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stage_waves<T>()))) k_extend_stage(T* __restrict__ out, const T* __restrict__ cs,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_extend_stage(T* __restrict__ out, const T* __restrict__ cs,
                                                       const T* __restrict__ cn, const T* __restrict__ vx,
                                                       const T* __restrict__ vy, const T* __restrict__ vz,
                                                       IList il, const double* __restrict__ lcp,

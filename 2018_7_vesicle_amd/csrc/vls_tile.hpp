@@ -552,14 +552,12 @@ __device__ __forceinline__ void block_reduce_store(KSum (&k)[NQ], double* __rest
 // result bit for bit either way.
 // ---------------------------------------------------------------------------
 
-// Waves per SIMD the fused stage kernels are compiled for: their bulk
-// z-march fits 128 VGPRs in FP64 and 96 in FP32; the interface lanes (the
-// nonuniform WENO, inlined) are fitted into the same budget.
-template <typename T>
-constexpr int stage_waves()
-{
-    return sizeof(T) == 8 ? 4 : 5;
-}
+// Waves per SIMD the fused stage kernels are compiled for (128 VGPRs): the
+// FP64 bulk z-march fits them, and so do the interface lanes (the nonuniform
+// WENO, inlined).  The FP32 bulk needs 92 VGPRs, but at 5 waves (96) the
+// interface lanes spill 100 bytes: the batch of 96 FP32 grids of 32..96 runs
+// 58.9 ms a step with 5 waves and 56.6 ms with 4, 256^3 is equal.
+constexpr int kStageWaves = 4;
 
 // ---------------------------------------------------------------------------
 // z-marching walk (single grid): a block takes one tile column (TR rows x TC
@@ -791,7 +789,7 @@ __device__ __forceinline__ ReinitLane reinit_iface_lane(const T* __restrict__ fs
     }
     if (q.dt >= 0) {
         double v[7], fo, bk;
-        line7(fs, r, c, p, a, b, v);
+        line7_lane(fs, r, c, p, a, b, v);
         if constexpr (SCHEME == IFACE_CUBIC) reinit_axis_cubic(fo, bk, v, r1, l1, sp[a], inv.jd[a]);
         else reinit_axis<true>(fo, bk, v, r1, l1, sp[a], inv.jd[a]);
         q.m = godunov_axis(q.inside, bk, fo);
@@ -858,7 +856,7 @@ __device__ __forceinline__ ExtendLane extend_iface_lane(const T* __restrict__ cs
         int r, c, p;
         coords_of(b, ind, r, c, p);
         double v[7];
-        line7(cs, r, c, p, a, b, v);
+        line7_lane(cs, r, c, p, a, b, v);
         const double vel = lv[(size_t)a * il.cap + slot];
         const double r1 = il.dist[(size_t)(2 * a) * il.cap + slot];
         const double l1 = il.dist[(size_t)(2 * a + 1) * il.cap + slot];

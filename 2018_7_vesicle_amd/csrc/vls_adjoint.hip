@@ -12,9 +12,11 @@
 // every branch (upwind side, sign-change test, Godunov selection, frozen
 // points) is the one the forward pass took, and stores, per point, the 21
 // derivatives of out_i along its three lines (rows a*7+k, a = x,y,z, k =
-// offset+3) and the parameter derivatives.  The adjoint sweep gathers the
-// transposed stencil (deterministic: each output point sums its own
-// contributions in a fixed order); the tangent sweep applies it.
+// offset+3), for the adjoint times lam_i; the parameter derivatives go to
+// their gradients at once in the adjoint and to memory in the tangent.  The
+// adjoint sweep gathers the transposed stencil (deterministic: each output
+// point sums its own contributions in a fixed order); the tangent sweep
+// applies it.
 //
 // The subcell distances of the reinitialization depend on its initial field
 // F0 through the root of the quintic through six values (six_distance,
@@ -46,57 +48,174 @@ __device__ __forceinline__ idx_t shifted(const Box& b, int r, int c, int p, int 
 __device__ __forceinline__ void point_coords(const Box& b, idx_t i, int& r, int& c, int& p) { coords_of(b, i, r, c, p); }
 
 // ---------------------------------------------------------------------------
-// advection stage Jacobian: J (21 rows of n), JU (3 rows of n): d out_i / d u_a,i
+// advection stage Jacobian, a wave per axis over 64 points.  Tangent (lam
+// null): J (21 rows of n) and U[a] = d out_i / d u_a,i.  Adjoint: J times
+// lam_i, and U[a] += d out_i / d u_a,i lam_i (the velocity gradient).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) ka_advect_jac(double* __restrict__ J, double* __restrict__ JU,
+// Derivatives of the uniform WENO5 derivatives of a line.  The correction Q
+// depends on four second differences (Dual<4>); the seven line values enter
+// through the second differences D_j = p_j - 2 p_{j+1} + p_{j+2} and the central
+// part C = p_1 - p_5 + 8 (p_4 - p_2), whose derivatives are constants
+// (line_row).  Carrying the seven values through Q took half as many
+// instructions again.
+// Q(d[i0], d[i1], d2, d[i3]) of the back (0, 1, 3) or fore (4, 3, 1) side
+__device__ __forceinline__ Dual<4> jp_q_dual(const JPcd<double>& m, bool fore, double e)
+{
+    return jp_q(ad::dvar<4>(fore ? m.d[4] : m.d[0], 0), ad::dvar<4>(fore ? m.d[3] : m.d[1], 1),
+                ad::dvar<4>(m.d[2], 2), ad::dvar<4>(fore ? m.d[1] : m.d[3], 3), e);
+}
+// row k of sc * C + sum_j ed[j] D_j
+__device__ __forceinline__ double line_row(int k, double sc, const double ed[5])
+{
+    const double c = k == 1 ? 1.0 : (k == 5 ? -1.0 : (k == 4 ? 8.0 : (k == 2 ? -8.0 : 0.0)));
+    double w = c * sc;
+    if (k < 5) w += ed[k];
+    if (k >= 1 && k < 6) w -= 2.0 * ed[k - 1];
+    if (k >= 2) w += ed[k - 2];
+    return w;
+}
+
+struct Grad3 {
+    double* g[3];
+};
+
+__global__ void __launch_bounds__(192) ka_advect_jac(double* __restrict__ J, Grad3 U, const double* __restrict__ lam,
                                                      const double* __restrict__ fs, const double* __restrict__ vx,
                                                      const double* __restrict__ vy, const double* __restrict__ vz,
                                                      double dt, Box b, Inv inv, int stage)
 {
     const idx_t n = (idx_t)b.rows * b.cols * b.pges;
-    const idx_t i = (idx_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int a = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const idx_t i = (idx_t)blockIdx.x * 64 + (threadIdx.x & 63);
     if (i >= n) return;
     int r, c, p;
     point_coords(b, i, r, c, p);
     const double cs = stage_c(stage);
-    const double vel[3] = {vx[i], vy[i], vz[i]};
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) {
-        double v[7];
-        line7(fs, r, c, p, a, b, v);
-        D8 q[7];
+    const double vel = (a == 0 ? vx : (a == 1 ? vy : vz))[i];
+    double v[7];
+    line7(fs, r, c, p, a, b, v);
+    // the term of axis a: coef(u_a) * D_a (upwind_axis), D = (C -+ Q) k
+    const JPd jp = inv.jd[a];
+    const JPcd<double> m = jp_centre(v);
+    const bool fore = vel < 0;
+    const Dual<4> q = jp_q_dual(m, fore, jp.e);
+    const double d = (fore ? m.c + q.v : m.c - q.v) * jp.k;
+    const double li = lam ? lam[i] : 1.0;
+    // out = c (fs - dt * sum_a t_a) + e fn
+    const double w0 = -cs * dt * (fore ? vel : dmax(0.0, vel)) * jp.k, sq = fore ? w0 : -w0;
+    const double ed[5] = {fore ? 0.0 : sq * q.d[0], sq * (fore ? q.d[3] : q.d[1]), sq * q.d[2],
+                          sq * (fore ? q.d[1] : q.d[3]), fore ? sq * q.d[0] : 0.0};
 #pragma unroll
-        for (int k = 0; k < 7; ++k) q[k] = ad::dvar<8>(v[k], k);
-        // the term of axis a: coef(u_a) * D_a (upwind_axis), u_a is input 7
-        const D8 t = upwind_axis(D8(0.0), ad::dvar<8>(vel[a], 7), q, inv.jd[a]);
-#pragma unroll
-        for (int k = 0; k < 7; ++k) {
-            // out = c (fs - dt * sum_a t_a) + e fn
-            double j = -cs * dt * t.d[k];
-            if (a == 0 && k == 3) j += cs;
-            J[(size_t)(a * 7 + k) * n + i] = j;
-        }
-        JU[(size_t)a * n + i] = -cs * dt * t.d[7];
+    for (int k = 0; k < 7; ++k) {
+        double w = line_row(k, w0, ed);
+        if (a == 0 && k == 3) w += cs;
+        J[(size_t)(a * 7 + k) * n + i] = w * li;
     }
+    const double ju = (vel < 0 || vel > 0) ? -cs * dt * d : 0.0;
+    U.g[a][i] = lam ? U.g[a][i] + ju * li : ju;
 }
 
 // ---------------------------------------------------------------------------
 // reinitialization stage Jacobian (re_step.cu:283-393 as the fused stage
-// kernels evaluate it).  Points without subcell distances: spacing
-// distances and the bulk time step, no parameter derivatives.  Listed points:
-// distances and time step from the list, and JP (7 rows of cap, list order):
-// d out / d (xpr, xpl, ypf, ypb, zpu, zpd, dt).
+// kernels evaluate it) in two launches.  The first takes the points without
+// subcell distances on the uniform WENO5 (spacing distances, the bulk time
+// step, no parameter derivatives) and appends those next to a sign change of
+// fs to `extra`, which the forward evaluates on the nonuniform form too; the
+// second takes the listed points and those.  Parameter derivatives of a
+// listed point, d out / d (xpr, xpl, ypf, ypb, zpu, zpd, dt), 7 rows of cap in
+// list order: tangent (lam null) JP, adjoint JP += derivative times lam_i.
+//
+// In both launches a block takes 64 points with one wave per axis; the values
+// of the three axes' pairs meet in LDS for the Godunov step, and each wave
+// writes its axis's rows.  In the second the 9 inputs of an axis (7 line
+// values, r1, l1) are three groups (blockIdx.y), so that the duals of the
+// nonuniform form stay in registers.  (With one lane per point the duals of 9
+// inputs and 3 axes spilled 2.9 KB a lane, and a list of a few thousand points
+// filled a few dozen CUs.  Measured on MI355X at 64^3:
+// 68 + 172 us -> 24 + 22 us; the first is bound by its FP64 arithmetic, the
+// second by the dependent chain of the nonuniform form.)
 // ---------------------------------------------------------------------------
-// axis pair (fore, back) on duals of the 7 line values (inputs 0..6) and
-// r1, l1 (inputs 7, 8), with reinit_axis's branch
-__device__ __forceinline__ void reinit_axis_dual(D9& fo, D9& bk, const double v[7], double r1, double l1, double ds,
-                                                 JPd jp)
+// the Godunov step's derivatives with respect to this axis's pair (d[0], d[1])
+// and dt (d[2]) from the six values of the pairs; dt < 0: frozen, step 0
+__device__ __forceinline__ Dual<3> godunov_dual(const double (&val6)[3][2][64], int lane, int a, bool inside, double dt)
 {
-    D9 q[7];
+    typedef Dual<3> D3;
+    D3 e[6];
 #pragma unroll
-    for (int k = 0; k < 7; ++k) q[k] = ad::dvar<9>(v[k], k);
+    for (int k = 0; k < 6; ++k) {
+        e[k] = D3(val6[k >> 1][k & 1][lane]);
+        if ((k >> 1) == a) e[k].d[k & 1] = 1.0;
+    }
+    return dt >= 0 ? godunov_step(inside, e[0], e[1], e[2], e[3], e[4], e[5], ad::dvar<3>(dt, 2)) : D3(0.0);
+}
+
+__global__ void __launch_bounds__(192)
+ka_reinit_jac_bulk(double* __restrict__ J, const double* __restrict__ lam, const double* __restrict__ fs,
+                   const uint8_t* __restrict__ flags, Box b, Inv inv, int stage, int* __restrict__ extra,
+                   int* __restrict__ extra_count, int seq)
+{
+    __shared__ double val6[3][2][64];
+    __shared__ unsigned long long crossing[3];
+    const idx_t n = (idx_t)b.rows * b.cols * b.pges;
+    const int lane = (int)(threadIdx.x & 63), a = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const idx_t i = (idx_t)blockIdx.x * 64 + lane;
+    if (blockIdx.x == 0 && threadIdx.x == 0) extra_count[(seq + 1) & 1] = 0;
+    const uint8_t fl = i < n ? flags[i] : (uint8_t)FLAG_SUBCELL;
+    const bool mine = !(fl & FLAG_SUBCELL);
+    Dual<4> qf(0.0), qb(0.0);
+    double fo = 0.0, bk = 0.0;
+    const JPd jp = inv.jd[a];
+    bool cross = false;
+    if (mine) {
+        int r, c, p;
+        point_coords(b, i, r, c, p);
+        double v[7];
+        line7(fs, r, c, p, a, b, v);
+        cross = sign_change3(v);
+        const JPcd<double> cd = jp_centre(v);
+        qb = jp_q_dual(cd, false, jp.e);
+        qf = jp_q_dual(cd, true, jp.e);
+        bk = (cd.c - qb.v) * jp.k;
+        fo = (cd.c + qf.v) * jp.k;
+    }
+    val6[a][0][lane] = fo;
+    val6[a][1][lane] = bk;
+    const unsigned long long m = __ballot(cross);
+    if (lane == 0) crossing[a] = m;
+    __syncthreads();
+    const bool any = ((crossing[0] | crossing[1] | crossing[2]) >> lane) & 1;
+    if (a == 0) wave_append(any, (int)i, extra, &extra_count[seq & 1]);
+    if (!mine || any) return;
+    const Dual<3> g = godunov_dual(val6, lane, a, (fl & FLAG_MASK) != 0, inv.dt_bulk);
+    const double cs = stage_c(stage), li = lam ? lam[i] : 1.0;
+    const double wf = -cs * g.d[0] * jp.k, wb = -cs * g.d[1] * jp.k;
+    const double ed[5] = {-wb * qb.d[0], wf * qf.d[3] - wb * qb.d[1], wf * qf.d[2] - wb * qb.d[2],
+                          wf * qf.d[1] - wb * qb.d[3], wf * qf.d[0]};
+#pragma unroll
+    for (int k = 0; k < 7; ++k) {
+        double w = line_row(k, wf + wb, ed);
+        if (k == 3 && a == 0) w += cs;
+        J[(size_t)(a * 7 + k) * n + i] = w * li;
+    }
+}
+
+// axis pair (fore, back) with reinit_axis's branch, on duals that carry the
+// derivatives with respect to M of its 9 inputs, the 7 line values (0..6), r1
+// and l1 (7, 8): inputs first .. first + M - 1
+template <int M>
+__device__ __forceinline__ void reinit_axis_dual(Dual<M>& fo, Dual<M>& bk, const double v[7], double r1, double l1,
+                                                 double ds, JPd jp, int first)
+{
+    Dual<M> q[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) {
+        q[k] = Dual<M>(k < 7 ? v[k] : (k == 7 ? r1 : l1));
+#pragma unroll
+        for (int m = 0; m < M; ++m) q[k].d[m] = (k == first + m) ? 1.0 : 0.0;
+    }
     if (v[2] * v[3] < 0 || v[3] * v[4] < 0) {
-        const PairT<D9> pr = weno_nonuniform_pair(q, ad::dvar<9>(r1, 7), ad::dvar<9>(l1, 8), ds, D9(0.0), D9(0.0));
+        const PairT<Dual<M>> pr = weno_nonuniform_pair_inl(q[0], q[1], q[2], q[3], q[4], q[5], q[6], q[7], q[8], ds,
+                                                           Dual<M>(0.0), Dual<M>(0.0));
         fo = pr.fore;
         bk = pr.back;
     } else {
@@ -104,124 +223,112 @@ __device__ __forceinline__ void reinit_axis_dual(D9& fo, D9& bk, const double v[
     }
 }
 
-// one point: fills its 21 J entries (and, when jp is not null, its 7
-// parameter derivatives); dt < 0 is a frozen point (step 0)
-__device__ __forceinline__ void reinit_point_jac(double* __restrict__ J, double* jp, idx_t n, idx_t i,
-                                                 const double* __restrict__ fs, const Box& b, const Inv& inv,
-                                                 const double r1[3], const double l1[3], double dt, bool inside,
-                                                 int stage)
-{
-    int r, c, p;
-    point_coords(b, i, r, c, p);
-    const double cs = stage_c(stage);
-    const double sp[3] = {b.dx, b.dy, b.dz};
-    if (!(dt >= 0)) {
-        for (int e = 0; e < 21; ++e) J[(size_t)e * n + i] = (e == 3) ? cs : 0.0;
-        if (jp)
-            for (int e = 0; e < 7; ++e) jp[e] = 0.0;
-        return;
-    }
-    D9 fo[3], bk[3];
-    double v[3][7];
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) {
-        line7(fs, r, c, p, a, b, v[a]);
-        reinit_axis_dual(fo[a], bk[a], v[a], r1[a], l1[a], sp[a], inv.jd[a]);
-    }
-    // Godunov step on duals of its 7 arguments (fore/back per axis, dt)
-    const D7 g = godunov_step(inside, ad::dvar<7>(fo[0].v, 0), ad::dvar<7>(bk[0].v, 1), ad::dvar<7>(fo[1].v, 2),
-                              ad::dvar<7>(bk[1].v, 3), ad::dvar<7>(fo[2].v, 4), ad::dvar<7>(bk[2].v, 5),
-                              ad::dvar<7>(dt, 6));
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) {
-        for (int k = 0; k < 7; ++k) {
-            double j = -cs * (g.d[2 * a] * fo[a].d[k] + g.d[2 * a + 1] * bk[a].d[k]);
-            if (a == 0 && k == 3) j += cs;
-            J[(size_t)(a * 7 + k) * n + i] = j;
-        }
-        if (jp) {
-            jp[2 * a] = -cs * (g.d[2 * a] * fo[a].d[7] + g.d[2 * a + 1] * bk[a].d[7]);
-            jp[2 * a + 1] = -cs * (g.d[2 * a] * fo[a].d[8] + g.d[2 * a + 1] * bk[a].d[8]);
-        }
-    }
-    if (jp) jp[6] = -cs * g.d[6];
-}
+constexpr int kJacGroup = 3;  // inputs per block of the listed points' launch
 
-__global__ void __launch_bounds__(256) ka_reinit_jac_bulk(double* __restrict__ J, const double* __restrict__ fs,
-                                                          const uint8_t* __restrict__ flags, Box b, Inv inv,
-                                                          int stage)
-{
-    const idx_t n = (idx_t)b.rows * b.cols * b.pges;
-    const idx_t i = (idx_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const uint8_t fl = flags[i];
-    if (fl & FLAG_SUBCELL) return;
-    const double r1[3] = {b.dx, b.dy, b.dz};
-    reinit_point_jac(J, nullptr, n, i, fs, b, inv, r1, r1, inv.dt_bulk, (fl & FLAG_MASK) != 0, stage);
-}
-
-__global__ void __launch_bounds__(256) ka_reinit_jac_list(double* __restrict__ J, double* __restrict__ JP,
+__global__ void __launch_bounds__(192) ka_reinit_jac_list(double* __restrict__ J, double* __restrict__ JP,
+                                                          const double* __restrict__ lam,
                                                           const double* __restrict__ fs,
                                                           const uint8_t* __restrict__ flags, IList il, Box b, Inv inv,
-                                                          int stage)
+                                                          int stage, const int* __restrict__ extra,
+                                                          const int* __restrict__ extra_count, int seq)
 {
+    __shared__ double val6[3][2][64];
     const idx_t n = (idx_t)b.rows * b.cols * b.pges;
-    const int cnt = *il.count;
-    for (int j = (int)(blockIdx.x * blockDim.x + threadIdx.x); j < cnt; j += (int)(gridDim.x * blockDim.x)) {
-        const idx_t i = il.idx[j];
-        double r1[3], l1[3];
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            r1[a] = il.dist[(size_t)(2 * a) * il.cap + j];
-            l1[a] = il.dist[(size_t)(2 * a + 1) * il.cap + j];
+    const int lane = (int)(threadIdx.x & 63), a = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int first = (int)blockIdx.y * kJacGroup;
+    const int listed = *il.count, total = listed + extra_count[seq & 1];
+    const double ds = a == 0 ? b.dx : (a == 1 ? b.dy : b.dz);
+    const double cs = stage_c(stage);
+    for (int j0 = (int)blockIdx.x * 64; j0 < total; j0 += (int)gridDim.x * 64) {
+        const int j = j0 + lane;
+        const bool in = j < total, list = j < listed;
+        const idx_t i = in ? (list ? (idx_t)il.idx[j] : (idx_t)extra[j - listed]) : 0;
+        const uint8_t fl = flags[i];
+        const double dt = list ? il.dt[j] : inv.dt_bulk;
+        Dual<kJacGroup> fo(0.0), bk(0.0);
+        if (in && dt >= 0) {
+            int r, c, p;
+            point_coords(b, i, r, c, p);
+            double v[7], r1 = ds, l1 = ds;
+            line7(fs, r, c, p, a, b, v);
+            if (list) {
+                r1 = il.dist[(size_t)(2 * a) * il.cap + j];
+                l1 = il.dist[(size_t)(2 * a + 1) * il.cap + j];
+            }
+            reinit_axis_dual(fo, bk, v, r1, l1, ds, inv.jd[a], first);
         }
-        double jp[7];
-        reinit_point_jac(J, jp, n, i, fs, b, inv, r1, l1, il.dt[j], (flags[i] & FLAG_MASK) != 0, stage);
+        val6[a][0][lane] = fo.v;
+        val6[a][1][lane] = bk.v;
+        __syncthreads();
+        if (in) {
+            const Dual<3> g = godunov_dual(val6, lane, a, (fl & FLAG_MASK) != 0, dt);
+            const double li = lam ? lam[i] : 1.0;
 #pragma unroll
-        for (int e = 0; e < 7; ++e) JP[(size_t)e * il.cap + j] = jp[e];
+            for (int m = 0; m < kJacGroup; ++m) {
+                const int k = first + m;
+                double w = -cs * (g.d[0] * fo.d[m] + g.d[1] * bk.d[m]);
+                if (k == 3 && a == 0) w += cs;
+                w *= li;
+                if (k < 7) {
+                    J[(size_t)(a * 7 + k) * n + i] = w;
+                } else if (list) {
+                    double* o = JP + (size_t)(2 * a + k - 7) * il.cap + j;
+                    *o = lam ? *o + w : w;
+                }
+            }
+            if (list && a == 0 && first == 0) {
+                double* o = JP + (size_t)6 * il.cap + j;
+                const double w = -cs * g.d[2] * li;
+                *o = lam ? *o + w : w;
+            }
+        }
+        __syncthreads();  // val6 is read before the next points' values come in
     }
 }
 
 // ---------------------------------------------------------------------------
 // sweeps
 // ---------------------------------------------------------------------------
-// adjoint: lam_in[j] = beta*lam_in[j] + sum over (i, a, k) with
-// clamp(i + (k-3) e_a) = j of J[a*7+k][i] lam[i]
-__global__ void __launch_bounds__(256) ka_transpose(double* __restrict__ lam_in, const double* __restrict__ J,
-                                                    const double* __restrict__ lam, Box b, double beta)
+// adjoint: out[j] = sum over (i, a, k) with clamp(i + (k-3) e_a) = j of
+// P[a*7+k][i] (the Jacobian's rows times lam_i), plus ca*A[j] + cb*B[j] (A, B may
+// be null).  Every (a, k) has the point i = j - (k-3) e_a if that is in the box;
+// these 21 loads are issued together.  A point on a face of the box also
+// takes the rows of the points whose taps were clamped to it.  out may be A
+// or B.  Reads 21 rows once: 44 MB at 64^3 in 8.9 us
+// (4.9 TB/s; 20 us with the loads one after another near a face, which every
+// wave of 64 rows touches).
+__global__ void __launch_bounds__(256) ka_transpose(double* out, const double* __restrict__ P, Box b, double ca,
+                                                    const double* A, double cb, const double* B)
 {
     const idx_t n = (idx_t)b.rows * b.cols * b.pges;
     const idx_t j = (idx_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n) return;
     int r, c, p;
     point_coords(b, j, r, c, p);
-    double acc = 0.0;
-#pragma unroll 1
-    for (int a = 0; a < 3; ++a) {
-        const int ja = (a == 0) ? c : (a == 1 ? r : p);
-        const int Na = (a == 0) ? b.cols : (a == 1 ? b.rows : b.pges);
-#pragma unroll 1
-        for (int k = 0; k < 7; ++k) {
-            const int o = k - 3;
-            int lo, hi;  // the i_a with clamp(i_a + o) == ja
-            if (ja > 0 && ja < Na - 1) {
-                lo = hi = ja - o;
-            } else if (ja == 0) {
-                lo = 0;
-                hi = -o;
-            } else {
-                lo = Na - 1 - o;
-                hi = Na - 1;
-            }
-            lo = lo < 0 ? 0 : lo;
-            hi = hi > Na - 1 ? Na - 1 : hi;
-            for (int ia = lo; ia <= hi; ++ia) {
-                const idx_t i = shifted(b, r, c, p, a, ia - ja);
-                acc += J[(size_t)(a * 7 + k) * n + i] * lam[i];
-            }
-        }
+    const double va = A ? A[j] : 0.0, vb = B ? B[j] : 0.0;
+    const idx_t st[3] = {(idx_t)b.rows, 1, (idx_t)b.rows * b.cols};
+    const int pos[3] = {c, r, p}, len[3] = {b.cols, b.rows, b.pges};
+    double w[21], acc = 0.0;
+#pragma unroll
+    for (int e = 0; e < 21; ++e) {
+        const int a = e / 7, o = e % 7 - 3, ia = pos[a] - o;
+        const bool in = ia >= 0 && ia < len[a];
+        w[e] = P[(size_t)e * n + (in ? j - o * st[a] : j)];
+        if (!in) w[e] = 0.0;
     }
-    lam_in[j] = (beta == 0.0 ? 0.0 : beta * lam_in[j]) + acc;
+#pragma unroll
+    for (int e = 0; e < 21; ++e) acc += w[e];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        // the taps beyond the face: offset -o of the points 0 .. o-1, and mirrored
+        if (pos[a] == 0)
+            for (int o = 1; o <= 3; ++o)
+                for (int ia = 0; ia < o; ++ia) acc += P[(size_t)(a * 7 + 3 - o) * n + (j + ia * st[a])];
+        if (pos[a] == len[a] - 1)
+            for (int o = 1; o <= 3; ++o)
+                for (int ia = 0; ia < o; ++ia) acc += P[(size_t)(a * 7 + 3 + o) * n + (j - ia * st[a])];
+    }
+    out[j] = (ca * va + cb * vb) + acc;
 }
 
 // tangent: out[i] = sum_{a,k} J[a*7+k][i] x[clamp(i + (k-3) e_a)]
@@ -254,18 +361,6 @@ __global__ void ka_axpby(double* __restrict__ y, const double* __restrict__ x, d
     y[i] = alpha * x[i] + (beta == 0.0 ? 0.0 : beta * y[i]);
 }
 
-// g_a[i] += JU[a][i] * lam[i]   (velocity gradient)
-__global__ void ka_velocity_grad(double* __restrict__ gx, double* __restrict__ gy, double* __restrict__ gz,
-                                 const double* __restrict__ JU, const double* __restrict__ lam, idx_t n)
-{
-    const idx_t i = (idx_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const double l = lam[i];
-    gx[i] += JU[i] * l;
-    gy[i] += JU[(size_t)n + i] * l;
-    gz[i] += JU[(size_t)2 * n + i] * l;
-}
-
 // out[i] += sum_a JU[a][i] * udot_a[i]   (velocity tangent)
 __global__ void ka_velocity_tangent(double* __restrict__ out, const double* __restrict__ JU,
                                     const double* __restrict__ ux, const double* __restrict__ uy,
@@ -277,17 +372,7 @@ __global__ void ka_velocity_tangent(double* __restrict__ out, const double* __re
 }
 
 // reinitialization parameters, list order (7 rows of cap):
-// adjoint  lamP[e][j] += JP[e][j] * lam[idx[j]];  tangent out[idx[j]] += sum_e JP[e][j] Pdot[e][j]
-__global__ void ka_param_grad(double* __restrict__ lamP, const double* __restrict__ JP, const double* __restrict__ lam,
-                              IList il)
-{
-    const int cnt = *il.count;
-    for (int j = (int)(blockIdx.x * blockDim.x + threadIdx.x); j < cnt; j += (int)(gridDim.x * blockDim.x)) {
-        const double l = lam[il.idx[j]];
-        for (int e = 0; e < 7; ++e) lamP[(size_t)e * il.cap + j] += JP[(size_t)e * il.cap + j] * l;
-    }
-}
-
+// out[idx[j]] += sum_e JP[e][j] Pdot[e][j]
 __global__ void ka_param_tangent(double* __restrict__ out, const double* __restrict__ JP,
                                  const double* __restrict__ Pdot, IList il)
 {
@@ -455,25 +540,30 @@ static inline Inv ainv(const Geom& g)
 }
 static inline IList alist(const ListView& lv) { return IList{lv.idx, lv.count, lv.dist, lv.dt, lv.cap}; }
 
-hipError_t launch_adj_advect_jac(double* J, double* JU, const double* fs, const double* vx, const double* vy,
-                                 const double* vz, double dt, const Geom& g, int stage, hipStream_t s)
+hipError_t launch_adj_advect_jac(double* J, double* ux, double* uy, double* uz, const double* lam, const double* fs,
+                                 const double* vx, const double* vy, const double* vz, double dt, const Geom& g,
+                                 int stage, hipStream_t s)
 {
-    ka_advect_jac<<<grid1(g.n()), 256, 0, s>>>(J, JU, fs, vx, vy, vz, dt, abox(g), ainv(g), stage);
+    ka_advect_jac<<<dim3((unsigned)((g.n() + 63) / 64)), 192, 0, s>>>(J, Grad3{{ux, uy, uz}}, lam, fs, vx, vy, vz, dt,
+                                                                     abox(g), ainv(g), stage);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_reinit_jac(double* J, double* JP, const double* fs, const uint8_t* flags, const ListView& lv,
-                                 const Geom& g, int stage, hipStream_t s)
+hipError_t launch_adj_reinit_jac(double* J, double* JP, const double* lam, const double* fs, const uint8_t* flags,
+                                 const ListView& lv, const Geom& g, int stage, int* extra, int* extra_count, int seq,
+                                 hipStream_t s)
 {
-    ka_reinit_jac_bulk<<<grid1(g.n()), 256, 0, s>>>(J, fs, flags, abox(g), ainv(g), stage);
-    ka_reinit_jac_list<<<256, 256, 0, s>>>(J, JP, fs, flags, alist(lv), abox(g), ainv(g), stage);
+    ka_reinit_jac_bulk<<<dim3((unsigned)((g.n() + 63) / 64)), 192, 0, s>>>(J, lam, fs, flags, abox(g), ainv(g), stage,
+                                                                         extra, extra_count, seq);
+    ka_reinit_jac_list<<<dim3(512, 9 / kJacGroup), 192, 0, s>>>(J, JP, lam, fs, flags, alist(lv), abox(g), ainv(g),
+                                                               stage, extra, extra_count, seq);
     return hipGetLastError();
 }
 
-hipError_t launch_adj_transpose(double* lam_in, const double* J, const double* lam, const Geom& g, double beta,
-                                hipStream_t s)
+hipError_t launch_adj_transpose(double* out, const double* P, const Geom& g, double ca, const double* A, double cb,
+                                const double* B, hipStream_t s)
 {
-    ka_transpose<<<grid1(g.n()), 256, 0, s>>>(lam_in, J, lam, abox(g), beta);
+    ka_transpose<<<grid1(g.n()), 256, 0, s>>>(out, P, abox(g), ca, A, cb, B);
     return hipGetLastError();
 }
 
@@ -495,23 +585,10 @@ hipError_t launch_adj_fill(double* y, double v, int64_t n, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_adj_velocity_grad(double* gx, double* gy, double* gz, const double* JU, const double* lam,
-                                    int64_t n, hipStream_t s)
-{
-    ka_velocity_grad<<<grid1(n), 256, 0, s>>>(gx, gy, gz, JU, lam, (idx_t)n);
-    return hipGetLastError();
-}
-
 hipError_t launch_adj_velocity_tangent(double* out, const double* JU, const double* ux, const double* uy,
                                        const double* uz, int64_t n, hipStream_t s)
 {
     ka_velocity_tangent<<<grid1(n), 256, 0, s>>>(out, JU, ux, uy, uz, (idx_t)n);
-    return hipGetLastError();
-}
-
-hipError_t launch_adj_param_grad(double* lamP, const double* JP, const double* lam, const ListView& lv, hipStream_t s)
-{
-    ka_param_grad<<<256, 256, 0, s>>>(lamP, JP, lam, alist(lv));
     return hipGetLastError();
 }
 

@@ -2158,8 +2158,7 @@ int vls_sdf3_adjoint_advect_rk3(vls_sdf3_t h, const double* F, const double* vx,
     const int64_t n = g.n();
     if ((rc = ensure_adj(h, (size_t)n * (21 + 3 + 4)))) return rc;
     double* J = h->adj;
-    double* JU = J + 21 * n;
-    double* t1 = JU + 3 * n;
+    double* t1 = J + 21 * n;
     double* t2 = t1 + n;
     double* la = t2 + n;
     double* lb = la + n;
@@ -2167,20 +2166,14 @@ int vls_sdf3_adjoint_advect_rk3(vls_sdf3_t h, const double* F, const double* vx,
     VLS_HIP(launch_advect_stage<double>(t1, F, nullptr, vx, vy, vz, dt, g, 0, s));
     VLS_HIP(launch_advect_stage<double>(t2, t1, F, vx, vy, vz, dt, g, 1, s));
     // stage 2: out = S2(t2; F)
-    VLS_HIP(launch_adj_advect_jac(J, JU, t2, vx, vy, vz, dt, g, 2, s));
-    VLS_HIP(launch_adj_transpose(la, J, lam_out, g, 0.0, s));
-    VLS_HIP(launch_adj_velocity_grad(gx, gy, gz, JU, lam_out, n, s));
-    VLS_HIP(launch_adj_axpby(lb, lam_out, stage_e(2), 0.0, n, s));
+    VLS_HIP(launch_adj_advect_jac(J, gx, gy, gz, lam_out, t2, vx, vy, vz, dt, g, 2, s));
+    VLS_HIP(launch_adj_transpose(la, J, g, 0.0, nullptr, 0.0, nullptr, s));
     // stage 1: t2 = S1(t1; F)
-    VLS_HIP(launch_adj_advect_jac(J, JU, t1, vx, vy, vz, dt, g, 1, s));
-    VLS_HIP(launch_adj_transpose(t2, J, la, g, 0.0, s));  // t2 <- adjoint of t1
-    VLS_HIP(launch_adj_velocity_grad(gx, gy, gz, JU, la, n, s));
-    VLS_HIP(launch_adj_axpby(lb, la, stage_e(1), 1.0, n, s));
-    // stage 0: t1 = S0(F)
-    VLS_HIP(launch_adj_advect_jac(J, JU, F, vx, vy, vz, dt, g, 0, s));
-    VLS_HIP(launch_adj_transpose(lb, J, t2, g, 1.0, s));
-    VLS_HIP(launch_adj_velocity_grad(gx, gy, gz, JU, t2, n, s));
-    VLS_HIP(launch_copy<double>(lam_in, lb, n, s));
+    VLS_HIP(launch_adj_advect_jac(J, gx, gy, gz, la, t1, vx, vy, vz, dt, g, 1, s));
+    VLS_HIP(launch_adj_transpose(lb, J, g, 0.0, nullptr, 0.0, nullptr, s));
+    // stage 0: t1 = S0(F); F also enters stages 1 and 2 as the start value
+    VLS_HIP(launch_adj_advect_jac(J, gx, gy, gz, lb, F, vx, vy, vz, dt, g, 0, s));
+    VLS_HIP(launch_adj_transpose(lam_in, J, g, stage_e(2), lam_out, stage_e(1), la, s));
     return VLS_OK;
 }
 
@@ -2203,18 +2196,18 @@ int vls_sdf3_tangent_advect_rk3(vls_sdf3_t h, const double* F, const double* Fdo
     double* d2 = d1 + n;
     const hipStream_t s = S(stream);
     // stage 0
-    VLS_HIP(launch_adj_advect_jac(J, JU, F, vx, vy, vz, dt, g, 0, s));
+    VLS_HIP(launch_adj_advect_jac(J, JU, JU + n, JU + 2 * n, nullptr, F, vx, vy, vz, dt, g, 0, s));
     VLS_HIP(launch_adj_apply(d1, J, Fdot, g, s));
     VLS_HIP(launch_adj_velocity_tangent(d1, JU, udx, udy, udz, n, s));
     VLS_HIP(launch_advect_stage<double>(t1, F, nullptr, vx, vy, vz, dt, g, 0, s));
     // stage 1
-    VLS_HIP(launch_adj_advect_jac(J, JU, t1, vx, vy, vz, dt, g, 1, s));
+    VLS_HIP(launch_adj_advect_jac(J, JU, JU + n, JU + 2 * n, nullptr, t1, vx, vy, vz, dt, g, 1, s));
     VLS_HIP(launch_adj_apply(d2, J, d1, g, s));
     VLS_HIP(launch_adj_axpby(d2, Fdot, stage_e(1), 1.0, n, s));
     VLS_HIP(launch_adj_velocity_tangent(d2, JU, udx, udy, udz, n, s));
     VLS_HIP(launch_advect_stage<double>(t2, t1, F, vx, vy, vz, dt, g, 1, s));
     // stage 2
-    VLS_HIP(launch_adj_advect_jac(J, JU, t2, vx, vy, vz, dt, g, 2, s));
+    VLS_HIP(launch_adj_advect_jac(J, JU, JU + n, JU + 2 * n, nullptr, t2, vx, vy, vz, dt, g, 2, s));
     VLS_HIP(launch_adj_apply(Fdot_out, J, d2, g, s));
     VLS_HIP(launch_adj_axpby(Fdot_out, Fdot, stage_e(2), 1.0, n, s));
     VLS_HIP(launch_adj_velocity_tangent(Fdot_out, JU, udx, udy, udz, n, s));
@@ -2236,15 +2229,13 @@ int vls_sdf3_adjoint_reinit(vls_sdf3_t h, const double* F0, int iterations, cons
     const Geom& g = h->g;
     const int64_t n = g.n();
     const int K = iterations;
-    if ((rc = ensure_adj(h, (size_t)n * (21 + 7 + 7 + 4 + 3 * (size_t)K + 1)))) return rc;
+    if ((rc = ensure_adj(h, (size_t)n * (21 + 7 + 3 + 3 * (size_t)K + 1)))) return rc;
     double* J = h->adj;
-    double* JP = J + 21 * n;
-    double* lamP = JP + 7 * n;
+    double* lamP = J + 21 * n;
     double* lam = lamP + 7 * n;
     double* lt0 = lam + n;
     double* lt1 = lt0 + n;
-    double* lx = lt1 + n;
-    double* X = lx + n;  // X[k] = X + k*n, k = 0..K; then T0[k], T1[k]
+    double* X = lt1 + n;  // X[k] = X + k*n, k = 0..K; then T0[k], T1[k]
     double* T0 = X + (size_t)(K + 1) * n;
     double* T1 = T0 + (size_t)K * n;
     const hipStream_t s = S(stream);
@@ -2266,20 +2257,16 @@ int vls_sdf3_adjoint_reinit(vls_sdf3_t h, const double* F0, int iterations, cons
     for (int k = K - 1; k >= 0; --k) {
         const double* xk = X + (size_t)k * n;
         // stage 2: X[k+1] = S2(T1[k]; X[k])
-        VLS_HIP(launch_adj_reinit_jac(J, JP, T1 + (size_t)k * n, h->flags, ms.lv, g, 2, s));
-        VLS_HIP(launch_adj_transpose(lt1, J, lam, g, 0.0, s));
-        VLS_HIP(launch_adj_param_grad(lamP, JP, lam, ms.lv, s));
-        VLS_HIP(launch_adj_axpby(lx, lam, stage_e(2), 0.0, n, s));
+        VLS_HIP(launch_adj_reinit_jac(J, lamP, lam, T1 + (size_t)k * n, h->flags, ms.lv, g, 2, h->over, rs.counts,
+                                      rs.seq++, s));
+        VLS_HIP(launch_adj_transpose(lt1, J, g, 0.0, nullptr, 0.0, nullptr, s));
         // stage 1: T1[k] = S1(T0[k]; X[k])
-        VLS_HIP(launch_adj_reinit_jac(J, JP, T0 + (size_t)k * n, h->flags, ms.lv, g, 1, s));
-        VLS_HIP(launch_adj_transpose(lt0, J, lt1, g, 0.0, s));
-        VLS_HIP(launch_adj_param_grad(lamP, JP, lt1, ms.lv, s));
-        VLS_HIP(launch_adj_axpby(lx, lt1, stage_e(1), 1.0, n, s));
-        // stage 0: T0[k] = S0(X[k])
-        VLS_HIP(launch_adj_reinit_jac(J, JP, xk, h->flags, ms.lv, g, 0, s));
-        VLS_HIP(launch_adj_transpose(lx, J, lt0, g, 1.0, s));
-        VLS_HIP(launch_adj_param_grad(lamP, JP, lt0, ms.lv, s));
-        VLS_HIP(launch_copy<double>(lam, lx, n, s));
+        VLS_HIP(launch_adj_reinit_jac(J, lamP, lt1, T0 + (size_t)k * n, h->flags, ms.lv, g, 1, h->over, rs.counts,
+                                      rs.seq++, s));
+        VLS_HIP(launch_adj_transpose(lt0, J, g, 0.0, nullptr, 0.0, nullptr, s));
+        // stage 0: T0[k] = S0(X[k]); X[k] also enters stages 1 and 2 as the start value
+        VLS_HIP(launch_adj_reinit_jac(J, lamP, lt0, xk, h->flags, ms.lv, g, 0, h->over, rs.counts, rs.seq++, s));
+        VLS_HIP(launch_adj_transpose(lam, J, g, stage_e(2), lam, stage_e(1), lt1, s));
     }
     VLS_HIP(launch_copy<double>(lam_in, lam, n, s));
     VLS_HIP(launch_adj_dist(lam_in, F0, lamP, ms.lv, g, s));
@@ -2319,16 +2306,16 @@ int vls_sdf3_tangent_reinit(vls_sdf3_t h, const double* F0, const double* F0dot,
     ReinitSeq rs;
     if ((rc = reinit_begin(h, rs, s))) return rc;
     for (int k = 0; k < iterations; ++k) {
-        VLS_HIP(launch_adj_reinit_jac(J, JP, X, h->flags, ms.lv, g, 0, s));
+        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, X, h->flags, ms.lv, g, 0, h->over, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_apply(d0, J, Xd, g, s));
         VLS_HIP(launch_adj_param_tangent(d0, JP, Pd, ms.lv, s));
         if ((rc = reinit_stage<double>(h, rs, t0, X, nullptr, ms, 0, s))) return rc;
-        VLS_HIP(launch_adj_reinit_jac(J, JP, t0, h->flags, ms.lv, g, 1, s));
+        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, t0, h->flags, ms.lv, g, 1, h->over, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_apply(d1, J, d0, g, s));
         VLS_HIP(launch_adj_axpby(d1, Xd, stage_e(1), 1.0, n, s));
         VLS_HIP(launch_adj_param_tangent(d1, JP, Pd, ms.lv, s));
         if ((rc = reinit_stage<double>(h, rs, t1, t0, X, ms, 1, s))) return rc;
-        VLS_HIP(launch_adj_reinit_jac(J, JP, t1, h->flags, ms.lv, g, 2, s));
+        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, t1, h->flags, ms.lv, g, 2, h->over, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_apply(d0, J, d1, g, s));
         VLS_HIP(launch_adj_axpby(d0, Xd, stage_e(2), 1.0, n, s));
         VLS_HIP(launch_adj_param_tangent(d0, JP, Pd, ms.lv, s));

@@ -352,24 +352,26 @@ hipError_t launch_batch_ellipsoid(const BatchView& B, T* F, const double* axes, 
 
 // ---- discrete adjoint and tangent (vls_adjoint.hip), FP64, one grid ----------
 // stage Jacobians: J = 21 rows of n (d out_i / d fs along the three lines
-// through i, row a*7 + offset+3), JU = 3 rows of n (d out_i / d u_a,i),
-// JP = 7 rows of lv.cap (d out / d (xpr..zpd, dt) of the listed points)
-hipError_t launch_adj_advect_jac(double* J, double* JU, const double* fs, const double* vx, const double* vy,
-                                 const double* vz, double dt, const Geom& g, int stage, hipStream_t s);
-hipError_t launch_adj_reinit_jac(double* J, double* JP, const double* fs, const uint8_t* flags, const ListView& lv,
-                                 const Geom& g, int stage, hipStream_t s);
-// lam_in = beta*lam_in + J^T lam;  out = J x
-hipError_t launch_adj_transpose(double* lam_in, const double* J, const double* lam, const Geom& g, double beta,
-                                hipStream_t s);
+// through i, row a*7 + offset+3), times lam_i where lam is given (adjoint).
+// ux, uy, uz: d out_i / d u_a,i (tangent), or its product with lam_i added
+// (adjoint).  JP = 7 rows of lv.cap, d out / d (xpr..zpd, dt) of the listed
+// points, or its product with lam_i added.  extra (n ints), extra_count (2
+// ints, zero before seq 0) and seq, which numbers the stages of a call: work
+// memory as launch_reinit_stage's.
+hipError_t launch_adj_advect_jac(double* J, double* ux, double* uy, double* uz, const double* lam, const double* fs,
+                                 const double* vx, const double* vy, const double* vz, double dt, const Geom& g,
+                                 int stage, hipStream_t s);
+hipError_t launch_adj_reinit_jac(double* J, double* JP, const double* lam, const double* fs, const uint8_t* flags,
+                                 const ListView& lv, const Geom& g, int stage, int* extra, int* extra_count, int seq,
+                                 hipStream_t s);
+// out = J^T lam + ca*A + cb*B from the rows J lam (A, B may be null);  out = J x
+hipError_t launch_adj_transpose(double* out, const double* P, const Geom& g, double ca, const double* A, double cb,
+                                const double* B, hipStream_t s);
 hipError_t launch_adj_apply(double* out, const double* J, const double* x, const Geom& g, hipStream_t s);
 hipError_t launch_adj_fill(double* y, double v, int64_t n, hipStream_t s);
 hipError_t launch_adj_axpby(double* y, const double* x, double alpha, double beta, int64_t n, hipStream_t s);
-hipError_t launch_adj_velocity_grad(double* gx, double* gy, double* gz, const double* JU, const double* lam,
-                                    int64_t n, hipStream_t s);
 hipError_t launch_adj_velocity_tangent(double* out, const double* JU, const double* ux, const double* uy,
                                        const double* uz, int64_t n, hipStream_t s);
-hipError_t launch_adj_param_grad(double* lamP, const double* JP, const double* lam, const ListView& lv,
-                                 hipStream_t s);
 hipError_t launch_adj_param_tangent(double* out, const double* JP, const double* Pdot, const ListView& lv,
                                     hipStream_t s);
 // distances of the listed points as functions of F0: adjoint (atomic adds

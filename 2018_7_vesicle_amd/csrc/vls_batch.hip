@@ -217,17 +217,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
     ZFace<T> zf;
     zmarch<R, T, false, true>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, fs + off, shift(fn, off), nullptr, nullptr,
                         nullptr, flags + off, stage,
+                        [&](const T* w6) { zface_start(zf, w6, axis_arg(invs, 2, T())); },
                         [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st, int p) {
                             bool cross;
-                            const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs, stage, cross,
-                                                          zf, p == it.p0);
+                            const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs, stage, cross, zf);
                             const bool bulk = !(st.flags(zc) & FLAG_SUBCELL);
                             if constexpr (defers_crossings<T>()) {
-                                if (bulk && !cross) stp(o + (idx_t)p * plane, zc.in, res);
+                                if (bulk && !cross) stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
                                 wave_append(bulk && cross, (int)(off + (idx_t)p * plane + zc.in), over,
                                             &over_count[seq & 1]);
                             } else if (bulk) {
-                                stp(o + (idx_t)p * plane, zc.in, res);
+                                stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
                             }
                         });
 }
@@ -291,11 +291,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
     const idx_t off = G.off, plane = (idx_t)b.rows * b.cols;
     T* o = out + off;
     // the listed points carry a NaN x-velocity (kb_list_gather_vel)
+    ZDiff<T> zd;
     zmarch<R, T, true, false>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, cs + off, shift(cn, off), vx + off,
                        vy + off, vz + off, nullptr, stage,
+                       [&](const T* w6) { zdiff_start(zd, w6); },
                        [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, true>& st, int p) {
-                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, (T)inv.dt_bulk, inv, stage);
-                           if (zc.valid && st.vel[0] == st.vel[0]) stp(o + (idx_t)p * plane, zc.in, res);
+                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, (T)inv.dt_bulk, inv, stage, zd);
+                           if (zc.valid && st.vel[0] == st.vel[0]) stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
                        });
 }
 
@@ -313,11 +315,13 @@ __global__ void __launch_bounds__(256) kb_advect_stage(T* __restrict__ out, cons
     const T dtg = (T)dt[it.g];
     const idx_t off = G.off, plane = (idx_t)b.rows * b.cols;
     T* o = out + off;
+    ZDiff<T> zd;
     zmarch<R, T, true, false>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, fs + off, shift(fn, off), vx + off, vy + off,
                        vz + off, nullptr, stage,
+                       [&](const T* w6) { zdiff_start(zd, w6); },
                        [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, true>& st, int p) {
-                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, dtg, inv, stage);
-                           if (zc.valid) stp(o + (idx_t)p * plane, zc.in, res);
+                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, dtg, inv, stage, zd);
+                           if (zc.valid) stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
                        });
 }
 
@@ -355,6 +359,7 @@ __global__ void __launch_bounds__(256) kb_ext_vel_bulk(T* __restrict__ vx, T* __
     const double sp[3] = {b.dx, b.dy, b.dz};
     zmarch<R, T, false, true>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, F + off, nullptr, nullptr, nullptr,
                               nullptr, flags + off, 0,
+                              [](const T*) {},
                               [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st, int p) {
                                   if (st.flags(zc) & FLAG_SUBCELL) return;  // listed, or outside the box
                                   double n[3];
@@ -539,7 +544,8 @@ kb_eno2_extend_stage(double* __restrict__ out, const double* __restrict__ cs, co
     // stage != 0 loads the start value cn at each point (ZStep::fn)
     zmarch<R, double, true, true>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, cs + off, shift(cn, off), vx + off,
                                   vy + off, vz + off, flags + off, heun2,
-                                  [&](const double* l, const ZCol<R>& zc, const double w[7],
+                                  [](const double*) {},
+                              [&](const double* l, const ZCol<R>& zc, const double w[7],
                                       const ZStep<R, double, true>& st, int p) {
                                       double fo[3], bk[3];
                                       const double* x = l + zc.base;
@@ -549,7 +555,7 @@ kb_eno2_extend_stage(double* __restrict__ out, const double* __restrict__ cs, co
                                       eno2_bulk_pair(fo[2], bk[2], w[1], w[2], w[3], w[4], w[5], ez);
                                       const double step = upwind_sum(fo, bk, st.vel[0], st.vel[1], st.vel[2], dt);
                                       const double res = heun2 ? (st.fn + w[3] - step) / 2 : w[3] - step;
-                                      if (!(st.flags(zc) & FLAG_SUBCELL)) stp(o + (idx_t)p * plane, zc.in, res);
+                                      if (!(st.flags(zc) & FLAG_SUBCELL)) stb<double>(page_of(o, (idx_t)p * plane), zc.in, res);
                                   });
 }
 

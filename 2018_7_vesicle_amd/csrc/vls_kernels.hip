@@ -131,7 +131,8 @@ __global__ void __launch_bounds__(256) k_crossings_z(Dist6 d, double* __restrict
     const idx_t plane = (idx_t)b.rows * b.cols;
     const double md = dmin(dmin(b.dx, b.dx), dmin(dmin(b.dy, b.dy), dmin(b.dz, b.dz)));
     zmarch<R, T, false, false>(lds[0], lds[1], b, r0, c0, p0, p1, lsf, nullptr, nullptr, nullptr, nullptr, nullptr,
-                               0, [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>&, int p) {
+                               0, [](const T*) {},
+                              [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>&, int p) {
                                    const double f0 = (double)w[3];
                                    const double xu = (double)l[zc.base + Shape<R>::LR],
                                                 xd = (double)l[zc.base - Shape<R>::LR];
@@ -368,17 +369,17 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
     const idx_t plane = (idx_t)b.rows * b.cols;
     ZFace<T> zf;
     zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, fs, fn, nullptr, nullptr, nullptr, flags, stage,
+                        [&](const T* w6) { zface_start(zf, w6, axis_arg(invs, 2, T())); },
                         [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st, int p) {
                             bool cross;
-                            const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs, stage, cross,
-                                                          zf, p == p0);
+                            const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs, stage, cross, zf);
                             const bool bulk = !(st.flags(zc) & FLAG_SUBCELL);
                             if constexpr (defers_crossings<T>()) {
-                                if (bulk && !cross) stp(out + (idx_t)p * plane, zc.in, res);
+                                if (bulk && !cross) stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
                                 wave_append(bulk && cross, (int)((idx_t)p * plane + zc.in), over,
                                             &over_count[seq & 1]);
                             } else if (bulk) {
-                                stp(out + (idx_t)p * plane, zc.in, res);
+                                stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
                             }
                         });
 }
@@ -628,6 +629,7 @@ __global__ void __launch_bounds__(256) k_extension_normal_z(T* __restrict__ vx, 
     const idx_t plane = (idx_t)b.rows * b.cols;
     const double sp[3] = {b.dx, b.dy, b.dz};
     zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, lsf, nullptr, nullptr, nullptr, nullptr, flags, 0,
+                              [](const T*) {},
                               [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st, int p) {
                                   if (st.flags(zc) & FLAG_SUBCELL) return;  // listed, or outside the box
                                   double n[3];
@@ -774,10 +776,12 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
     const idx_t plane = (idx_t)b.rows * b.cols;
     // the listed points carry a NaN x-velocity (k_list_gather_vel), so the
     // bulk needs no flags: it skips them and the lanes outside the box
+    ZDiff<T> zd;
     zmarch<R, T, true, false>(lds[0], lds[1], b, r0, c0, p0, p1, cs, cn, vx, vy, vz, nullptr, stage,
+                       [&](const T* w6) { zdiff_start(zd, w6); },
                        [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, true>& st, int p) {
-                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, (T)inv.dt_bulk, inv, stage);
-                           if (zc.valid && st.vel[0] == st.vel[0]) stp(out + (idx_t)p * plane, zc.in, res);
+                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, (T)inv.dt_bulk, inv, stage, zd);
+                           if (zc.valid && st.vel[0] == st.vel[0]) stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
                        });
 }
 
@@ -821,10 +825,12 @@ __global__ void __launch_bounds__(256) k_advect_stage(T* __restrict__ out, const
     int r0, c0, p0, p1;
     zmarch_share<R>(b, depth, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
     const idx_t plane = (idx_t)b.rows * b.cols;
+    ZDiff<T> zd;
     zmarch<R, T, true, false>(lds[0], lds[1], b, r0, c0, p0, p1, fs, fn, vx, vy, vz, nullptr, stage,
+                       [&](const T* w6) { zdiff_start(zd, w6); },
                        [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, true>& st, int p) {
-                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, (T)dt, inv, stage);
-                           if (zc.valid) stp(out + (idx_t)p * plane, zc.in, res);
+                           const T res = upwind_value<R>(l, zc.base, w, st.vel, st.fn, (T)dt, inv, stage, zd);
+                           if (zc.valid) stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
                        });
 }
 

@@ -327,6 +327,41 @@ struct Tile {
     unsigned in;    // element offset of the point in its page, c * rows + r
 };
 
+// A page of a field as a buffer resource: a uniform base in scalar registers, to
+// which a buffer load or store adds the lane's 32-bit byte offset itself.
+// (With global loads the compiler kept 64-bit lane offsets and added them to
+// the page's base in a vector instruction per load.)
+struct Page {
+    __amdgpu_buffer_rsrc_t r;
+};
+template <typename T>
+__device__ __forceinline__ Page page_of(T* field, idx_t page)
+{
+    return Page{__builtin_amdgcn_make_buffer_rsrc((void*)(field + page), 0, 0xffffffffu, 0x00027000)};
+}
+// element `off` of the page; NT: non-temporal, for a stream read once per
+// launch (the velocity of the extension and advection stages), so that its
+// lines do not push the staged tiles' halos out of L2 (measured: extension
+// stage at 256^3 FP32 103-107 -> 98-100 us)
+template <typename T, bool NT = false>
+__device__ __forceinline__ T ldb(const Page& q, unsigned off)
+{
+    constexpr int aux = NT ? 2 : 0;
+    const int o = (int)(off * (unsigned)sizeof(T));
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(q.r, o, 0, aux));
+    else if constexpr (sizeof(T) == 4)
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(q.r, o, 0, aux));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b8(q.r, o, 0, aux));
+}
+template <typename T>
+__device__ __forceinline__ void stb(const Page& q, unsigned off, T v)
+{
+    const int o = (int)(off * (unsigned)sizeof(T));
+    typedef unsigned U2 __attribute__((ext_vector_type(2)));
+    if constexpr (sizeof(T) == 8) __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(U2, v), q.r, o, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), q.r, o, 0, 0);
+}
+
 // element `off` of a page: the uniform 64-bit page base plus a 32-bit byte
 // offset per lane, so a load or store is one instruction with a scalar base
 // (offsets reach 7 pages of doubles: pages hold fewer than 2^26 points,
@@ -335,15 +370,6 @@ template <typename T>
 __device__ __forceinline__ T ldp(const T* __restrict__ base, unsigned off)
 {
     return *(const T*)((const char*)base + off * (unsigned)sizeof(T));
-}
-// as ldp, marked non-temporal: for a stream read once per launch (the
-// velocity of the extension and advection stages), so that its lines do not
-// push the staged tiles' halos out of L2 (measured: extension stage at 256^3
-// FP32 103-107 -> 98-100 us)
-template <typename T>
-__device__ __forceinline__ T ldp_nt(const T* __restrict__ base, unsigned off)
-{
-    return __builtin_nontemporal_load((const T*)((const char*)base + off * (unsigned)sizeof(T)));
 }
 template <typename T>
 __device__ __forceinline__ void stp(T* __restrict__ base, unsigned off, T v)
@@ -686,20 +712,20 @@ __device__ __forceinline__ void zstep_load(ZStep<R, T, VEL>& s, const ZCol<R>& z
                                            const T* __restrict__ vz, const uint8_t* __restrict__ flags, int stage)
 {
     const idx_t po = (idx_t)p * plane;
-    const T* fp = fs + po;
+    const Page fp = page_of(fs, po);
 #pragma unroll
-    for (int k = 0; k < TileRegs<R, T>::NK; ++k) s.reg.m[k] = ldp(fp, zc.m[k]);
-    s.reg.s = ldp(fp, zc.s);
-    s.w = ldp(fs + (idx_t)min(p + 3, b.pges - 1) * plane, zc.in);
+    for (int k = 0; k < TileRegs<R, T>::NK; ++k) s.reg.m[k] = ldb<T>(fp, zc.m[k]);
+    s.reg.s = ldb<T>(fp, zc.s);
+    s.w = ldb<T>(page_of(fs, (idx_t)min(p + 3, b.pges - 1) * plane), zc.in);
     if (VEL) {
-        s.vel[0] = ldp_nt(vx + po, zc.in);
-        s.vel[1] = ldp_nt(vy + po, zc.in);
-        s.vel[2] = ldp_nt(vz + po, zc.in);
+        s.vel[0] = ldb<T, true>(page_of(vx, po), zc.in);
+        s.vel[1] = ldb<T, true>(page_of(vy, po), zc.in);
+        s.vel[2] = ldb<T, true>(page_of(vz, po), zc.in);
     }
     // at stage 0 (no start value) the point's own value is read and not used
     // (rk_combine does not read fn at stage 0)
-    s.fn = ldp((stage != 0 ? fn : fs) + po, zc.in);
-    if (FL) s.fl = ldp(flags + po, zc.in);
+    s.fn = ldb<T>(page_of(stage != 0 ? fn : fs, po), zc.in);
+    if (FL) s.fl = ldb<uint8_t>(page_of(flags, po), zc.in);
     else s.fl = 0;
 }
 
@@ -711,13 +737,14 @@ __device__ __forceinline__ void window_shift(T w[7], T in)
     w[6] = in;
 }
 
-// body(lds, zc, w, step, p) evaluates page p: x- and y-taps from lds, z-taps w
-template <int R, typename T, bool VEL, bool FL, class Body>
+// body(lds, zc, w, step, p) evaluates page p: x- and y-taps from lds, z-taps w;
+// start(w) is called once before it with the values of pages p0-3 .. p0+2
+template <int R, typename T, bool VEL, bool FL, class Start, class Body>
 __device__ __forceinline__ void zmarch(T* lds0, T* lds1, const Box& b, int r0, int c0, int p0, int p1,
                                        const T* __restrict__ fs, const T* __restrict__ fn,
                                        const T* __restrict__ vx, const T* __restrict__ vy,
                                        const T* __restrict__ vz, const uint8_t* __restrict__ flags, int stage,
-                                       Body body)
+                                       Start start, Body body)
 {
     if (p0 >= p1) return;
     const ZCol<R> zc = zcol<R>(b, r0, c0);
@@ -730,6 +757,7 @@ __device__ __forceinline__ void zmarch(T* lds0, T* lds1, const Box& b, int r0, i
     for (int k = 1; k < 7; ++k) w[k] = ldp(fs + (idx_t)clampi(p0 - 4 + k, b.pges - 1) * plane, zc.in);
     ZStep<R, T, VEL> sa, sb;
     zstep_load<R, T, VEL, FL>(sa, zc, p0, b, plane, fs, fn, vx, vy, vz, flags, stage);
+    start(w + 1);
     for (int p = p0;;) {
         window_shift(w, sa.w);
         store_tile<R>(lds0, sa.reg);
@@ -787,11 +815,10 @@ constexpr bool defers_crossings()
 // the start value fn and flags fl.  Returns the new value; where the bulk
 // defers crossings (FP64), cross is set for a point next to a sign change of
 // the stage field (it is left to the interface pass), else it stays false.
-// zf: the z-faces the march's previous page left (first: this is the
-// block's first page, zf is set up here)
+// zf: the z-faces the march's previous page left (zface_start at its start)
 template <int R, typename T>
 __device__ __forceinline__ T reinit_value(const T* lds, int base, const T z[7], T fn, uint8_t fl, const Inv& invs,
-                                          int stage, bool& cross, ZFace<T>& zf, bool first)
+                                          int stage, bool& cross, ZFace<T>& zf)
 {
     cross = false;
     T fo[3], bk[3];
@@ -803,7 +830,6 @@ __device__ __forceinline__ T reinit_value(const T* lds, int base, const T z[7], 
         if constexpr (defers_crossings<T>()) cross |= sign_change3(v);
         weno5_pair(fo[a], bk[a], v, axis_arg(invs, a, T()));
     }
-    if (first) zface_start(zf, z, axis_arg(invs, 2, T()));
     if constexpr (defers_crossings<T>()) {
         bool cz;
         weno5_pair_z(fo[2], bk[2], cz, z, zf, axis_arg(invs, 2, T()));
@@ -875,10 +901,12 @@ __device__ __forceinline__ void reinit_iface_finish(T* __restrict__ out, const T
 
 // upwind WENO5 rate of the extension and advection stages at a bulk point
 // (x- and y-taps from the staged tile, z-taps z[0..6]) and the RK
-// combination with the stage's time step: acc * scale is the step
+// combination with the stage's time step: acc * scale is the step.
+// zd: the second differences along z that the march's previous page left
+// (zdiff_start at its start)
 template <int R, typename T>
 __device__ __forceinline__ T upwind_value(const T* lds, int base, const T z[7], const T vel[3], T fn, T scale,
-                                          const Inv& inv, int stage)
+                                          const Inv& inv, int stage, ZDiff<T>& zd)
 {
     T acc = 0;
     T v[7];
@@ -886,7 +914,7 @@ __device__ __forceinline__ T upwind_value(const T* lds, int base, const T z[7], 
     acc = upwind_axis(acc, vel[0], v, axis_arg(inv, 0, T()));
     tile_line_y(lds, base, v);
     acc = upwind_axis(acc, vel[1], v, axis_arg(inv, 1, T()));
-    acc = upwind_axis(acc, vel[2], z, axis_arg(inv, 2, T()));
+    acc = upwind_axis_z(acc, vel[2], z, zd, axis_arg(inv, 2, T()));
     return rk_combine(stage, z[3], acc * scale, fn);
 }
 

@@ -1033,7 +1033,7 @@ int vls_sdf3_set_zmarch_depth(vls_sdf3_t h, int depth)
 int vls_sdf3_get_launch(vls_sdf3_t h, int* tile_rows, int* depth)
 {
     VLS_REQUIRE(h, "null handle");
-    if (tile_rows) *tile_rows = h->g.tr;
+    if (tile_rows) *tile_rows = vls::tile_rows(h->g);
     if (depth) *depth = vls::zmarch_depth(h->g);
     return VLS_OK;
 }
@@ -1436,10 +1436,13 @@ int build_tiles(vls_batch* b, int tr)
     for (int g = 0; g < b->ngrids; ++g) {
         const BGrid& G = b->grids[(size_t)g];
         const int ntr = (G.rows + tr - 1) / tr, ntc = (G.cols + tc - 1) / tc;
-        for (int p0 = 0; p0 < G.pges; p0 += b->zd)
+        // the pages in equal chunks of at most zd
+        const int nch = (G.pges + b->zd - 1) / b->zd;
+        for (int ch = 0; ch < nch; ++ch)
             for (int cb = 0; cb < ntc; ++cb)
                 for (int rb = 0; rb < ntr; ++rb)
-                    items.push_back(ZItem{g, rb * tr, cb * tc, p0, std::min(p0 + b->zd, G.pges)});
+                    items.push_back(ZItem{g, rb * tr, cb * tc, (int)((int64_t)ch * G.pges / nch),
+                                          (int)((int64_t)(ch + 1) * G.pges / nch)});
         if (items.size() >= ((size_t)1 << 31)) return fail(VLS_ERR_INVALID, "too many work items");
     }
     (void)hipFree(b->d_tile_grid);
@@ -2014,14 +2017,17 @@ int sdf3_autotune_try(vls_sdf3* h, const T* F, int iterations, hipStream_t s, in
     const DSet ms = main_set(h);
     T *vx = vel<T>(h, 0), *vy = vel<T>(h, 1), *vz = vel<T>(h, 2);
     float best = 1e30f;
-    int best_tr = h->g.tr, best_zd = h->g.zd;
-    const int trs[2] = {64, 32};
+    // the shape the box's size asks for at its depth, half and twice that, and
+    // the other shape at its own
+    h->g.tr = 0;
+    int best_tr = tile_rows(h->g), best_zd = h->g.zd;
+    const int trs[2] = {best_tr, best_tr == 32 ? 64 : 32};
     int rc;
     for (int i = 0; i < 2; ++i) {
         h->g.tr = trs[i];
         h->g.zd = 0;
         const int d0 = zmarch_depth(h->g);
-        const int depths[3] = {d0, d0 > 1 ? d0 / 2 : 0, 2 * d0 <= h->g.pges ? 2 * d0 : 0};
+        const int depths[3] = {d0, i == 0 && d0 > 1 ? d0 / 2 : 0, i == 0 && 2 * d0 <= h->g.pges ? 2 * d0 : 0};
         for (int j = 0; j < 3; ++j) {
             if (depths[j] <= 0) continue;
             h->g.zd = depths[j];

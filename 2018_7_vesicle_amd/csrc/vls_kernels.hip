@@ -1298,7 +1298,7 @@ hipError_t launch_set_distance(int order, const Dist6& d, double* min_dist, uint
     k_zero_pair<<<dim3(1), dim3(64), 0, s>>>(cand_count, lv.idx ? lv.count : nullptr);
     if (!mask_src || (const void*)mask_src == (const void*)lsf) {
         const int zd = zmarch_depth(g), m = mask_src ? 1 : 0;
-        if (g.tr == 32)
+        if (tile_rows(g) == 32)
             k_crossings_z<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(d, min_dist, flags, m, lsf, box_of(g),
                                                                                zd, cand, cand_count);
         else
@@ -1373,23 +1373,42 @@ int deferred_blocks(const Geom& g)
     return b < 8 ? 8 : b;
 }
 
-// pages per block of the z-marching bulk stage launches: g.zd, or by
-// default the largest power of two up to 16 (and pges) that still gives at
-// least 2048 blocks (8 per CU of a 256-CU device); measured on MI355X,
-// depths 4-16 are within 3% of the best at 128^3 and 256^3
+// rows per tile of the z-marching bulk stage launches: g.tr, or by default 32
+// unless 64 needs fewer tiles.  32 x 8 stages a smaller halo than 64 x 4 (532
+// values against 700) and fits more box sizes; measured on MI355X over boxes of
+// 32^3 to 256^3 and ragged ones it is 0-20% faster, at worst 1% slower (113 x 97
+// x 81).
+int tile_rows(const Geom& g)
+{
+    if (g.tr != 0) return g.tr;
+    const int64_t t32 = (int64_t)tiles_per_col<32>(g.rows) * tiles_per_row<32>(g.cols);
+    const int64_t t64 = (int64_t)tiles_per_col<64>(g.rows) * tiles_per_row<64>(g.cols);
+    return t32 <= t64 ? 32 : 64;
+}
+
+// pages per block of the z-marching bulk stage launches: g.zd, or by default
+// the smallest depth from 2 to 16 with which the blocks are all resident at
+// once, kStageWaves on each CU (16 where they cannot be).  A block's start-up
+// (window, first tile, carried faces) costs one to two pages, so deeper is
+// better until CUs run out of blocks; a second round of a few blocks costs a
+// whole march.  Measured on MI355X, extension + reinitialization stage: 96^3
+// FP64 32.7 us with 864 blocks of 4 pages, 35.0 with 1728 of 2 and 36.3 with
+// 432 of 8; 150 x 131 x 120 FP32 43.3 with 1020 of 10, 45.4 with 2550 of 4; the
+// rule is within 3% of the best depth on 12 of 15 boxes and within 8% on all.
 int zmarch_depth(const Geom& g)
 {
     if (g.zd > 0) return g.zd < g.pges ? g.zd : g.pges;
-    const int64_t cols_ = g.tr == 32 ? (int64_t)tiles_per_col<32>(g.rows) * tiles_per_row<32>(g.cols)
-                                     : (int64_t)tiles_per_col<64>(g.rows) * tiles_per_row<64>(g.cols);
-    int d = 1;
-    while (2 * d <= 16 && 2 * d <= g.pges && cols_ * g.pges / (2 * d) >= 2048) d *= 2;
-    return d;
+    const int64_t cols_ = tile_rows(g) == 32 ? (int64_t)tiles_per_col<32>(g.rows) * tiles_per_row<32>(g.cols)
+                                             : (int64_t)tiles_per_col<64>(g.rows) * tiles_per_row<64>(g.cols);
+    const int64_t resident = (int64_t)kStageWaves * device_cus();
+    int d = 2;
+    while (d < 16 && cols_ * ((g.pges + d - 1) / d) > resident) ++d;
+    return d < g.pges ? d : g.pges;
 }
 
 static inline int bulk_blocks(const Geom& g, int depth)
 {
-    return g.tr == 32 ? zmarch_blocks<32>(g.rows, g.cols, g.pges, depth)
+    return tile_rows(g) == 32 ? zmarch_blocks<32>(g.rows, g.cols, g.pges, depth)
                       : zmarch_blocks<64>(g.rows, g.cols, g.pges, depth);
 }
 
@@ -1420,7 +1439,7 @@ static hipError_t reinit_stage_scheme(T* out, const T* fs, const T* fn, const ui
     const IList il{lv.idx, lv.count, lv.dist, lv.dt, lv.cap};
     const int zd = zmarch_depth(g), ni = fused_iface_blocks(g);
     const dim3 grid(bulk_blocks(g, zd) + ni);
-    if (g.tr == 32)
+    if (tile_rows(g) == 32)
         k_reinit_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage,
                                                             over, over_count, seq, zd, ni);
     else
@@ -1493,7 +1512,7 @@ hipError_t launch_extension_normal(T* vx, T* vy, T* vz, const T* F, const uint8_
                                    double floor_, const Geom& g, hipStream_t s)
 {
     const int zd = zmarch_depth(g);
-    if (g.tr == 32)
+    if (tile_rows(g) == 32)
         k_extension_normal_z<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(vx, vy, vz, F, flags, floor_,
                                                                                   box_of(g), zd);
     else
@@ -1532,7 +1551,7 @@ static hipError_t extend_stage_scheme(T* out, const T* cs, const T* cn, const T*
     const IList il{lv.idx, lv.count, lv.dist, lv.dt, lv.cap};
     const int zd = zmarch_depth(g), ni = fused_iface_blocks(g);
     const dim3 grid(bulk_blocks(g, zd) + ni);
-    if (g.tr == 32)
+    if (tile_rows(g) == 32)
         k_extend_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, cs, cn, vx, vy, vz, il, lcp, lvel,
                                                             box_of(g), inv_of(g), stage, zd, ni);
     else
@@ -1567,7 +1586,7 @@ hipError_t launch_advect_stage(T* out, const T* fs, const T* fn, const T* vx, co
                                const Geom& g, int stage, hipStream_t s)
 {
     const int zd = zmarch_depth(g);
-    if (g.tr == 32)
+    if (tile_rows(g) == 32)
         k_advect_stage<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(out, fs, fn, vx, vy, vz, dt, box_of(g),
                                                                               inv_of(g), stage, zd);
     else

@@ -62,7 +62,7 @@ enum { IFACE_WENO = 0, IFACE_CUBIC = 1, IFACE_ENO2 = 2 };
 struct Geom {
     int rows, cols, pges;
     double dx, dy, dz;
-    int tr = 64;      // rows per tile of the bulk stage kernels: 64 or 32
+    int tr = 0;       // rows per tile of the bulk stage kernels: 64 or 32 (0: by the box size)
     int zd = 0;       // pages per block of the z-marching bulk stage kernels (0: by the box size)
     int64_t n() const { return (int64_t)rows * cols * pges; }
 };
@@ -88,6 +88,8 @@ hipError_t launch_set_distance(int order, const Dist6& d, double* min_dist, uint
 // without them, from its interface list
 hipError_t launch_fill_dense(const Dist6& d, double* min_dist, const ListView& lv, const Geom& g, hipStream_t s);
 int iface_blocks(const Geom& g);
+// rows per tile of the bulk stage kernels (g.tr, or chosen by the box size)
+int tile_rows(const Geom& g);
 // pages per block of the z-marching bulk stage kernels (g.zd, or chosen by the box size)
 int zmarch_depth(const Geom& g);
 template <typename T>

@@ -787,8 +787,11 @@ __device__ __forceinline__ void zmarch_share(const Box& b, int depth, int blk, i
     const int cb = ct / ntr;
     r0 = (ct - cb * ntr) * R;
     c0 = cb * Shape<R>::TC;
-    p0 = ch * depth;
-    p1 = min(p0 + depth, b.pges);
+    // the pages in equal chunks of at most `depth` (a last chunk of a page or
+    // two would pay a whole block's start-up)
+    const int nch = (b.pges + depth - 1) / depth;
+    p0 = (int)((int64_t)ch * b.pges / nch);
+    p1 = (int)((int64_t)(ch + 1) * b.pges / nch);
 }
 
 // blocks of a z-march launch with `depth` pages per block

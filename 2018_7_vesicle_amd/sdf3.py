@@ -181,7 +181,7 @@ class SDF3:
 
     # -- launch shape ------------------------------------------------------------
     def setTileRows(self, tile_rows):
-        """tile shape of the bulk stage kernels: 64 (64 x 4, default) or 32 (32 x 8)"""
+        """tile shape of the bulk stage kernels: 64 (64 x 4) or 32 (32 x 8); unset, chosen by the box size"""
         call("vls_sdf3_set_tile_rows", self._h, int(tile_rows))
 
     def setZmarchDepth(self, depth):

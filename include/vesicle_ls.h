@@ -258,12 +258,13 @@ typedef struct vls_sdf3 *vls_sdf3_t;
  * (rows x cols) holds fewer than 2^26 points. */
 int vls_sdf3_create(vls_sdf3_t *out, int rows, int cols, int pges, double dx, double dy, double dz);
 int vls_sdf3_destroy(vls_sdf3_t h);
-/* tile shape of the fused bulk stage kernels: 64 (64 x 4 points of a page,
- * the default) or 32 (32 x 8); results do not depend on it */
+/* tile shape of the fused bulk stage kernels: 64 (64 x 4 points of a page) or
+ * 32 (32 x 8); unset, it is chosen by the box size; results do not depend on it */
 int vls_sdf3_set_tile_rows(vls_sdf3_t h, int tile_rows);
 /* pages per block of the z-marching bulk stage kernels: each block walks one
  * tile column over `depth` consecutive pages (0, the default: chosen by the
- * box size, about 8 blocks per CU); results do not depend on it */
+ * box size, so that the blocks are resident together); results do not depend
+ * on it */
 int vls_sdf3_set_zmarch_depth(vls_sdf3_t h, int depth);
 /* the tile rows and z-march depth the bulk stage kernels launch with */
 int vls_sdf3_get_launch(vls_sdf3_t h, int *tile_rows, int *depth);

@@ -345,3 +345,27 @@ def test_batch_variants_equal_single_grids():
     b32 = bm.Batch([(g.rows, g.cols, g.pges) for g in grids], [g.spacing for g in grids], dtype=torch.float32)
     with pytest.raises(vls.VLSError, match="FP64"):
         b32.wenork3_extend(b32.zeros(), b32.zeros(), 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("box", [(64, 4, 2), (33, 9, 3), (40, 36, 44), (130, 5, 17), (32, 8, 33)])
+def test_default_launch_shape_gives_same_results(box, dtype):
+    """the launch shape the box size chooses (either tile shape, depths of all
+    pages or several uneven chunks) against 64 x 4 tiles of one page a block"""
+    rows, cols, pges = box
+    ax = [(np.arange(k) - (k - 1) / 2) * 0.1 for k in (cols, rows, pges)]
+    g = cases.Grid(*ax)
+    F = 0.8 * g.X + 0.35 * g.Y - 0.45 * g.Z + 0.017 + 0.03 * np.sin(9 * g.Y)
+    C, u = cases.smooth_scalar(g), cases.smooth_velocity(g)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dtype)  # noqa: E731
+    outs = []
+    for shape in (None, (64, 1)):
+        m = vls.SDF3(vls.GD3(*ax), T(F))
+        if shape:
+            m.setTileRows(shape[0])
+            m.setZmarchDepth(shape[1])
+        m.setDistance()
+        outs.append((m.WENO5RK3Reinitialization(m.F, 3), m.WENO5RK3Extend(T(C), 3),
+                     m.WENO5RK3Advection(m.F, *[T(c) for c in u], 0.01, 2)))
+    for a, b in zip(*outs):
+        assert torch.equal(a, b)

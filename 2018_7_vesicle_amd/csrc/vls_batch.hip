@@ -823,7 +823,6 @@ hipError_t launch_batch_reinit_stage(const BatchView& B, T* out, const T* fs, co
                                      hipStream_t s, int scheme)
 {
     const int ni = fused_list_blocks(B);
-    const int nd = ni / 10 < 8 ? 8 : ni / 10;
     if constexpr (std::is_same<T, double>::value) {
         if (scheme == IFACE_CUBIC) {
             if (B.tr == 32)
@@ -832,7 +831,7 @@ hipError_t launch_batch_reinit_stage(const BatchView& B, T* out, const T* fs, co
             else
                 kb_reinit_stage<64, T, IFACE_CUBIC><<<B.nitems + ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B,
                                                                                   stage, over, over_count, seq, ni);
-            kb_reinit_deferred<T, IFACE_CUBIC><<<nd, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B, stage,
+            kb_reinit_deferred<T, IFACE_CUBIC><<<ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B, stage,
                                                                     (const int*)over, (const int*)over_count, seq);
             return hipGetLastError();
         }
@@ -840,7 +839,7 @@ hipError_t launch_batch_reinit_stage(const BatchView& B, T* out, const T* fs, co
     if (scheme != IFACE_WENO) return hipErrorInvalidValue;
     TR_LAUNCH(kb_reinit_stage, T, B.nitems + ni, out, fs, fn, flags, ilist(lv), B, stage, over, over_count, seq, ni);
     if constexpr (defers_crossings<T>())
-        kb_reinit_deferred<T><<<nd, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B, stage, (const int*)over,
+        kb_reinit_deferred<T><<<ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B, stage, (const int*)over,
                                                    (const int*)over_count, seq);
     return hipGetLastError();
 }

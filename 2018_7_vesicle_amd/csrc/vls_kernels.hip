@@ -1365,14 +1365,6 @@ static int fused_iface_blocks(const Geom& g)
     return b < c ? b : c;
 }
 
-// blocks of the deferred-point launch: the deferred points are few (points
-// the interface reached during the reinitialization), a tenth of a list
-int deferred_blocks(const Geom& g)
-{
-    const int b = iface_blocks(g) / 10;
-    return b < 8 ? 8 : b;
-}
-
 // rows per tile of the z-marching bulk stage launches: g.tr, or by default 32
 // unless 64 needs fewer tiles.  32 x 8 stages a smaller halo than 64 x 4 (532
 // values against 700) and fits more box sizes; measured on MI355X over boxes of
@@ -1446,9 +1438,13 @@ static hipError_t reinit_stage_scheme(T* out, const T* fs, const T* fn, const ui
         k_reinit_stage<64, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage,
                                                             over, over_count, seq, zd, ni);
     if constexpr (defers_crossings<T>())
-        k_reinit_deferred<T, S><<<dim3(deferred_blocks(g)), dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g),
-                                                                                inv_of(g), stage, over, over_count,
-                                                                                seq);
+        // as many blocks as a list of the interface's points takes: where the
+        // surface has moved, or runs along a grid plane, a stage defers up to 10^4
+        // points, and a sweep is one long dependent chain.  A tenth of the blocks
+        // took 11-16 us a stage in the 96^3 relaxation, these 5.4 us; blocks that
+        // find no point leave at once (113x97x81, few points: 3.9 us either way)
+        k_reinit_deferred<T, S><<<dim3(iface_blocks(g)), dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g),
+                                                                            inv_of(g), stage, over, over_count, seq);
     return hipGetLastError();
 }
 

@@ -918,6 +918,17 @@ __device__ __forceinline__ void towers_h_delta(double& H, double& delta, const B
     delta = (pxx + pyy + pzz) / g2 - dot * t.lap / (g2 * t.g * t.g);
 }
 
+// one value of an output field, past the caches: the fields are written once
+// and together are larger than any cache (302 and 453 MB at 128^3).  At 128^3
+// the toolbox of F takes 90 us with plain stores and 65 with these (its 336 MB
+// at 5.2 TB/s), that of A 174 and 169, the tail that reads them 58 and 48.
+// Dividing through shared reciprocals gains 1% of this and is not done.
+template <typename O>
+__device__ __forceinline__ void put(const O& o, int k, idx_t ind, double v)
+{
+    __builtin_nontemporal_store(v, &o.f[k][ind]);
+}
+
 __global__ void __launch_bounds__(256) k_set_calculus_toolbox(Fields18 o, const double* __restrict__ lsf,
                                                               const double* __restrict__ hp, Box b, double ds)
 {
@@ -928,26 +939,26 @@ __global__ void __launch_bounds__(256) k_set_calculus_toolbox(Fields18 o, const 
     load_box27(F, lsf, r, c, p, b);
     load_box27(P, hp, r, c, p, b);
     const Toolbox t = toolbox_of(F, b, ds);
-    o.f[0][ind] = t.fx; o.f[1][ind] = t.fy; o.f[2][ind] = t.fz; o.f[3][ind] = t.g;
-    o.f[4][ind] = t.fx / t.g; o.f[5][ind] = t.fy / t.g; o.f[6][ind] = t.fz / t.g;
-    o.f[7][ind] = t.fxx; o.f[8][ind] = t.fyy; o.f[9][ind] = t.fzz;
-    o.f[10][ind] = t.fxy; o.f[11][ind] = t.fyz; o.f[12][ind] = t.fzx; o.f[13][ind] = t.lap;
+    put(o, 0, ind, t.fx); put(o, 1, ind, t.fy); put(o, 2, ind, t.fz); put(o, 3, ind, t.g);
+    put(o, 4, ind, t.fx / t.g); put(o, 5, ind, t.fy / t.g); put(o, 6, ind, t.fz / t.g);
+    put(o, 7, ind, t.fxx); put(o, 8, ind, t.fyy); put(o, 9, ind, t.fzz);
+    put(o, 10, ind, t.fxy); put(o, 11, ind, t.fyz); put(o, 12, ind, t.fzx); put(o, 13, ind, t.lap);
     double c1 = t.fxx * t.fx + t.fxy * t.fy + t.fzx * t.fz;
     double c2 = t.fxy * t.fx + t.fyy * t.fy + t.fyz * t.fz;
     double c3 = t.fzx * t.fx + t.fyz * t.fy + t.fzz * t.fz;
     const double g3 = t.g * t.g * t.g;
-    o.f[14][ind] = -t.lap / t.g + (t.fx * c1 + t.fy * c2 + t.fz * c3) / g3;
+    put(o, 14, ind, -t.lap / t.g + (t.fx * c1 + t.fy * c2 + t.fz * c3) / g3);
     c1 = (t.fyy * t.fzz - t.fyz * t.fyz) * t.fx + (t.fzx * t.fyz - t.fxy * t.fzz) * t.fy
          + (t.fxy * t.fyz - t.fzx * t.fyy) * t.fz;
     c2 = (t.fyz * t.fzx - t.fxy * t.fzz) * t.fx + (t.fxx * t.fzz - t.fzx * t.fzx) * t.fy
          + (t.fzx * t.fxy - t.fxx * t.fyz) * t.fz;
     c3 = (t.fxy * t.fyz - t.fyy * t.fzx) * t.fx + (t.fzx * t.fxy - t.fxx * t.fyz) * t.fy
          + (t.fxx * t.fyy - t.fxy * t.fxy) * t.fz;
-    o.f[15][ind] = (t.fx * c1 + t.fy * c2 + t.fz * c3) / (g3 * t.g);
+    put(o, 15, ind, (t.fx * c1 + t.fy * c2 + t.fz * c3) / (g3 * t.g));
     double H, delta;
     towers_h_delta(H, delta, P, t, b);
-    o.f[16][ind] = H;
-    o.f[17][ind] = delta;
+    put(o, 16, ind, H);
+    put(o, 17, ind, delta);
 }
 #undef T27
 
@@ -981,19 +992,19 @@ __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, c
     load_box27(Ab, A, r, c, p, b);
     load_box27(Pb, ahp, r, c, p, b);
     const Toolbox a = toolbox_of(Ab, b, ds);  // Ax..Azx, |grad A| = norm, ALaplacian
-    o.f[0][ind] = a.fx; o.f[1][ind] = a.fy; o.f[2][ind] = a.fz; o.f[3][ind] = a.g;
+    put(o, 0, ind, a.fx); put(o, 1, ind, a.fy); put(o, 2, ind, a.fz); put(o, 3, ind, a.g);
     const double fx = fin.f[0][ind], fy = fin.f[1][ind], fz = fin.f[2][ind], fg = fin.f[3][ind];
     double cx, cy, cz;
     cross3(cx, cy, cz, fx, fy, fz, a.fx, a.fy, a.fz);
     const double ncr = norm3(cx, cy, cz);
-    o.f[4][ind] = cx; o.f[5][ind] = cy; o.f[6][ind] = cz; o.f[7][ind] = ncr;
+    put(o, 4, ind, cx); put(o, 5, ind, cy); put(o, 6, ind, cz); put(o, 7, ind, ncr);
     const double tx = cx / ncr, ty = cy / ncr, tz = cz / ncr;
-    o.f[8][ind] = tx; o.f[9][ind] = ty; o.f[10][ind] = tz;
+    put(o, 8, ind, tx); put(o, 9, ind, ty); put(o, 10, ind, tz);
     double nx, ny, nz;
     cross3(nx, ny, nz, tx, ty, tz, fin.f[4][ind], fin.f[5][ind], fin.f[6][ind]);
-    o.f[11][ind] = nx; o.f[12][ind] = ny; o.f[13][ind] = nz;
-    o.f[14][ind] = a.fxx; o.f[15][ind] = a.fyy; o.f[16][ind] = a.fzz;
-    o.f[17][ind] = a.fxy; o.f[18][ind] = a.fyz; o.f[19][ind] = a.fzx; o.f[20][ind] = a.lap;
+    put(o, 11, ind, nx); put(o, 12, ind, ny); put(o, 13, ind, nz);
+    put(o, 14, ind, a.fxx); put(o, 15, ind, a.fyy); put(o, 16, ind, a.fzz);
+    put(o, 17, ind, a.fxy); put(o, 18, ind, a.fyz); put(o, 19, ind, a.fzx); put(o, 20, ind, a.lap);
     const double fxx = fin.f[7][ind], fyy = fin.f[8][ind], fzz = fin.f[9][ind];
     const double fxy = fin.f[10][ind], fyz = fin.f[11][ind], fzx = fin.f[12][ind];
     // geodesic curvature (auxi_set_calculus_toolbox.cu:115-131)
@@ -1007,7 +1018,7 @@ __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, c
     vz = tx * a.fzx + ty * a.fyz + tz * a.fzz;
     double w2x, w2y, w2z;
     cross3(w2x, w2y, w2z, fx, fy, fz, vx, vy, vz);
-    o.f[21][ind] = (nx * (w1x + w2x) + ny * (w1y + w2y) + nz * (w1z + w2z)) / ncr;
+    put(o, 21, ind, (nx * (w1x + w2x) + ny * (w1y + w2y) + nz * (w1z + w2z)) / ncr);
     // the shape operator of F's level sets, dN/dx (:135-145)
     const double g3 = fg * fg * fg;
     const double sx = fxx * fx + fxy * fy + fzx * fz;
@@ -1019,17 +1030,17 @@ __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, c
     vx = Nxx * tx + Nxy * ty + Nxz * tz;
     vy = Nyx * tx + Nyy * ty + Nyz * tz;
     vz = Nzx * tx + Nzy * ty + Nzz * tz;
-    o.f[22][ind] = -(tx * vx + ty * vy + tz * vz);
+    put(o, 22, ind, -(tx * vx + ty * vy + tz * vz));
     vx = Nxx * nx + Nxy * ny + Nxz * nz;
     vy = Nyx * nx + Nyy * ny + Nyz * nz;
     vz = Nzx * nx + Nzy * ny + Nzz * nz;
-    o.f[23][ind] = -(tx * vx + ty * vy + tz * vz);
-    o.f[24][ind] = -(nx * vx + ny * vy + nz * vz);
+    put(o, 23, ind, -(tx * vx + ty * vy + tz * vz));
+    put(o, 24, ind, -(nx * vx + ny * vy + nz * vz));
     // Heaviside and delta of A from its primal (:166-197)
     double H, delta;
     towers_h_delta(H, delta, Pb, a, b);
-    o.f[25][ind] = H;
-    o.f[26][ind] = delta;
+    put(o, 25, ind, H);
+    put(o, 26, ind, delta);
 }
 
 // periodic neighbour index of the @GD3 index maps (circshift, GD3.m:112-117)

@@ -219,8 +219,8 @@ struct vls_sdf3 {
     Dist6 fd{};       // distances of F inside the surface redistance
     uint8_t* fflags = nullptr;
     int* flist = nullptr;      // counts[2]
-    int* over = nullptr;       // reinitialization points deferred by the bulk pass
-    int* counts = nullptr;     // [0..2] list counts, [4..5] deferred counts
+    int* cand = nullptr;       // candidate points of a set_distance; crossing points of a stage Jacobian
+    int* counts = nullptr;     // [0..2] list counts, [3] candidate count, [4..5] crossing counts
     double* ldist[3] = {nullptr, nullptr, nullptr};  // list-order distances of d, ad, fd (6 rows of n)
     double* ldt[3] = {nullptr, nullptr, nullptr};    // list-order pseudo-time steps
     double* lcp = nullptr;   // interface values of the extended field, list order (6 rows of n)
@@ -296,22 +296,21 @@ int extend_loop(vls_sdf3* h, T* C, int iterations, const DSet& ds, hipStream_t s
     return VLS_OK;
 }
 
-// WENO5-RK3 reinitialization stages of one call share a sequence number for
-// the deferred-point counters (see launch_reinit_stage)
+// the stage Jacobians of one adjoint or tangent reinitialization share a
+// sequence number for their deferred-point counters (see launch_adj_reinit_jac)
 struct ReinitSeq {
     int* counts;
     int seq;
 };
 
 template <typename T>
-int reinit_stage(vls_sdf3* h, ReinitSeq& rs, T* out, const T* fs, const T* fn, const DSet& ds, int stage,
-                 hipStream_t s)
+int reinit_stage(vls_sdf3* h, T* out, const T* fs, const T* fn, const DSet& ds, int stage, hipStream_t s)
 {
-    VLS_HIP(launch_reinit_stage<T>(out, fs, fn, ds.flags, ds.lv, h->g, stage, h->over, rs.counts, rs.seq++, s));
+    VLS_HIP(launch_reinit_stage<T>(out, fs, fn, ds.flags, ds.lv, h->g, stage, s));
     return VLS_OK;
 }
 
-int reinit_begin(vls_sdf3* h, ReinitSeq& rs, hipStream_t s)
+int jac_begin(vls_sdf3* h, ReinitSeq& rs, hipStream_t s)
 {
     rs.counts = h->counts + 4;
     rs.seq = 0;
@@ -323,14 +322,13 @@ int reinit_begin(vls_sdf3* h, ReinitSeq& rs, hipStream_t s)
 template <typename T>
 int reinit_loop(vls_sdf3* h, T* F, int iterations, const DSet& ds, hipStream_t s)
 {
-    ReinitSeq rs;
     T* t0 = tmp<T>(h, 0);
     T* t1 = tmp<T>(h, 1);
-    int rc = reinit_begin(h, rs, s);
+    int rc = VLS_OK;
     for (int it = 0; it < iterations && rc == VLS_OK; ++it) {
-        if ((rc = reinit_stage<T>(h, rs, t0, F, nullptr, ds, 0, s))) break;
-        if ((rc = reinit_stage<T>(h, rs, t1, t0, F, ds, 1, s))) break;
-        rc = reinit_stage<T>(h, rs, F, t1, F, ds, 2, s);
+        if ((rc = reinit_stage<T>(h, t0, F, nullptr, ds, 0, s))) break;
+        if ((rc = reinit_stage<T>(h, t1, t0, F, ds, 1, s))) break;
+        rc = reinit_stage<T>(h, F, t1, F, ds, 2, s);
     }
     return rc;
 }
@@ -338,14 +336,14 @@ int reinit_loop(vls_sdf3* h, T* F, int iterations, const DSet& ds, hipStream_t s
 // the distances of F into the set `ds`: flags and interface list always;
 // the dense arrays (six distances, and min_dist if given) only if `dense`
 // (the kernels of the WENO5 path read the list; the ENO2 and cubic variants
-// read the dense arrays).  The candidate points go through h->over and
-// h->counts[3], free outside a reinitialization call.
+// read the dense arrays).  The candidate points go through h->cand and
+// h->counts[3].
 template <typename T>
 int set_distance_into(vls_sdf3* h, int order, const DSet& ds, double* min_dist, const T* F, const T* mask_src,
                       bool dense, hipStream_t s)
 {
     const Dist6 d = dense ? ds.d : Dist6{};
-    VLS_HIP(launch_set_distance<T>(order, d, dense ? min_dist : nullptr, ds.flags, mask_src, F, ds.lv, h->over,
+    VLS_HIP(launch_set_distance<T>(order, d, dense ? min_dist : nullptr, ds.flags, mask_src, F, ds.lv, h->cand,
                                    h->counts + 3, h->g, s));
     return VLS_OK;
 }
@@ -427,15 +425,13 @@ int surface_redistance_issue(vls_sdf3* h, const T* F, T* A, int iter1, int iter2
     VLS_HIP(launch_list_gather_vel<T>(h->lvel, fs.lv, vx, vy, vz, g, s));
     T* a1 = tmp<T>(h, 2);
     T* a05 = tmp<T>(h, 3);
-    ReinitSeq rs;
-    if ((rc = reinit_begin(h, rs, s))) return rc;
     for (int it = 0; it < iter1; ++it) {
         if ((rc = extend_loop<T>(h, A, iter2, fs, s))) return rc;
-        if ((rc = reinit_stage<T>(h, rs, a1, A, nullptr, as, 0, s))) return rc;
+        if ((rc = reinit_stage<T>(h, a1, A, nullptr, as, 0, s))) return rc;
         if ((rc = extend_loop<T>(h, a1, iter2, fs, s))) return rc;
-        if ((rc = reinit_stage<T>(h, rs, a05, a1, A, as, 1, s))) return rc;
+        if ((rc = reinit_stage<T>(h, a05, a1, A, as, 1, s))) return rc;
         if ((rc = extend_loop<T>(h, a05, iter2, fs, s))) return rc;
-        if ((rc = reinit_stage<T>(h, rs, A, a05, A, as, 2, s))) return rc;
+        if ((rc = reinit_stage<T>(h, A, a05, A, as, 2, s))) return rc;
     }
     return extend_loop<T>(h, A, iter2, fs, s);
 }
@@ -518,7 +514,7 @@ int area_volume(vls_sdf3* h, int kind, const T* F, double eps, double* dev_out, 
 // when it loads the code object on a device and it stays until the process
 // ends.  Per grid point: the list-order distances (six rows) and
 // pseudo-time steps, two RK stage fields (9 doubles), the interface list and
-// the deferred points (2 ints) and the flags (1 byte); 16 counters; every
+// its candidate points (2 ints) and the flags (1 byte); 16 counters; every
 // piece starts on a 256-byte boundary.
 constexpr int kStaticPieces = 8;
 constexpr size_t kStaticBytes =
@@ -1006,7 +1002,7 @@ int vls_sdf3_create(vls_sdf3_t* out, int rows, int cols, int pges, double dx, do
     h->list = h->int_pool;
     h->alist = h->int_pool + n;
     h->flist = h->int_pool + 2 * n;
-    h->over = h->int_pool + 3 * n;
+    h->cand = h->int_pool + 3 * n;
     h->counts = h->int_pool + 4 * n;
     *out = h;
     return VLS_OK;
@@ -1129,7 +1125,7 @@ int vls_weno5_rk3_reinit_static(double* F, int iterations, int rows, int cols, i
     h.t[0] = reinterpret_cast<double*>(take(sizeof(double) * n));
     h.t[1] = reinterpret_cast<double*>(take(sizeof(double) * n));
     h.list = reinterpret_cast<int*>(take(sizeof(int) * n));
-    h.over = reinterpret_cast<int*>(take(sizeof(int) * n));
+    h.cand = reinterpret_cast<int*>(take(sizeof(int) * n));
     h.counts = reinterpret_cast<int*>(take(sizeof(int) * 16));
     h.flags = take((size_t)n);
     VLS_REQUIRE(used <= kStaticBytes, "static work memory layout overflows (%zu > %zu bytes)", used, kStaticBytes);
@@ -1184,12 +1180,10 @@ int vls_sdf3_wenork3_reinit(vls_sdf3_t h, double* F, int iterations, vls_stream_
         int rc = set_distance_into<double>(h, 3, as, nullptr, F, F, false, s);
         if (rc) return rc;
         double *t0 = h->t[0], *t1 = h->t[1];
-        ReinitSeq rs;
-        if ((rc = reinit_begin(h, rs, s))) return rc;
         for (int it = 0; it < iterations; ++it) {
-            VLS_HIP(launch_cubic_reinit_stage(t0, F, nullptr, as.flags, as.lv, g, 0, h->over, rs.counts, rs.seq++, s));
-            VLS_HIP(launch_cubic_reinit_stage(t1, t0, F, as.flags, as.lv, g, 1, h->over, rs.counts, rs.seq++, s));
-            VLS_HIP(launch_cubic_reinit_stage(F, t1, F, as.flags, as.lv, g, 2, h->over, rs.counts, rs.seq++, s));
+            VLS_HIP(launch_cubic_reinit_stage(t0, F, nullptr, as.flags, as.lv, g, 0, s));
+            VLS_HIP(launch_cubic_reinit_stage(t1, t0, F, as.flags, as.lv, g, 1, s));
+            VLS_HIP(launch_cubic_reinit_stage(F, t1, F, as.flags, as.lv, g, 2, s));
         }
         return VLS_OK;
     });
@@ -1364,6 +1358,7 @@ struct vls_batch {
     int tr = 64;     // rows per tile
     int zd = 8;      // pages per work item of the z-marching bulk stage kernels
     int nitems = 0;
+    int item_pages = 0;  // most pages of an item
     ZItem* d_items = nullptr;
     std::vector<BGrid> grids;
     std::vector<int64_t> offs;
@@ -1374,9 +1369,9 @@ struct vls_batch {
     uint8_t* flags = nullptr;
     int* int_pool = nullptr;
     ListView lv{};
-    int* over = nullptr;
+    int* cand = nullptr;       // candidate points of the list build
     int* list_grid = nullptr;  // grid of each interface-list entry
-    int* counts = nullptr;     // [0] list count, [3] candidate count of the list build, [4..5] deferred counts
+    int* counts = nullptr;     // [0] list count, [3] candidate count of the list build
     double* lcp = nullptr;
     double* lvel = nullptr;
     double* t[2] = {nullptr, nullptr};
@@ -1387,7 +1382,8 @@ struct vls_batch {
 
     BatchView view() const
     {
-        return BatchView{d_grids, d_tile_grid, d_offs, ngrids, ntiles, blocks, tr, d_items, nitems, list_grid};
+        return BatchView{d_grids, d_tile_grid, d_offs,  ngrids, ntiles,   blocks,
+                         tr,      item_pages,  d_items, nitems, list_grid};
     }
     ~vls_batch()
     {
@@ -1432,12 +1428,14 @@ int build_tiles(vls_batch* b, int tr)
     // z-march work list: per grid, per chunk of zd pages, the tile columns
     // (neighbouring columns adjacent, so consecutive blocks share halos)
     std::vector<ZItem> items;
+    int item_pages = 0;
     const int tc = 256 / tr;
     for (int g = 0; g < b->ngrids; ++g) {
         const BGrid& G = b->grids[(size_t)g];
         const int ntr = (G.rows + tr - 1) / tr, ntc = (G.cols + tc - 1) / tc;
         // the pages in equal chunks of at most zd
         const int nch = (G.pges + b->zd - 1) / b->zd;
+        item_pages = std::max(item_pages, (G.pges + nch - 1) / nch);
         for (int ch = 0; ch < nch; ++ch)
             for (int cb = 0; cb < ntc; ++cb)
                 for (int rb = 0; rb < ntr; ++rb)
@@ -1458,6 +1456,7 @@ int build_tiles(vls_batch* b, int tr)
     VLS_HIP(hipMemcpy(b->d_grids, b->grids.data(), sizeof(BGrid) * (size_t)b->ngrids, hipMemcpyHostToDevice));
     b->ntiles = (int)tiles;
     b->nitems = (int)items.size();
+    b->item_pages = item_pages;
     b->tr = tr;
     return VLS_OK;
 }
@@ -1477,7 +1476,7 @@ template <typename T>
 int batch_set_distance(vls_batch* b, const T* F, const T* mask_src, hipStream_t s)
 {
     VLS_HIP(launch_zero_ints(b->counts, 4, s));  // the list count and the candidate count (counts[3])
-    VLS_HIP(launch_batch_build_list<T>(b->view(), F, mask_src, b->flags, b->lv, 6, b->over, b->counts + 3, s));
+    VLS_HIP(launch_batch_build_list<T>(b->view(), F, mask_src, b->flags, b->lv, 6, b->cand, b->counts + 3, s));
     return VLS_OK;
 }
 
@@ -1485,16 +1484,13 @@ template <typename T>
 int batch_reinit_loop(vls_batch* b, T* F, int iterations, hipStream_t s)
 {
     const BatchView B = b->view();
-    int* oc = b->counts + 4;
     T* t0 = btmp<T>(b, 0);
     T* t1 = btmp<T>(b, 1);
     VLS_HIP(launch_batch_set_mask_bit<T>(b->flags, F, b->total, s));
-    VLS_HIP(launch_zero_ints(oc, 2, s));
-    int seq = 0;
     for (int it = 0; it < iterations; ++it) {
-        VLS_HIP(launch_batch_reinit_stage<T>(B, t0, F, nullptr, b->flags, b->lv, 0, b->over, oc, seq++, s));
-        VLS_HIP(launch_batch_reinit_stage<T>(B, t1, t0, F, b->flags, b->lv, 1, b->over, oc, seq++, s));
-        VLS_HIP(launch_batch_reinit_stage<T>(B, F, t1, F, b->flags, b->lv, 2, b->over, oc, seq++, s));
+        VLS_HIP(launch_batch_reinit_stage<T>(B, t0, F, nullptr, b->flags, b->lv, 0, s));
+        VLS_HIP(launch_batch_reinit_stage<T>(B, t1, t0, F, b->flags, b->lv, 1, s));
+        VLS_HIP(launch_batch_reinit_stage<T>(B, F, t1, F, b->flags, b->lv, 2, s));
     }
     return VLS_OK;
 }
@@ -1558,20 +1554,14 @@ int batch_step(vls_batch* b, T* F, T* Vn, const T* vx, const T* vy, const T* vz,
 int batch_wenork3_reinit(vls_batch* b, double* F, int iterations, hipStream_t s)
 {
     const BatchView B = b->view();
-    int* oc = b->counts + 4;
     double* t0 = btmp<double>(b, 0);
     double* t1 = btmp<double>(b, 1);
     VLS_HIP(launch_zero_ints(b->counts, 4, s));
-    VLS_HIP(launch_batch_build_list<double>(B, F, F, b->flags, b->lv, 3, b->over, b->counts + 3, s));
-    VLS_HIP(launch_zero_ints(oc, 2, s));
-    int seq = 0;
+    VLS_HIP(launch_batch_build_list<double>(B, F, F, b->flags, b->lv, 3, b->cand, b->counts + 3, s));
     for (int it = 0; it < iterations; ++it) {
-        VLS_HIP(launch_batch_reinit_stage<double>(B, t0, F, nullptr, b->flags, b->lv, 0, b->over, oc, seq++, s,
-                                                  IFACE_CUBIC));
-        VLS_HIP(launch_batch_reinit_stage<double>(B, t1, t0, F, b->flags, b->lv, 1, b->over, oc, seq++, s,
-                                                  IFACE_CUBIC));
-        VLS_HIP(launch_batch_reinit_stage<double>(B, F, t1, F, b->flags, b->lv, 2, b->over, oc, seq++, s,
-                                                  IFACE_CUBIC));
+        VLS_HIP(launch_batch_reinit_stage<double>(B, t0, F, nullptr, b->flags, b->lv, 0, s, IFACE_CUBIC));
+        VLS_HIP(launch_batch_reinit_stage<double>(B, t1, t0, F, b->flags, b->lv, 1, s, IFACE_CUBIC));
+        VLS_HIP(launch_batch_reinit_stage<double>(B, F, t1, F, b->flags, b->lv, 2, s, IFACE_CUBIC));
     }
     return VLS_OK;
 }
@@ -1591,7 +1581,7 @@ int batch_variant_extend(vls_batch* b, const double* F, double* C, int iteration
     double* t1 = btmp<double>(b, 1);
     const int scheme = weno ? 1 : 2;  // the cubic ENO, the quadratic ENO
     VLS_HIP(launch_zero_ints(b->counts, 4, s));
-    VLS_HIP(launch_batch_build_list<double>(B, F, nullptr, b->flags, b->lv, weno ? 3 : 2, b->over, b->counts + 3,
+    VLS_HIP(launch_batch_build_list<double>(B, F, nullptr, b->flags, b->lv, weno ? 3 : 2, b->cand, b->counts + 3,
                                             s));
     VLS_HIP(launch_batch_extension_velocity<double>(B, vx, vy, vz, F, b->flags, b->lv, 1e-6, s, scheme));
     VLS_HIP(launch_batch_list_interp<double>(B, b->lcp, b->lv, C, s, scheme));
@@ -1698,7 +1688,7 @@ int vls_batch_create(vls_batch_t* out, int ngrids, const int* rows, const int* c
     for (int k = 0; k < 2; ++k) { b->t[k] = p; p += n; }
     for (int a = 0; a < 3; ++a) { b->v[a] = p; p += n; }
     b->lv.idx = b->int_pool;
-    b->over = b->int_pool + n;
+    b->cand = b->int_pool + n;
     b->list_grid = b->int_pool + 2 * n;
     b->counts = b->int_pool + 3 * n;
     b->lv.count = b->counts;
@@ -2251,27 +2241,27 @@ int vls_sdf3_adjoint_reinit(vls_sdf3_t h, const double* F0, int iterations, cons
     VLS_HIP(launch_set_mask_bit<double>(h->flags, F0, g, s));
     VLS_HIP(launch_copy<double>(X, F0, n, s));
     ReinitSeq rs;
-    if ((rc = reinit_begin(h, rs, s))) return rc;
+    if ((rc = jac_begin(h, rs, s))) return rc;
     for (int k = 0; k < K; ++k) {
         double* xk = X + (size_t)k * n;
-        if ((rc = reinit_stage<double>(h, rs, T0 + (size_t)k * n, xk, nullptr, ms, 0, s))) return rc;
-        if ((rc = reinit_stage<double>(h, rs, T1 + (size_t)k * n, T0 + (size_t)k * n, xk, ms, 1, s))) return rc;
-        if ((rc = reinit_stage<double>(h, rs, xk + n, T1 + (size_t)k * n, xk, ms, 2, s))) return rc;
+        if ((rc = reinit_stage<double>(h, T0 + (size_t)k * n, xk, nullptr, ms, 0, s))) return rc;
+        if ((rc = reinit_stage<double>(h, T1 + (size_t)k * n, T0 + (size_t)k * n, xk, ms, 1, s))) return rc;
+        if ((rc = reinit_stage<double>(h, xk + n, T1 + (size_t)k * n, xk, ms, 2, s))) return rc;
     }
     VLS_HIP(launch_copy<double>(lam, lam_out, n, s));
     VLS_HIP(launch_adj_fill(lamP, 0.0, 7 * n, s));
     for (int k = K - 1; k >= 0; --k) {
         const double* xk = X + (size_t)k * n;
         // stage 2: X[k+1] = S2(T1[k]; X[k])
-        VLS_HIP(launch_adj_reinit_jac(J, lamP, lam, T1 + (size_t)k * n, h->flags, ms.lv, g, 2, h->over, rs.counts,
+        VLS_HIP(launch_adj_reinit_jac(J, lamP, lam, T1 + (size_t)k * n, h->flags, ms.lv, g, 2, h->cand, rs.counts,
                                       rs.seq++, s));
         VLS_HIP(launch_adj_transpose(lt1, J, g, 0.0, nullptr, 0.0, nullptr, s));
         // stage 1: T1[k] = S1(T0[k]; X[k])
-        VLS_HIP(launch_adj_reinit_jac(J, lamP, lt1, T0 + (size_t)k * n, h->flags, ms.lv, g, 1, h->over, rs.counts,
+        VLS_HIP(launch_adj_reinit_jac(J, lamP, lt1, T0 + (size_t)k * n, h->flags, ms.lv, g, 1, h->cand, rs.counts,
                                       rs.seq++, s));
         VLS_HIP(launch_adj_transpose(lt0, J, g, 0.0, nullptr, 0.0, nullptr, s));
         // stage 0: T0[k] = S0(X[k]); X[k] also enters stages 1 and 2 as the start value
-        VLS_HIP(launch_adj_reinit_jac(J, lamP, lt0, xk, h->flags, ms.lv, g, 0, h->over, rs.counts, rs.seq++, s));
+        VLS_HIP(launch_adj_reinit_jac(J, lamP, lt0, xk, h->flags, ms.lv, g, 0, h->cand, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_transpose(lam, J, g, stage_e(2), lam, stage_e(1), lt1, s));
     }
     VLS_HIP(launch_copy<double>(lam_in, lam, n, s));
@@ -2310,22 +2300,22 @@ int vls_sdf3_tangent_reinit(vls_sdf3_t h, const double* F0, const double* F0dot,
     VLS_HIP(launch_copy<double>(X, F0, n, s));
     VLS_HIP(launch_copy<double>(Xd, F0dot, n, s));
     ReinitSeq rs;
-    if ((rc = reinit_begin(h, rs, s))) return rc;
+    if ((rc = jac_begin(h, rs, s))) return rc;
     for (int k = 0; k < iterations; ++k) {
-        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, X, h->flags, ms.lv, g, 0, h->over, rs.counts, rs.seq++, s));
+        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, X, h->flags, ms.lv, g, 0, h->cand, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_apply(d0, J, Xd, g, s));
         VLS_HIP(launch_adj_param_tangent(d0, JP, Pd, ms.lv, s));
-        if ((rc = reinit_stage<double>(h, rs, t0, X, nullptr, ms, 0, s))) return rc;
-        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, t0, h->flags, ms.lv, g, 1, h->over, rs.counts, rs.seq++, s));
+        if ((rc = reinit_stage<double>(h, t0, X, nullptr, ms, 0, s))) return rc;
+        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, t0, h->flags, ms.lv, g, 1, h->cand, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_apply(d1, J, d0, g, s));
         VLS_HIP(launch_adj_axpby(d1, Xd, stage_e(1), 1.0, n, s));
         VLS_HIP(launch_adj_param_tangent(d1, JP, Pd, ms.lv, s));
-        if ((rc = reinit_stage<double>(h, rs, t1, t0, X, ms, 1, s))) return rc;
-        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, t1, h->flags, ms.lv, g, 2, h->over, rs.counts, rs.seq++, s));
+        if ((rc = reinit_stage<double>(h, t1, t0, X, ms, 1, s))) return rc;
+        VLS_HIP(launch_adj_reinit_jac(J, JP, nullptr, t1, h->flags, ms.lv, g, 2, h->cand, rs.counts, rs.seq++, s));
         VLS_HIP(launch_adj_apply(d0, J, d1, g, s));
         VLS_HIP(launch_adj_axpby(d0, Xd, stage_e(2), 1.0, n, s));
         VLS_HIP(launch_adj_param_tangent(d0, JP, Pd, ms.lv, s));
-        if ((rc = reinit_stage<double>(h, rs, X, t1, X, ms, 2, s))) return rc;
+        if ((rc = reinit_stage<double>(h, X, t1, X, ms, 2, s))) return rc;
         VLS_HIP(launch_copy<double>(Xd, d0, n, s));
     }
     VLS_HIP(launch_copy<double>(Fout, X, n, s));

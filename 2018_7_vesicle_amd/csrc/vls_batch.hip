@@ -182,74 +182,73 @@ __global__ void kb_set_mask_bit(uint8_t* __restrict__ flags, const T* __restrict
 // k_extend_stage): the first niface blocks walk the interface list, the
 // others take one z-march work item each (a tile column of one grid over a
 // range of its pages) with the single-grid kernels' walk and per-point
-// bodies, called with the item's grid.
+// bodies, called with the item's grid.  An FP64 reinitialization block takes
+// kDeferPages pages at most, so an item is split over reinit_parts blocks.
+// B.grids[...] and the lane's point are picked before one call of the lane
+// code: a call for each kind of block spilled 3 values a page of the march.
 template <int R, typename T, int S = IFACE_WENO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) kb_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                        const T* __restrict__ fn, const uint8_t* __restrict__ flags,
-                                                       IList il, BatchView B, int stage, int* __restrict__ over,
-                                                       int* __restrict__ over_count, int seq, int niface)
+                                                       IList il, BatchView B, int stage, int niface)
 {
     __shared__ T lds[2][Shape<R>::N];
+    __shared__ unsigned short job[defers_crossings<T>() ? 256 * kDeferPages : 1];
+    __shared__ int njobs;
     const int blk = (int)blockIdx.x;
-    if (blk == 0 && threadIdx.x == 0) over_count[(seq + 1) & 1] = 0;
-    if (blk < niface) {
-        const int total = *il.count;
-        for (int j0 = 0; j0 < total; j0 += axis_lane_stride(niface)) {
-            const AxisLane al = axis_lane(j0, blk);
-            const bool active = al.point >= 0 && al.point < total;
-            ReinitLane q;
-            if (active) {
-                const int64_t gind = il.idx[al.point];
-                const BGrid G = B.grids[B.list_grid[al.point]];
-                q = reinit_iface_lane<T, S>(fs + G.off, flags + G.off, box_of(G), inv_of(G), il, al.point,
-                                            gind - G.off, gind, al.axis);
-            }
-            reinit_iface_finish(out, fs, fn, q, al, active, stage);
-        }
-        return;
-    }
-    const ZItem it = B.items[xcd_remap(blk - niface, (int)gridDim.x - niface)];
+    const bool lists = blk < niface;  // this block walks the interface list
+    const int parts = reinit_parts<T>(B.zd), wi = lists ? 0 : xcd_remap(blk - niface, (int)gridDim.x - niface);
+    const ZItem it = lists ? ZItem{0, 0, 0, 0, 1} : B.items[wi / parts];
     const BGrid G = B.grids[it.g];
     const Box b = box_of(G);
     const Inv invs = inv_of(G);
     const idx_t off = G.off, plane = (idx_t)b.rows * b.cols;
+    const int r0 = it.r0, c0 = it.c0, part = wi % parts, np = it.p1 - it.p0;
+    const int p0 = it.p0 + part * np / parts, p1 = it.p0 + (part + 1) * np / parts;
     T* o = out + off;
-    ZFace<T> zf;
-    zmarch<R, T, false, true>(lds[0], lds[1], b, it.r0, it.c0, it.p0, it.p1, fs + off, shift(fn, off), nullptr, nullptr,
-                        nullptr, flags + off, stage,
-                        [&](const T* w6) { zface_start(zf, w6, axis_arg(invs, 2, T())); },
-                        [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st, int p) {
-                            bool cross;
-                            const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs, stage, cross, zf);
-                            const bool bulk = !(st.flags(zc) & FLAG_SUBCELL);
-                            if constexpr (defers_crossings<T>()) {
-                                if (bulk && !cross) stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
-                                wave_append(bulk && cross, (int)(off + (idx_t)p * plane + zc.in), over,
-                                            &over_count[seq & 1]);
-                            } else if (bulk) {
-                                stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
-                            }
-                        });
-}
-
-// launch 2 of 2: the deferred bulk points (see k_reinit_deferred)
-template <typename T, int S = IFACE_WENO>
-__global__ void __launch_bounds__(256) kb_reinit_deferred(T* __restrict__ out, const T* __restrict__ fs,
-                                                          const T* __restrict__ fn, const uint8_t* __restrict__ flags,
-                                                          IList il, BatchView B, int stage,
-                                                          const int* __restrict__ over,
-                                                          const int* __restrict__ over_count, int seq)
-{
-    const int total = over_count[seq & 1];
-    for (int j0 = 0; j0 < total; j0 += axis_lane_stride()) {
-        const AxisLane al = axis_lane(j0);
+    if (!lists) {
+        if (threadIdx.x == 0) njobs = 0;  // before the march's first barrier
+        ZFace<T> zf;
+        zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, fs + off, shift(fn, off), nullptr, nullptr,
+                                  nullptr, flags + off, stage,
+                                  [&](const T* w6) { zface_start(zf, w6, axis_arg(invs, 2, T())); },
+                                  [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st,
+                                      int p) {
+                                      bool cross;
+                                      const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs,
+                                                                    stage, cross, zf);
+                                      const bool bulk = !(st.flags(zc) & FLAG_SUBCELL);
+                                      if (bulk && !cross) stb<T>(page_of(o, (idx_t)p * plane), zc.in, res);
+                                      if constexpr (defers_crossings<T>())
+                                          if (bulk && cross)
+                                              job[atomicAdd(&njobs, 1)] =
+                                                  (unsigned short)((p - p0) << 8 | (int)threadIdx.x);
+                                  });
+        if constexpr (!defers_crossings<T>()) return;
+        __syncthreads();
+    }
+    const int total = lists ? *il.count : njobs, first = lists ? blk * axis_lane_stride(1) : 0;
+    for (int j0 = first; j0 < total; j0 += lists ? axis_lane_stride(niface) : axis_lane_stride(1)) {
+        const AxisLane al = axis_lane(j0, 0);
         const bool active = al.point >= 0 && al.point < total;
         ReinitLane q;
         if (active) {
-            const int64_t gind = over[al.point];
-            const BGrid G = B.grids[grid_of(B, gind)];
-            q = reinit_iface_lane<T, S>(fs + G.off, flags + G.off, box_of(G), inv_of(G), il, -1, gind - G.off,
-                                        gind, al.axis);
+            int r, c, p, slot = -1;
+            if (lists) slot = al.point;
+            const BGrid L = B.grids[lists ? B.list_grid[al.point] : it.g];
+            const Box lb = box_of(L);
+            idx_t ind;
+            if (lists) {
+                ind = (idx_t)il.idx[slot] - L.off;
+                coords_of(lb, ind, r, c, p);
+            } else {
+                const int e = job[al.point], th = e & 255;
+                r = r0 + th % R;
+                c = c0 + th / R;
+                p = p0 + (e >> 8);
+                ind = lin(lb, r, c, p);
+            }
+            q = reinit_iface_lane<T, S>(fs + L.off, flags + L.off, lb, inv_of(L), il, slot, r, c, p, ind,
+                                        L.off + ind, al.axis);
         }
         reinit_iface_finish(out, fs, fn, q, al, active, stage);
     }
@@ -819,28 +818,22 @@ hipError_t launch_batch_set_mask_bit(uint8_t* flags, const T* F, int64_t n, hipS
 
 template <typename T>
 hipError_t launch_batch_reinit_stage(const BatchView& B, T* out, const T* fs, const T* fn, const uint8_t* flags,
-                                     const ListView& lv, int stage, int* over, int* over_count, int seq,
-                                     hipStream_t s, int scheme)
+                                     const ListView& lv, int stage, hipStream_t s, int scheme)
 {
-    const int ni = fused_list_blocks(B);
+    const int ni = fused_list_blocks(B), nb = B.nitems * reinit_parts<T>(B.zd) + ni;
     if constexpr (std::is_same<T, double>::value) {
         if (scheme == IFACE_CUBIC) {
             if (B.tr == 32)
-                kb_reinit_stage<32, T, IFACE_CUBIC><<<B.nitems + ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B,
-                                                                                  stage, over, over_count, seq, ni);
+                kb_reinit_stage<32, T, IFACE_CUBIC><<<nb, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B,
+                                                                                  stage, ni);
             else
-                kb_reinit_stage<64, T, IFACE_CUBIC><<<B.nitems + ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B,
-                                                                                  stage, over, over_count, seq, ni);
-            kb_reinit_deferred<T, IFACE_CUBIC><<<ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B, stage,
-                                                                    (const int*)over, (const int*)over_count, seq);
+                kb_reinit_stage<64, T, IFACE_CUBIC><<<nb, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B,
+                                                                                  stage, ni);
             return hipGetLastError();
         }
     }
     if (scheme != IFACE_WENO) return hipErrorInvalidValue;
-    TR_LAUNCH(kb_reinit_stage, T, B.nitems + ni, out, fs, fn, flags, ilist(lv), B, stage, over, over_count, seq, ni);
-    if constexpr (defers_crossings<T>())
-        kb_reinit_deferred<T><<<ni, 256, 0, s>>>(out, fs, fn, flags, ilist(lv), B, stage, (const int*)over,
-                                                   (const int*)over_count, seq);
+    TR_LAUNCH(kb_reinit_stage, T, nb, out, fs, fn, flags, ilist(lv), B, stage, ni);
     return hipGetLastError();
 }
 
@@ -985,7 +978,7 @@ hipError_t launch_batch_ellipsoid(const BatchView& B, T* F, const double* axes, 
                                                    int, int*, int*, hipStream_t);                                   \
     template hipError_t launch_batch_set_mask_bit<T>(uint8_t*, const T*, int64_t, hipStream_t);                     \
     template hipError_t launch_batch_reinit_stage<T>(const BatchView&, T*, const T*, const T*, const uint8_t*,      \
-                                                     const ListView&, int, int*, int*, int, hipStream_t, int);      \
+                                                     const ListView&, int, hipStream_t, int);                       \
     template hipError_t launch_batch_extend_stage<T>(const BatchView&, T*, const T*, const T*, const T*, const T*,  \
                                                      const T*, const ListView&, const double*, const double*, int,  \
                                                      hipStream_t, int);                                             \

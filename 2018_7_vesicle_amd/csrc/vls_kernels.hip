@@ -322,85 +322,73 @@ __global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, cons
     step[ind] = reinit_residual(lsf, r, c, p, b, q, mask[ind] != 0, deltat[ind]);
 }
 
-// ---------------------------------------------------------------------------
-// split stage kernels.  Bulk kernels cover the box in 64x4 (rows x cols)
-// tiles of one page and take every point without subcell distances through
-// uniform WENO5 only (few registers, high occupancy); interface kernels
-// stride over a list of points and evaluate the full residual.
-// ---------------------------------------------------------------------------
-
-
-
-// Fused WENO5-RK3 reinitialization stage, launch 1 of 2: the first niface
-// blocks walk the interface list with three lanes per point (the full
-// residual with subcell distances), the others z-march over every point
-// without subcell distances.  The list blocks are dispatched first, so their
-// long dependent chains (the nonuniform WENO divides ~30 times per face) run
-// beside the bulk instead of after it.  In FP64 a bulk point whose stage
-// field changes sign beside it takes the reference's nonuniform stencil: it
-// is appended to `over`, counted in over_count[seq & 1], for launch 2; the
-// other slot is cleared here for the next stage.  FP32 evaluates such a
-// point in the bulk (defers_crossings) and has no launch 2.
+// Fused WENO5-RK3 reinitialization stage, one launch: the first niface blocks
+// walk the interface list with three lanes per point (the full residual with
+// subcell distances), the others z-march over every point without subcell
+// distances.  The list blocks are dispatched first, so their long dependent
+// chains (the nonuniform WENO divides ~30 times per face) run beside the bulk
+// instead of after it.  In FP64 a bulk point whose stage field changes sign
+// beside it takes the reference's nonuniform stencil (defers_crossings): its
+// block lists it in LDS and evaluates its few such points after the march, on
+// the list blocks' code.  A second launch for them took 3.9 us a stage where
+// there were a handful and 5.4 us for the 10^4 of a flat vesicle, a sixth of the
+// stage; 60 stages x 113x97x81 took 1340 us with it and take 1174 us, 300 x
+// 96^3 in the relaxation 7.4 ms and 7.0 ms.  The list blocks' code has to come
+// after the march as straight text: inside a loop over parts of the pages its
+// constants are hoisted into the march, which then spills (1377 us).
 template <int R, typename T, int S = IFACE_WENO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                       const T* __restrict__ fn, const uint8_t* __restrict__ flags,
-                                                      IList il, Box b, Inv invs, int stage, int* __restrict__ over,
-                                                      int* __restrict__ over_count, int seq, int depth, int niface)
+                                                      IList il, Box b, Inv invs, int stage, int depth, int niface)
 {
     __shared__ T lds[2][Shape<R>::N];
+    __shared__ unsigned short job[defers_crossings<T>() ? 256 * kDeferPages : 1];
+    __shared__ int njobs;
     const int blk = (int)blockIdx.x;
-    if (blk == 0 && threadIdx.x == 0) over_count[(seq + 1) & 1] = 0;
-    if (blk < niface) {
-        const int total = *il.count;
-        for (int j0 = 0; j0 < total; j0 += axis_lane_stride(niface)) {
-            const AxisLane al = axis_lane(j0, blk);
-            const bool active = al.point >= 0 && al.point < total;
-            ReinitLane q;
-            if (active) {
-                const idx_t ind = (idx_t)il.idx[al.point];
-                q = reinit_iface_lane<T, S>(fs, flags, b, invs, il, al.point, ind, ind, al.axis);
-            }
-            reinit_iface_finish(out, fs, fn, q, al, active, stage);
-        }
-        return;
-    }
-    int r0, c0, p0, p1;
-    zmarch_share<R>(b, depth, blk - niface, (int)gridDim.x - niface, r0, c0, p0, p1);
+    const bool lists = blk < niface;  // this block walks the interface list
     const idx_t plane = (idx_t)b.rows * b.cols;
-    ZFace<T> zf;
-    zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, fs, fn, nullptr, nullptr, nullptr, flags, stage,
-                        [&](const T* w6) { zface_start(zf, w6, axis_arg(invs, 2, T())); },
-                        [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st, int p) {
-                            bool cross;
-                            const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs, stage, cross, zf);
-                            const bool bulk = !(st.flags(zc) & FLAG_SUBCELL);
-                            if constexpr (defers_crossings<T>()) {
-                                if (bulk && !cross) stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
-                                wave_append(bulk && cross, (int)((idx_t)p * plane + zc.in), over,
-                                            &over_count[seq & 1]);
-                            } else if (bulk) {
-                                stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
-                            }
-                        });
-}
-
-// launch 2 of 2: the deferred bulk points, three lanes per point, with the
-// interface pass's arithmetic (spacing distances, the bulk pseudo-time step)
-template <typename T, int S = IFACE_WENO>
-__global__ void __launch_bounds__(256) k_reinit_deferred(T* __restrict__ out, const T* __restrict__ fs,
-                                                         const T* __restrict__ fn, const uint8_t* __restrict__ flags,
-                                                         IList il, Box b, Inv inv, int stage,
-                                                         const int* __restrict__ over,
-                                                         const int* __restrict__ over_count, int seq)
-{
-    const int total = over_count[seq & 1];
-    for (int j0 = 0; j0 < total; j0 += axis_lane_stride()) {
-        const AxisLane al = axis_lane(j0);
+    int r0 = 0, c0 = 0, p0 = 0, p1 = 0;
+    if (!lists) {
+        zmarch_share<R>(b, depth, blk - niface, (int)gridDim.x - niface, r0, c0, p0, p1);
+        if (threadIdx.x == 0) njobs = 0;  // before the march's first barrier
+        ZFace<T> zf;
+        zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, fs, fn, nullptr, nullptr, nullptr, flags, stage,
+                                  [&](const T* w6) { zface_start(zf, w6, axis_arg(invs, 2, T())); },
+                                  [&](const T* l, const ZCol<R>& zc, const T w[7], const ZStep<R, T, false>& st,
+                                      int p) {
+                                      bool cross;
+                                      const T res = reinit_value<R>(l, zc.base, w, st.fn, st.flags(zc), invs,
+                                                                    stage, cross, zf);
+                                      const bool bulk = !(st.flags(zc) & FLAG_SUBCELL);
+                                      if (bulk && !cross) stb<T>(page_of(out, (idx_t)p * plane), zc.in, res);
+                                      if constexpr (defers_crossings<T>())
+                                          if (bulk && cross)
+                                              job[atomicAdd(&njobs, 1)] =
+                                                  (unsigned short)((p - p0) << 8 | (int)threadIdx.x);
+                                  });
+        if constexpr (!defers_crossings<T>()) return;
+        __syncthreads();
+    }
+    const int total = lists ? *il.count : njobs, first = lists ? blk * axis_lane_stride(1) : 0;
+    for (int j0 = first; j0 < total; j0 += lists ? axis_lane_stride(niface) : axis_lane_stride(1)) {
+        const AxisLane al = axis_lane(j0, 0);
         const bool active = al.point >= 0 && al.point < total;
         ReinitLane q;
         if (active) {
-            const idx_t ind = (idx_t)over[al.point];
-            q = reinit_iface_lane<T, S>(fs, flags, b, inv, il, -1, ind, ind, al.axis);
+            int r, c, p, slot = -1;
+            idx_t ind;
+            if (lists) {
+                slot = al.point;
+                ind = (idx_t)il.idx[slot];
+                coords_of(b, ind, r, c, p);
+            } else {
+                const int e = job[al.point], th = e & 255;
+                r = r0 + th % R;
+                c = c0 + th / R;
+                p = p0 + (e >> 8);
+                ind = lin(b, r, c, p);
+            }
+            q = reinit_iface_lane<T, S>(fs, flags, b, invs, il, slot, r, c, p, ind, ind, al.axis);
         }
         reinit_iface_finish(out, fs, fn, q, al, active, stage);
     }
@@ -1434,43 +1422,33 @@ hipError_t launch_eno2_re_step(double* step, const double* lsf, const uint8_t* m
     VLS_POINT_LAUNCH(k_eno2_re_step, step, lsf, mask, deltat, d, box_of(g));
 }
 
-// bulk, then the interface list and the deferred bulk points (FP64), in stream order
 template <typename T, int S>
 static hipError_t reinit_stage_scheme(T* out, const T* fs, const T* fn, const uint8_t* flags, const ListView& lv,
-                                      const Geom& g, int stage, int* over, int* over_count, int seq, hipStream_t s)
+                                      const Geom& g, int stage, hipStream_t s)
 {
     const IList il{lv.idx, lv.count, lv.dist, lv.dt, lv.cap};
-    const int zd = zmarch_depth(g), ni = fused_iface_blocks(g);
+    const int zd = reinit_depth<T>(zmarch_depth(g)), ni = fused_iface_blocks(g);
     const dim3 grid(bulk_blocks(g, zd) + ni);
     if (tile_rows(g) == 32)
-        k_reinit_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage,
-                                                            over, over_count, seq, zd, ni);
+        k_reinit_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage, zd,
+                                                            ni);
     else
-        k_reinit_stage<64, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage,
-                                                            over, over_count, seq, zd, ni);
-    if constexpr (defers_crossings<T>())
-        // as many blocks as a list of the interface's points takes: where the
-        // surface has moved, or runs along a grid plane, a stage defers up to 10^4
-        // points, and a sweep is one long dependent chain.  A tenth of the blocks
-        // took 11-16 us a stage in the 96^3 relaxation, these 5.4 us; blocks that
-        // find no point leave at once (113x97x81, few points: 3.9 us either way)
-        k_reinit_deferred<T, S><<<dim3(iface_blocks(g)), dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g),
-                                                                            inv_of(g), stage, over, over_count, seq);
+        k_reinit_stage<64, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage, zd,
+                                                            ni);
     return hipGetLastError();
 }
 
 template <typename T>
 hipError_t launch_reinit_stage(T* out, const T* fs, const T* fn, const uint8_t* flags, const ListView& lv,
-                               const Geom& g, int stage, int* over, int* over_count, int seq, hipStream_t s)
+                               const Geom& g, int stage, hipStream_t s)
 {
-    return reinit_stage_scheme<T, IFACE_WENO>(out, fs, fn, flags, lv, g, stage, over, over_count, seq, s);
+    return reinit_stage_scheme<T, IFACE_WENO>(out, fs, fn, flags, lv, g, stage, s);
 }
 
 hipError_t launch_cubic_reinit_stage(double* out, const double* fs, const double* fn, const uint8_t* flags,
-                                     const ListView& lv, const Geom& g, int stage, int* over, int* over_count,
-                                     int seq, hipStream_t s)
+                                     const ListView& lv, const Geom& g, int stage, hipStream_t s)
 {
-    return reinit_stage_scheme<double, IFACE_CUBIC>(out, fs, fn, flags, lv, g, stage, over, over_count, seq, s);
+    return reinit_stage_scheme<double, IFACE_CUBIC>(out, fs, fn, flags, lv, g, stage, s);
 }
 
 template <typename T>
@@ -1707,7 +1685,7 @@ hipError_t launch_narrow(float* dst, const double* src, int64_t n, hipStream_t s
     template hipError_t launch_set_distance<T>(int, const Dist6&, double*, uint8_t*, const T*, const T*,            \
                                                const ListView&, int*, int*, const Geom&, hipStream_t);              \
     template hipError_t launch_reinit_stage<T>(T*, const T*, const T*, const uint8_t*, const ListView&, const Geom&, \
-                                               int, int*, int*, int, hipStream_t);                                  \
+                                               int, hipStream_t);                                                   \
     template hipError_t launch_list_interp<T>(double*, const ListView&, const T*, const Geom&, hipStream_t);        \
     template hipError_t launch_list_gather_vel<T>(double*, const ListView&, T*, const T*, const T*,                \
                                                   const Geom&, hipStream_t);                                        \

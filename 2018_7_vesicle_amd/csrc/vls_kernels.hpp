@@ -98,12 +98,10 @@ hipError_t launch_re_step(double* step, const double* lsf, const uint8_t* mask, 
                           const Dist6c& d, const Geom& g, hipStream_t s);
 hipError_t launch_eno2_re_step(double* step, const double* lsf, const uint8_t* mask, const double* deltat,
                                const Dist6c& d, const Geom& g, hipStream_t s);
-// one WENO5-RK3 reinitialization stage (two launches); `seq` numbers the
-// stages of one reinitialization call from 0, over_count holds 2 ints that
-// are zero before seq 0
+// one WENO5-RK3 reinitialization stage (one launch)
 template <typename T>
 hipError_t launch_reinit_stage(T* out, const T* fs, const T* fn, const uint8_t* flags, const ListView& lv,
-                               const Geom& g, int stage, int* over, int* over_count, int seq, hipStream_t s);
+                               const Geom& g, int stage, hipStream_t s);
 // interface values of C at the listed points, list order (6 rows of cap)
 template <typename T>
 hipError_t launch_list_interp(double* lcp, const ListView& lv, const T* C, const Geom& g, hipStream_t s);
@@ -144,8 +142,7 @@ hipError_t launch_wenork3_extend_step(double* step, const double* deltat, const 
 // z-marching bulk; cubic ENO instead of the nonuniform WENO at the listed and
 // deferred points), FP64; lcp from launch_list_interp_cubic
 hipError_t launch_cubic_reinit_stage(double* out, const double* fs, const double* fn, const uint8_t* flags,
-                                     const ListView& lv, const Geom& g, int stage, int* over, int* over_count,
-                                     int seq, hipStream_t s);
+                                     const ListView& lv, const Geom& g, int stage, hipStream_t s);
 hipError_t launch_cubic_extend_stage(double* out, const double* cs, const double* cn, const double* vx,
                                      const double* vy, const double* vz, const ListView& lv, const double* lcp,
                                      const double* lvel, const Geom& g, int stage, hipStream_t s);
@@ -274,6 +271,7 @@ struct BatchView {
     int ngrids, ntiles;
     int blocks;            // persistent blocks of a tile-loop launch (multiple of 8)
     int tr;                // rows per tile: 64 or 32
+    int zd;                // most pages of a work item
     const ZItem* items;    // z-march work list of the bulk stage kernels
     int nitems;
     int* list_grid;        // grid of each interface-list entry (written with the list)
@@ -300,8 +298,7 @@ hipError_t launch_batch_set_mask_bit(uint8_t* flags, const T* F, int64_t n, hipS
 // WENO5 path, 1 the cubic ENO of the WENO-RK3 variants (FP64 only)
 template <typename T>
 hipError_t launch_batch_reinit_stage(const BatchView& B, T* out, const T* fs, const T* fn, const uint8_t* flags,
-                                     const ListView& lv, int stage, int* over, int* over_count, int seq,
-                                     hipStream_t s, int scheme = 0);
+                                     const ListView& lv, int stage, hipStream_t s, int scheme = 0);
 template <typename T>
 hipError_t launch_batch_extend_stage(const BatchView& B, T* out, const T* cs, const T* cn, const T* vx,
                                      const T* vy, const T* vz, const ListView& lv, const double* lcp,
@@ -357,9 +354,9 @@ hipError_t launch_batch_ellipsoid(const BatchView& B, T* F, const double* axes, 
 // through i, row a*7 + offset+3), times lam_i where lam is given (adjoint).
 // ux, uy, uz: d out_i / d u_a,i (tangent), or its product with lam_i added
 // (adjoint).  JP = 7 rows of lv.cap, d out / d (xpr..zpd, dt) of the listed
-// points, or its product with lam_i added.  extra (n ints), extra_count (2
-// ints, zero before seq 0) and seq, which numbers the stages of a call: work
-// memory as launch_reinit_stage's.
+// points, or its product with lam_i added.  extra (n ints) is work memory;
+// extra_count holds 2 ints that are zero before seq 0, seq numbers the stages
+// of a call.
 hipError_t launch_adj_advect_jac(double* J, double* ux, double* uy, double* uz, const double* lam, const double* fs,
                                  const double* vx, const double* vy, const double* vz, double dt, const Geom& g,
                                  int stage, hipStream_t s);

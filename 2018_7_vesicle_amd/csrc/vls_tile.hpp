@@ -817,7 +817,7 @@ constexpr bool defers_crossings()
 // staged tile (lds, the point at index base), z-taps z[0..6] (z[3] the point),
 // the start value fn and flags fl.  Returns the new value; where the bulk
 // defers crossings (FP64), cross is set for a point next to a sign change of
-// the stage field (it is left to the interface pass), else it stays false.
+// the stage field (its block evaluates it after the march), else it stays false.
 // zf: the z-faces the march's previous page left (zface_start at its start)
 template <int R, typename T>
 __device__ __forceinline__ T reinit_value(const T* lds, int base, const T z[7], T fn, uint8_t fl, const Inv& invs,
@@ -844,6 +844,23 @@ __device__ __forceinline__ T reinit_value(const T* lds, int base, const T z[7], 
     return rk_combine(stage, z[3], step, fn);
 }
 
+// A block of an FP64 reinitialization stage lists in LDS the bulk points of its
+// tile that take the nonuniform stencil (defers_crossings), as page << 8 | thread,
+// and evaluates them after its march.  The list holds every point of this many
+// pages, which bounds the pages of such a block.
+constexpr int kDeferPages = 16;
+template <typename T>
+constexpr int reinit_depth(int depth)
+{
+    return defers_crossings<T>() && depth > kDeferPages ? kDeferPages : depth;
+}
+// the parts that items of at most `depth` pages are split into for it
+template <typename T>
+__host__ __device__ constexpr int reinit_parts(int depth)
+{
+    return defers_crossings<T>() ? (depth + kDeferPages - 1) / kDeferPages : 1;
+}
+
 // one lane (point, axis) of the reinitialization interface pass
 struct ReinitLane {
     double m = 0.0;   // this axis's Godunov term
@@ -852,20 +869,18 @@ struct ReinitLane {
     bool inside = false;
 };
 
-// slot: the point's position in the interface list, or -1 for a deferred
-// bulk point (spacing distances, bulk time step); ind: its index in the grid
-// (fs, flags of that grid); gind: its index in the output fields
+// the point (r, c, p); slot: its position in the interface list, or -1 for a
+// deferred bulk point (spacing distances, bulk time step); ind: its index in
+// the grid (fs, flags of that grid); gind: its index in the output fields
 template <typename T, int SCHEME = IFACE_WENO>
 __device__ __forceinline__ ReinitLane reinit_iface_lane(const T* __restrict__ fs, const uint8_t* __restrict__ flags,
-                                                        const Box& b, const Inv& inv, const IList& il, int slot,
-                                                        idx_t ind, idx_t gind, int a)
+                                                        const Box& b, const Inv& inv, const IList& il, int slot, int r,
+                                                        int c, int p, idx_t ind, idx_t gind, int a)
 {
     const double sp[3] = {b.dx, b.dy, b.dz};
     ReinitLane q;
     q.gind = gind;
     q.dt = inv.dt_bulk;
-    int r, c, p;
-    coords_of(b, ind, r, c, p);
     q.inside = (flags[ind] & FLAG_MASK) != 0;
     double r1 = sp[a], l1 = sp[a];
     if (slot >= 0) {

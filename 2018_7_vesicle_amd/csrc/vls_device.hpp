@@ -829,13 +829,22 @@ __device__ __forceinline__ double cubic_distance(double v0, double v1, double v2
 // Lagrange -> monomial coefficients of the quintic through (x_i, y_i)
 // (Poly<5>::setInterpolation, shared_utilities.hpp:57-103).  The monomial form
 // is ill-conditioned (~1e-11 relative near the data), so this and the
-// evaluation below keep one operation order without contraction; interface
-// cells are few, the cost does not matter.
+// evaluation below keep one operation order without contraction.  The 30
+// divisions are by the 15 differences of the nodes and their negatives, so
+// they share 15 reciprocals (quot_ieee: the division's own bits).
 __device__ __forceinline__ void poly5_interp(const double* x, const double* y, double coef[6])
 {
 #pragma clang fp contract(off)
     double c[6][6];
     double kk[6];
+    RecipT<double> rx[6][6];
+#pragma unroll
+    for (int i = 0; i < 6; ++i)
+#pragma unroll
+        for (int j = i + 1; j < 6; ++j) {
+            rx[i][j] = recip(x[i] - x[j]);
+            rx[j][i] = RecipT<double>{-rx[i][j].b, -rx[i][j].y};
+        }
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
         double k = y[i];
@@ -846,7 +855,7 @@ __device__ __forceinline__ void poly5_interp(const double* x, const double* y, d
 #pragma unroll
         for (int j = 0; j < 6; ++j) {
             if (j == i) continue;
-            k /= x[i] - x[j];
+            k = quot_ieee(k, rx[i][j]);
             // multiply c[i] (degree deg) by (x - x[j])
 #pragma unroll
             for (int m = 5; m >= 1; --m)
@@ -944,24 +953,36 @@ __device__ __noinline__ double six_distance(double v0, double v1, double v2, dou
     return xc - 2 * s;
 }
 
-// sixth_interp: 2_2_WENO5RK3_Extend/boundary_interpolant.cu:77-99
+// sixth_interp: 2_2_WENO5RK3_Extend/boundary_interpolant.cu:77-99, the value on
+// one side: at dis_f beyond the point from the nodes 1..6 of v (s apart from s),
+// or at dis_b before it from the nodes 0..5 (from 0).  One text for both, so a
+// wave whose lanes take different sides runs it once.
+__device__ __forceinline__ double sixth_interp_side(bool back, double dis, double s, const double v[7])
+{
+#pragma clang fp contract(off)
+    double x[6], y[6], coef[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        x[k] = back ? k * s : (k + 1) * s;
+        y[k] = back ? v[k] : v[k + 1];
+    }
+    poly5_interp(x, y, coef);
+    return poly5_eval(coef, back ? 3 * s - dis : 3 * s + dis);
+}
+// both sides (0 on a side without a crossing)
 __device__ __noinline__ Pair sixth_interp(double dis_f, double dis_b, double s, double v0, double v1, double v2,
                                           double v3, double v4, double v5, double v6)
 {
+    const double v[7] = {v0, v1, v2, v3, v4, v5, v6};
+    const bool fore = dis_f < s, back = dis_b < s;
     Pair out{0.0, 0.0};
-    if (dis_f < s) {
-        const double xf[6] = {s, 2 * s, 3 * s, 4 * s, 5 * s, 6 * s};
-        const double yf[6] = {v1, v2, v3, v4, v5, v6};
-        double coef[6];
-        poly5_interp(xf, yf, coef);
-        out.fore = poly5_eval(coef, 3 * s + dis_f);
-    }
-    if (dis_b < s) {
-        const double xb[6] = {0.0, s, 2 * s, 3 * s, 4 * s, 5 * s};
-        const double yb[6] = {v0, v1, v2, v3, v4, v5};
-        double coef[6];
-        poly5_interp(xb, yb, coef);
-        out.back = poly5_eval(coef, 3 * s - dis_b);
+    for (int k = 0; k < 2; ++k) {
+        // the fore side if there is one, then the back side
+        const bool bk = k == 1 || !fore;
+        if (bk ? !(back && (k == 0 || fore)) : k == 1) continue;
+        const double h = sixth_interp_side(bk, bk ? dis_b : dis_f, s, v);
+        if (bk) out.back = h;
+        else out.fore = h;
     }
     return out;
 }

@@ -60,6 +60,41 @@ inline dim3 page_grid(int rows, int cols, int pges)
     return dim3((unsigned)(((int64_t)rows * cols + 255) / 256), (unsigned)pges);
 }
 
+// thread t of this block as page_point numbers it (a valid one)
+__device__ __forceinline__ PagePoint page_point_of(const Box& b, RowDiv d, int t)
+{
+    PagePoint q;
+    q.in = blockIdx.x * 256u + (unsigned)t;
+    q.valid = true;
+    q.p = (int)blockIdx.y;
+    q.c = (int)(((unsigned long long)q.in * d.m) >> d.s);
+    q.r = (int)q.in - q.c * b.rows;
+    return q;
+}
+
+// The long evaluations of a point kernel (the nonuniform stencil, the quintic
+// root or interpolation), which a few points of a block need on one or two
+// axes: `need` is this thread's set of them (bit k < 6).  The block lists them in
+// LDS (job, 256 per bit in use) and its threads take one each, body(t, k) for
+// bit k of thread t, so that a wave runs the long code once per 64 evaluations.
+// Where a lane does its own three axes, a wave runs it three times, however few of
+// its lanes need it, and every wave near the interface does.  Every thread of the
+// block calls this; the caller synchronizes before it reads what body left in LDS.
+template <class Body>
+__device__ __forceinline__ void axis_jobs(unsigned need, unsigned short* job, int* count, Body body)
+{
+    if (threadIdx.x == 0) *count = 0;
+    __syncthreads();
+    if (need != 0) {
+        int at = atomicAdd(count, __popc(need));
+        for (; need != 0; need &= need - 1)
+            job[at++] = (unsigned short)((__ffs((int)need) - 1) << 8 | (int)threadIdx.x);
+    }
+    __syncthreads();
+    const int total = *count;
+    for (int j = (int)threadIdx.x; j < total; j += 256) body((int)(job[j] & 255), (int)(job[j] >> 8));
+}
+
 // 1/dx, 1/dy, 1/dz and the pseudo-time step of a point without subcell
 // distances, 0.3*min(dx,dx,dy,dy,dz,dz) (setDistance.m:17-21 with every
 // distance equal to the spacing), computed once on the host

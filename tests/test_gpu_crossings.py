@@ -52,3 +52,38 @@ def test_batch(depth):
     for i, q in enumerate(probs):
         got = b.grid_view(A, i).cpu().numpy()
         assert np.array_equal(got, q[3]), (i, np.abs(got - q[3]).max())
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (7, 5, 3), (16, 16, 5), (17, 31, 4)])
+def test_point_kernels_with_every_axis_beside_a_crossing(shape):
+    """the drop-ins whose blocks list their long evaluations: all three axes (six
+    sides) of every point of a block, on boxes of less than a block, of whole
+    blocks and of ragged ones; some points frozen, some sides at the spacing"""
+    rows, cols, pges = shape
+    sp = (0.11, 0.07, 0.13)
+    rng = np.random.default_rng(rows * cols)
+    p, c, r = np.meshgrid(np.arange(pges), np.arange(cols), np.arange(rows), indexing="ij")
+    F = np.ascontiguousarray(np.where((r + c + p) % 2, 1.0, -1.0) * rng.uniform(0.2, 1.0, r.shape) * sp[0])
+    C = rng.normal(size=F.shape)
+    d6 = [h * rng.choice([1.0, 0.9, 0.4, 1e-9], p=[0.2, 0.4, 0.39, 0.01], size=F.shape)
+          for h in np.repeat(sp, 2)]
+    vel = [rng.normal(size=F.shape) for _ in range(3)]
+    dt = 0.3 * np.min(np.stack(d6), axis=0)
+    mask = (F < 0).astype(np.uint8)
+    geo, n, d = (rows, cols, pges, *sp), F.size, [T(a) for a in d6]
+    empty = lambda k: [torch.full(F.shape, np.nan, dtype=torch.float64, device="cuda") for _ in range(k)]  # noqa: E731
+
+    loc, loc_ref = [T(a) for a in po.prefilled_distances(F.shape, *sp)], po.prefilled_distances(F.shape, *sp)
+    po.boundary_location(loc_ref, F, *sp)
+    vls.feval_boundary_location(*loc, T(F), n, *geo)
+    step, cp, ext, nrm = empty(1), empty(6), empty(1), empty(3)
+    vls.feval_re_step(step[0], T(F), T(mask).to(torch.uint8), T(dt), *d, *geo, n)
+    vls.feval_upwind_normal(*nrm, T(F), *d, *geo, n)
+    vls.feval_boundary_interpolant(*cp, *d, T(C), *geo, n)
+    cp_ref = po.boundary_interpolant(d6, C, *sp)
+    vls.feval_extend_step(ext[0], T(dt), T(C), *[T(a) for a in vel], *d, *[T(a) for a in cp_ref], *geo, n)
+    for name, got, ref in (("distance", loc, loc_ref), ("re_step", step, [po.re_step(F, mask, dt, d6, *sp)]),
+                           ("normal", nrm, po.upwind_normal(F, d6, *sp)), ("interpolant", cp, cp_ref),
+                           ("extend_step", ext, [po.extend_step(dt, C, vel, d6, cp_ref, *sp)])):
+        for k, (a, b) in enumerate(zip(got, ref)):
+            assert np.array_equal(a.cpu().numpy(), b), (name, k)

@@ -112,37 +112,45 @@ __global__ void __launch_bounds__(256) kb_crossing_distances(const T* __restrict
                                                              ListView il, BatchView B, const int* __restrict__ cand,
                                                              const int* __restrict__ cand_count)
 {
-    __shared__ int lcnt, lbase;
+    __shared__ double dist[6][256];
+    __shared__ int index[256], grid[256], njobs, lcnt, lbase;
+    __shared__ unsigned short job[6 * 256];
     const int total = *cand_count;
-    for (int j0 = (int)(blockIdx.x * 256); j0 < total; j0 += (int)(gridDim.x * 256)) {
-        const int j = j0 + (int)threadIdx.x;
-        Dists q;
+    for (int j0 = (int)blockIdx.x * 256; j0 < total; j0 += (int)gridDim.x * 256) {
+        crossing_jobs<256>(
+            dist, job, &njobs,
+            [&](int t, int a) {
+                if (j0 + t >= total) return 0u;
+                const int64_t gind = cand[j0 + t];
+                const int g = grid_of(B, gind);
+                const BGrid G = B.grids[g];
+                if (a == 0) {
+                    index[t] = (int)gind;
+                    grid[t] = g;
+                }
+                const double ds = a == 0 ? G.dx : (a == 1 ? G.dy : G.dz);
+                dist[2 * a][t] = ds;
+                dist[2 * a + 1][t] = ds;
+                return crossing_sides(F + G.off, box_of(G), gind - G.off, a);
+            },
+            [&](int t, int k) {
+                const BGrid G = B.grids[grid[t]];
+                return crossing_distance<ORDER>(F + G.off, box_of(G), (idx_t)index[t] - G.off, k,
+                                                k < 2 ? G.dx : (k < 4 ? G.dy : G.dz));
+            });
+        const int t = (int)threadIdx.x;
         bool sub = false;
         int64_t gind = 0;
         int g = 0;
-        if (j < total) {
-            gind = cand[j];
-            g = grid_of(B, gind);
-            const BGrid G = B.grids[g];
-            const Box b = box_of(G);
-            int r, c, p;
-            coords_of(b, gind - G.off, r, c, p);
-            const T* f = F + G.off;
-            const double sp[3] = {b.dx, b.dy, b.dz};
-#pragma unroll 1
+        Dists q;
+        if (j0 + t < total) {
+            gind = index[t];
+            g = grid[t];
+            const Box b = box_of(B.grids[g]);
+#pragma unroll
             for (int a = 0; a < 3; ++a) {
-                double v[7];
-                line7(f, r, c, p, a, b, v);
-                q.r[a] = sp[a];
-                q.l[a] = sp[a];
-                if (v[3] * v[4] < 0)
-                    q.r[a] = (ORDER == 2)   ? eno_quadratic_distance(v[2], v[3], v[4], v[5], sp[a])
-                             : (ORDER == 3) ? cubic_distance(v[2], v[3], v[4], v[5], sp[a])
-                                            : six_distance(v[1], v[2], v[3], v[4], v[5], v[6], sp[a]);
-                if (v[2] * v[3] < 0)
-                    q.l[a] = sp[a] - ((ORDER == 2)   ? eno_quadratic_distance(v[1], v[2], v[3], v[4], sp[a])
-                                      : (ORDER == 3) ? cubic_distance(v[1], v[2], v[3], v[4], sp[a])
-                                                     : six_distance(v[0], v[1], v[2], v[3], v[4], v[5], sp[a]));
+                q.r[a] = dist[2 * a][t];
+                q.l[a] = dist[2 * a + 1][t];
             }
             // a distance that differs from the spacing (the quadratic ENO
             // locator is not clamped and can land just above it)

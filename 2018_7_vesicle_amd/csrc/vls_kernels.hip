@@ -158,58 +158,47 @@ __global__ void __launch_bounds__(256) k_crossings_z(Dist6 d, double* __restrict
     bl.flush(cand, cand_count);
 }
 
-// the second pass, one lane per candidate.  The r-side distance on an axis is
-// the locator at the point (crossing with the +1 neighbour); the l-side one
-// is ds minus the locator of the -1 neighbour's crossing, evaluated here
-// from that neighbour's stencil (the point's own line shifted by one,
-// clamped the same way), so it is the value k_boundary_location stores from
-// the neighbour's thread.  FLAG_SUBCELL marks a distance that differs from
-// the spacing: below it, or, for the quadratic ENO locator, which is not
-// clamped, a root within rounding of the far node that lands just above it,
-// where the ENO2 schemes treat it as a crossing.
+// the second pass: 64 candidates a sweep of a block (crossing_jobs).
+// FLAG_SUBCELL marks a distance that differs from the spacing: below it, or, for
+// the quadratic ENO locator, which is not clamped, a root within rounding of the
+// far node that lands just above it, where the ENO2 schemes treat it as a
+// crossing.
 template <int ORDER, typename T>
 __global__ void __launch_bounds__(256) k_crossing_distances(Dist6 d, double* __restrict__ min_dist,
                                                             uint8_t* __restrict__ flags, const T* __restrict__ lsf,
                                                             Box b, const int* __restrict__ cand,
                                                             const int* __restrict__ cand_count, ListView lv)
 {
+    __shared__ double dist[6][64];
+    __shared__ int index[64], njobs;
+    __shared__ unsigned short job[6 * 64];
     const int total = *cand_count;
-    const double sp[3] = {b.dx, b.dy, b.dz};
-    // whole waves per sweep, so that the list append sees every lane
-    for (int j0 = (int)(blockIdx.x * 256); j0 < total; j0 += (int)(gridDim.x * 256)) {
-        const int j = j0 + (int)threadIdx.x;
+    for (int j0 = (int)blockIdx.x * 64; j0 < total; j0 += (int)gridDim.x * 64) {
+        crossing_jobs<64>(
+            dist, job, &njobs,
+            [&](int t, int a) {
+                if (j0 + t >= total) return 0u;
+                const idx_t ind = (idx_t)cand[j0 + t];
+                if (a == 0) index[t] = (int)ind;
+                const double ds = a == 0 ? b.dx : (a == 1 ? b.dy : b.dz);
+                dist[2 * a][t] = ds;
+                dist[2 * a + 1][t] = ds;
+                return crossing_sides(lsf, b, ind, a);
+            },
+            [&](int t, int k) {
+                return crossing_distance<ORDER>(lsf, b, (idx_t)index[t], k, k < 2 ? b.dx : (k < 4 ? b.dy : b.dz));
+            });
+        if (threadIdx.x >= 64) continue;
+        const int t = (int)threadIdx.x;
         bool sub = false;
         idx_t ind = 0;
         Dists q;
-        if (j < total) {
-            ind = (idx_t)cand[j];
-            int r, c, p;
-            coords_of(b, ind, r, c, p);
-            const idx_t plane = (idx_t)b.rows * b.cols;
-            const double f0 = (double)lsf[ind];
-#pragma unroll 1
-            for (int a = 0; a < 3; ++a) {
-                const double ds = sp[a];
-                q.r[a] = ds;
-                q.l[a] = ds;
-                const int pos = a == 0 ? c : (a == 1 ? r : p);
-                const int last = a == 0 ? b.cols - 1 : (a == 1 ? b.rows - 1 : b.pges - 1);
-                const idx_t stride = a == 0 ? (idx_t)b.rows : (a == 1 ? (idx_t)1 : plane);
-                const idx_t base = ind - (idx_t)pos * stride;
-                double v[8];  // the line at offsets -4..+3, clamped
+        if (j0 + t < total) {
+            ind = (idx_t)index[t];
 #pragma unroll
-                for (int s = -4; s <= 3; ++s) v[s + 4] = (double)lsf[base + (idx_t)clampi(pos + s, last) * stride];
-                const double fu = v[5], fd = v[3];
-                // the locator at the point: its line is v[1..7], its f2 = fu
-                if (f0 * fu < 0)
-                    q.r[a] = (ORDER == 2)   ? eno_quadratic_distance(v[3], f0, fu, v[6], ds)
-                             : (ORDER == 3) ? cubic_distance(v[3], f0, fu, v[6], ds)
-                                            : six_distance(v[2], v[3], f0, fu, v[6], v[7], ds);
-                // the -1 neighbour's locator: its line is v[0..6], its f0 = fd, its f2 = f0
-                if (fd * f0 < 0)
-                    q.l[a] = ds - ((ORDER == 2)   ? eno_quadratic_distance(v[2], fd, f0, v[5], ds)
-                                   : (ORDER == 3) ? cubic_distance(v[2], fd, f0, v[5], ds)
-                                                  : six_distance(v[1], v[2], fd, f0, v[5], v[6], ds));
+            for (int a = 0; a < 3; ++a) {
+                q.r[a] = dist[2 * a][t];
+                q.l[a] = dist[2 * a + 1][t];
             }
             sub = q.r[0] != b.dx || q.l[0] != b.dx || q.r[1] != b.dy || q.l[1] != b.dy || q.r[2] != b.dz ||
                   q.l[2] != b.dz;
@@ -1405,7 +1394,7 @@ hipError_t launch_set_distance(int order, const Dist6& d, double* min_dist, uint
     } else {
         k_crossings<T><<<grid, block, 0, s>>>(d, min_dist, flags, mask_src, lsf, box_of(g), cand, cand_count);
     }
-    const dim3 cg(iface_blocks(g));
+    const dim3 cg(4 * iface_blocks(g));  // 64 candidates a sweep: one sweep for 1/16 of the box
     if (order == 2)
         k_crossing_distances<2, T><<<cg, dim3(256), 0, s>>>(d, min_dist, flags, lsf, box_of(g), cand, cand_count, lv);
     else if (order == 3)

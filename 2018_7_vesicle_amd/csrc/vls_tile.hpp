@@ -95,6 +95,38 @@ __device__ __forceinline__ void axis_jobs(unsigned need, unsigned short* job, in
     for (int j = (int)threadIdx.x; j < total; j += 256) body((int)(job[j] & 255), (int)(job[j] >> 8));
 }
 
+// The six distances of a block's P candidate points (setDistance's second pass),
+// dist[k][point] with k = 2 axis + side: a thread per point and axis tests the two
+// sides (detect returns them as bits 0, 1 and presets their distances), the
+// block lists the crossings, and its threads locate one each.  Most points cross
+// on one or two of their six sides: with a lane per point a wave ran the root
+// finder, ~1000 dependent operations, for all six in turn: 38 us at 64^3 and
+// 40 at 113x97x81, 12 now (64 points a block, so that 10^4 candidates reach most
+// CUs); 176 and 97 for the 6 10^5 candidates of a batch (256 points, one atomic
+// for their list slots).
+template <int P, class Detect, class Locate>
+__device__ __forceinline__ void crossing_jobs(double (*dist)[P], unsigned short* job, int* count, Detect detect,
+                                              Locate locate)
+{
+    __syncthreads();  // the last points' distances are read
+    if (threadIdx.x == 0) *count = 0;
+    __syncthreads();
+    for (int e = (int)threadIdx.x; e < 3 * P; e += 256) {
+        const int point = e % P, axis = __builtin_amdgcn_readfirstlane(e / P);  // P is a multiple of the wave
+        unsigned need = detect(point, axis);
+        if (need != 0) {
+            int at = atomicAdd(count, __popc(need));
+            for (; need != 0; need &= need - 1)
+                job[at++] = (unsigned short)(point << 3 | (2 * axis + __ffs((int)need) - 1));
+        }
+    }
+    __syncthreads();
+    const int total = *count;
+    for (int j = (int)threadIdx.x; j < total; j += 256)
+        dist[job[j] & 7][job[j] >> 3] = locate((int)(job[j] >> 3), (int)(job[j] & 7));
+    __syncthreads();
+}
+
 // 1/dx, 1/dy, 1/dz and the pseudo-time step of a point without subcell
 // distances, 0.3*min(dx,dx,dy,dy,dz,dz) (setDistance.m:17-21 with every
 // distance equal to the spacing), computed once on the host
@@ -329,6 +361,46 @@ __device__ __forceinline__ void coords_of(const Box& b, idx_t ind, int& r, int& 
     p = (int)pp;
     c = (int)cc;
     r = (int)(rem - cc * rows);
+}
+
+// the crossings of a point on one axis: bit 0 with the +1 neighbour, bit 1 with
+// the -1 neighbour (the locators' own tests)
+template <typename T>
+__device__ __forceinline__ unsigned crossing_sides(const T* __restrict__ f, const Box& b, idx_t ind, int a)
+{
+    int r, c, p;
+    coords_of(b, ind, r, c, p);
+    const int pos = a == 0 ? c : (a == 1 ? r : p);
+    const int last = (a == 0 ? b.cols : (a == 1 ? b.rows : b.pges)) - 1;
+    const idx_t stride = a == 0 ? (idx_t)b.rows : (a == 1 ? (idx_t)1 : (idx_t)b.rows * b.cols);
+    const double f0 = (double)f[ind], fu = (double)f[ind + (idx_t)(clampi(pos + 1, last) - pos) * stride],
+                 fd = (double)f[ind + (idx_t)(clampi(pos - 1, last) - pos) * stride];
+    return (f0 * fu < 0 ? 1u : 0u) | (fd * f0 < 0 ? 2u : 0u);
+}
+
+// The distance from a point to its crossing on side k = 2 axis + (0: with the +1
+// neighbour, 1: with the -1 neighbour).  The r-side distance is the locator at
+// the point; the l-side one is ds minus the locator of the -1 neighbour's
+// crossing, evaluated here from that neighbour's stencil (the point's own line
+// shifted by one, clamped the same way), so it is the value
+// k_boundary_location stores from the neighbour's thread.
+template <int ORDER, typename T>
+__device__ __forceinline__ double crossing_distance(const T* __restrict__ f, const Box& b, idx_t ind, int k, double ds)
+{
+    int r, c, p;
+    coords_of(b, ind, r, c, p);
+    const int a = k >> 1;
+    const int pos = a == 0 ? c : (a == 1 ? r : p);
+    const int last = (a == 0 ? b.cols : (a == 1 ? b.rows : b.pges)) - 1;
+    const idx_t stride = a == 0 ? (idx_t)b.rows : (a == 1 ? (idx_t)1 : (idx_t)b.rows * b.cols);
+    const int at = pos - (k & 1);  // the lower point of the crossing pair
+    double v[6];                   // the line at offsets -2..+3 around it, clamped
+#pragma unroll
+    for (int s = -2; s <= 3; ++s) v[s + 2] = (double)f[ind + (idx_t)(clampi(at + s, last) - pos) * stride];
+    const double dist = (ORDER == 2)   ? eno_quadratic_distance(v[1], v[2], v[3], v[4], ds)
+                        : (ORDER == 3) ? cubic_distance(v[1], v[2], v[3], v[4], ds)
+                                       : six_distance(v[0], v[1], v[2], v[3], v[4], v[5], ds);
+    return (k & 1) ? ds - dist : dist;
 }
 
 __device__ __forceinline__ void load_dists(Dists& q, const Dist6c& d, idx_t ind)

@@ -53,16 +53,47 @@ __device__ __forceinline__ void point_coords(const Box& b, idx_t i, int& r, int&
 // lam_i, and U[a] += d out_i / d u_a,i lam_i (the velocity gradient).
 // ---------------------------------------------------------------------------
 // Derivatives of the uniform WENO5 derivatives of a line.  The correction Q
-// depends on four second differences (Dual<4>); the seven line values enter
-// through the second differences D_j = p_j - 2 p_{j+1} + p_{j+2} and the central
-// part C = p_1 - p_5 + 8 (p_4 - p_2), whose derivatives are constants
-// (line_row).  Carrying the seven values through Q took half as many
-// instructions again.
-// Q(d[i0], d[i1], d2, d[i3]) of the back (0, 1, 3) or fore (4, 3, 1) side
-__device__ __forceinline__ Dual<4> jp_q_dual(const JPcd<double>& m, bool fore, double e)
+// depends on four second differences; the seven line values enter through the
+// second differences D_j = p_j - 2 p_{j+1} + p_{j+2} and the central part
+// C = p_1 - p_5 + 8 (p_4 - p_2), whose derivatives are constants (line_row).
+//
+// Q(d[i0], d[i1], d2, d[i3]) of the back (0, 1, 3) or fore (4, 3, 1) side and its
+// four derivatives.  The value is jp_q's operation by operation; the derivatives
+// come from one sweep back through it (names with b: dQ / d that value), ~50
+// operations where four duals carried through jp_q took ~170: the bulk Jacobian,
+// bound by its FP64 issue, 24.2 -> 17.5 us at 64^3 (with godunov_grad below), the
+// advection one 16.4 -> 15.4.
+struct JpGrad {
+    double v, d[4];
+};
+__device__ __forceinline__ JpGrad jp_q_grad(const JPcd<double>& m, bool fore, double e)
 {
-    return jp_q(ad::dvar<4>(fore ? m.d[4] : m.d[0], 0), ad::dvar<4>(fore ? m.d[3] : m.d[1], 1),
-                ad::dvar<4>(m.d[2], 2), ad::dvar<4>(fore ? m.d[1] : m.d[3], 3), e);
+    const double k = 3.0 / 13.0;
+    const double a = fore ? m.d[4] : m.d[0], b = fore ? m.d[3] : m.d[1], c = m.d[2], d = fore ? m.d[1] : m.d[3];
+    const double t0 = a - b, t1 = b - c, t2 = c - d;
+    const double y0 = fma(-3.0, b, a), y1 = b + c, y2 = fma(3.0, c, -d);
+    const double k0 = k * y0, k1 = k * y1, k2 = k * y2;
+    const double s0 = fma(t0, t0, fma(k0, y0, e)), s1 = fma(t1, t1, fma(k1, y1, e)), s2 = fma(t2, t2, fma(k2, y2, e));
+    const double a0 = s0 * s0, a1 = s1 * s1, a2 = s2 * s2;
+    const double w0 = a1 * a2, w1 = 6.0 * (a0 * a2), w2 = 3.0 * (a0 * a1);
+    const double W = (w0 + w1) + w2, tA = t0 - t1, tB = t1 - t2, c2 = fma(2.0, w2, -W);
+    const RecipT<double> rW = recip(W);
+    JpGrad q;
+    q.v = quot(fma(4.0 * w0, tA, c2 * tB), rW);
+    // Q = (4 w0 tA + (2 w2 - W) tB) / W with W = w0 + w1 + w2
+    const double w1b = -(q.v + tB) * rW.y, w0b = fma(4.0 * tA, rW.y, w1b), w2b = fma(2.0 * tB, rW.y, w1b);
+    const double tAb = 4.0 * w0 * rW.y, tBb = c2 * rW.y;
+    // a_k = s_k^2, with the factor 2 s_k of ds_k and the 2 of dt_k, dy_k: 4 s_k
+    const double g0 = 4.0 * s0 * fma(6.0 * a2, w1b, 3.0 * a1 * w2b);
+    const double g1 = 4.0 * s1 * fma(a2, w0b, 3.0 * a0 * w2b);
+    const double g2 = 4.0 * s2 * fma(a1, w0b, 6.0 * a0 * w1b);
+    const double t0b = fma(g0, t0, tAb), t1b = fma(g1, t1, tBb - tAb), t2b = fma(g2, t2, -tBb);
+    const double y0b = g0 * k0, y1b = g1 * k1, y2b = g2 * k2;
+    q.d[0] = t0b + y0b;
+    q.d[1] = fma(-3.0, y0b, (t1b - t0b) + y1b);
+    q.d[2] = fma(3.0, y2b, (t2b - t1b) + y1b);
+    q.d[3] = -(t2b + y2b);
+    return q;
 }
 // row k of sc * C + sum_j ed[j] D_j
 __device__ __forceinline__ double line_row(int k, double sc, const double ed[5])
@@ -98,7 +129,7 @@ __global__ void __launch_bounds__(192) ka_advect_jac(double* __restrict__ J, Gra
     const JPd jp = inv.jd[a];
     const JPcd<double> m = jp_centre(v);
     const bool fore = vel < 0;
-    const Dual<4> q = jp_q_dual(m, fore, jp.e);
+    const JpGrad q = jp_q_grad(m, fore, jp.e);
     const double d = (fore ? m.c + q.v : m.c - q.v) * jp.k;
     const double li = lam ? lam[i] : 1.0;
     // out = c (fs - dt * sum_a t_a) + e fn
@@ -132,21 +163,36 @@ __global__ void __launch_bounds__(192) ka_advect_jac(double* __restrict__ J, Gra
 // nonuniform form stay in registers.  (With one lane per point the duals of 9
 // inputs and 3 axes spilled 2.9 KB a lane, and a list of a few thousand points
 // filled a few dozen CUs.  Measured on MI355X at 64^3:
-// 68 + 172 us -> 24 + 22 us; the first is bound by its FP64 arithmetic, the
+// 68 + 172 us -> 17.5 + 22 us; the first is bound by its FP64 arithmetic, the
 // second by the dependent chain of the nonuniform form.)
 // ---------------------------------------------------------------------------
-// the Godunov step's derivatives with respect to this axis's pair (d[0], d[1])
-// and dt (d[2]) from the six values of the pairs; dt < 0: frozen, step 0
-__device__ __forceinline__ Dual<3> godunov_dual(const double (&val6)[3][2][64], int lane, int a, bool inside, double dt)
+// the Godunov step's derivatives with respect to this axis's pair (d[0] fore,
+// d[1] back) and dt (d[2]) from the six values of the pairs: the selections of
+// godunov_axis and the square root of godunov_step; dt < 0: frozen, step 0
+struct GodunovGrad {
+    double d[3];
+};
+__device__ __forceinline__ GodunovGrad godunov_grad(const double (&val6)[3][2][64], int lane, int a, bool inside,
+                                                    double dt)
 {
-    typedef Dual<3> D3;
-    D3 e[6];
+    GodunovGrad r = {};
+    if (!(dt >= 0)) return r;
+    double g = 0.0;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        e[k] = D3(val6[k >> 1][k & 1][lane]);
-        if ((k >> 1) == a) e[k].d[k & 1] = 1.0;
+    for (int k = 0; k < 3; ++k) {
+        const double m = godunov_axis(inside, val6[k][1][lane], val6[k][0][lane]);
+        g = k == 0 ? m : g + m;
     }
-    return dt >= 0 ? godunov_step(inside, e[0], e[1], e[2], e[3], e[4], e[5], ad::dvar<3>(dt, 2)) : D3(0.0);
+    const double s = sqrt(g), h = s > 0 ? 0.5 / s : 0.0, sd = inside ? -dt : dt;
+    const double fo = val6[a][0][lane], bk = val6[a][1][lane];
+    const bool back = (0.0 < bk) != inside;
+    const double m = back ? bk : 0.0;
+    const bool fore = (m < -fo) != inside;
+    const double dn = 2.0 * (fore ? -fo : m) * h * sd;  // of the selected extremum
+    r.d[0] = fore ? -dn : 0.0;
+    r.d[1] = !fore && back ? dn : 0.0;
+    r.d[2] = inside ? -(s - 1.0) : s - 1.0;
+    return r;
 }
 
 __global__ void __launch_bounds__(192)
@@ -162,7 +208,7 @@ ka_reinit_jac_bulk(double* __restrict__ J, const double* __restrict__ lam, const
     if (blockIdx.x == 0 && threadIdx.x == 0) extra_count[(seq + 1) & 1] = 0;
     const uint8_t fl = i < n ? flags[i] : (uint8_t)FLAG_SUBCELL;
     const bool mine = !(fl & FLAG_SUBCELL);
-    Dual<4> qf(0.0), qb(0.0);
+    JpGrad qf = {}, qb = {};
     double fo = 0.0, bk = 0.0;
     const JPd jp = inv.jd[a];
     bool cross = false;
@@ -173,8 +219,8 @@ ka_reinit_jac_bulk(double* __restrict__ J, const double* __restrict__ lam, const
         line7(fs, r, c, p, a, b, v);
         cross = sign_change3(v);
         const JPcd<double> cd = jp_centre(v);
-        qb = jp_q_dual(cd, false, jp.e);
-        qf = jp_q_dual(cd, true, jp.e);
+        qb = jp_q_grad(cd, false, jp.e);
+        qf = jp_q_grad(cd, true, jp.e);
         bk = (cd.c - qb.v) * jp.k;
         fo = (cd.c + qf.v) * jp.k;
     }
@@ -186,7 +232,7 @@ ka_reinit_jac_bulk(double* __restrict__ J, const double* __restrict__ lam, const
     const bool any = ((crossing[0] | crossing[1] | crossing[2]) >> lane) & 1;
     if (a == 0) wave_append(any, (int)i, extra, &extra_count[seq & 1]);
     if (!mine || any) return;
-    const Dual<3> g = godunov_dual(val6, lane, a, (fl & FLAG_MASK) != 0, inv.dt_bulk);
+    const GodunovGrad g = godunov_grad(val6, lane, a, (fl & FLAG_MASK) != 0, inv.dt_bulk);
     const double cs = stage_c(stage), li = lam ? lam[i] : 1.0;
     const double wf = -cs * g.d[0] * jp.k, wb = -cs * g.d[1] * jp.k;
     const double ed[5] = {-wb * qb.d[0], wf * qf.d[3] - wb * qb.d[1], wf * qf.d[2] - wb * qb.d[2],
@@ -261,7 +307,7 @@ __global__ void __launch_bounds__(192) ka_reinit_jac_list(double* __restrict__ J
         val6[a][1][lane] = bk.v;
         __syncthreads();
         if (in) {
-            const Dual<3> g = godunov_dual(val6, lane, a, (fl & FLAG_MASK) != 0, dt);
+            const GodunovGrad g = godunov_grad(val6, lane, a, (fl & FLAG_MASK) != 0, dt);
             const double li = lam ? lam[i] : 1.0;
 #pragma unroll
             for (int m = 0; m < kJacGroup; ++m) {

@@ -1471,9 +1471,11 @@ int tile_rows(const Geom& g)
 // (window, first tile, carried faces) costs one to two pages, so deeper is
 // better until CUs run out of blocks; a second round of a few blocks costs a
 // whole march.  Measured on MI355X, extension + reinitialization stage: 96^3
-// FP64 32.7 us with 864 blocks of 4 pages, 35.0 with 1728 of 2 and 36.3 with
-// 432 of 8; 150 x 131 x 120 FP32 43.3 with 1020 of 10, 45.4 with 2550 of 4; the
-// rule is within 3% of the best depth on 12 of 15 boxes and within 8% on all.
+// FP64 29.7 us with 864 blocks of 4 pages, 32.9 with 1728 of 2 and 34.3 with
+// 432 of 8; 150 x 131 x 120 FP32 43.3 with 1020 of 10, 45.4 with 2550 of 4.  Over
+// 15 boxes of 32^3 to 256^3 and ragged ones (FP64, both shapes) the rule is within
+// 3% of the best on 10 and within 7% on all; limits of 900 or 1152 to 2048
+// blocks lose 1-2% more on average.
 int zmarch_depth(const Geom& g)
 {
     if (g.zd > 0) return g.zd < g.pges ? g.zd : g.pges;

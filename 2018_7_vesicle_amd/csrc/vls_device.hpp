@@ -243,17 +243,21 @@ __device__ __forceinline__ float fminf_(float a, float b) { return (a < b) ? a :
 //   Q = [4 x0 A + (6 x2 - W) B] / W = (4 x0 A + 6 x2 B) / W - B,  W = x0 + 6 x1 + 3 x2,
 // evaluated with numerator and denominator divided by 6:
 //   z = 2/3 x0,  Q = (z A + x2 B) / (x1 + x2/2 + z/4) - B.
-// The denominator starts from 1e-30 so that the quotient stays finite; it comes
-// near that only when every indicator exceeds ~1e15 (second differences beyond
-// ~1e7, far outside level-set data).  Two instructions fewer a side than with
-// the weights as written and a floor of W.  With the carried differences
+// The denominator starts from 2^-125 (its reciprocal is finite), so that the
+// quotient stays finite where every weight underflows.  While the largest
+// weight is above ~1e-30, that is up to second differences of ~1e7, the constant
+// is below its rounding; it costs Q an error of 2e-5 of the differences at 2e7 and
+// 1e-4 at 3e7 (random differences, against 64 bits; 4e-6 up to 1e7).  An
+// additive 1e-30 cost 5e-5 from differences of 3e5 on and all accuracy at 3e6,
+// a floor of W at 1e-30 all of it at 1e7.  Two instructions fewer a side than
+// with the weights as written and that floor.  With the carried differences
 // (ZDiff) and the buffer addressing of the march (Page) the FP32 extension
 // loop has 140 VALU instructions a point instead of 159 and the
 // reinitialization loop 218 instead of 240; both stages are bound by them.
 // Measured on MI355X at 256^3: 94.9 -> 92.0 and 112.6 -> 106.7 us a stage.
 __device__ __forceinline__ float jp_weights(float z, float r1, float x2)
 {
-    return __builtin_amdgcn_rcpf(fmaf(0.25f, z, fmaf(0.5f, x2, fmaf(r1, r1, 1e-30f))));
+    return __builtin_amdgcn_rcpf(fmaf(0.25f, z, fmaf(0.5f, x2, fmaf(r1, r1, 0x1p-125f))));
 }
 __device__ __forceinline__ float jp_q(float a, float b, float c, float d, float e)
 {

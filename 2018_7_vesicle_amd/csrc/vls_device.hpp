@@ -267,7 +267,7 @@ __device__ __forceinline__ float jp_q(float a, float b, float c, float d, float 
     const float r0 = __builtin_amdgcn_rcpf(fmaf(u0, u0, ib));
     const float r1 = __builtin_amdgcn_rcpf(fmaf(u1, u1, ic));
     const float r2 = __builtin_amdgcn_rcpf(fmaf(u2, u2, ic));
-    const float z = (2.f / 3.f * r0) * r0, x2 = r2 * r2;
+    const float z = 2.f / 3.f * (r0 * r0), x2 = r2 * r2;
     const float A = fmaf(-2.f, b, a) + c, B = fmaf(-2.f, c, b) + d;
     return fmaf(fmaf(z, A, x2 * B), jp_weights(z, r1, x2), -B);
 }
@@ -325,7 +325,7 @@ __device__ __forceinline__ void weno5_pair(float& d_fore, float& d_back, const f
         const float r0 = __builtin_amdgcn_rcpf(fmaf(u0, u0, ib));
         const float r1 = __builtin_amdgcn_rcpf(fmaf(u1, u1, ic));
         const float r2 = __builtin_amdgcn_rcpf(fmaf(u2, u2, ic));
-        const float z = (2.f / 3.f * r0) * r0, x2 = r2 * r2;
+        const float z = 2.f / 3.f * (r0 * r0), x2 = r2 * r2;
         const float A = fmaf(-2.f, d1, d0) + d2;
         qb = fmaf(fmaf(z, A, x2 * B), jp_weights(z, r1, x2), -B);
     }
@@ -336,7 +336,7 @@ __device__ __forceinline__ void weno5_pair(float& d_fore, float& d_back, const f
         const float r0 = __builtin_amdgcn_rcpf(fmaf(u0, u0, ib));
         const float r1 = __builtin_amdgcn_rcpf(fmaf(u1, u1, ic));
         const float r2 = __builtin_amdgcn_rcpf(fmaf(u2, u2, ic));
-        const float z = (2.f / 3.f * r0) * r0, x2 = r2 * r2;
+        const float z = 2.f / 3.f * (r0 * r0), x2 = r2 * r2;
         const float A = fmaf(-2.f, d3, d4) + d2;
         qf = fmaf(fmaf(z, A, x2 * B), jp_weights(z, r1, x2), -B);
     }

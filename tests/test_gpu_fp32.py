@@ -214,6 +214,30 @@ def test_fp32_operators_on_large_rough_fields(amplitude):
     assert all(e < 64 * U32 for e in errs.values()), errs
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_reinit_rounds_alike_on_every_axis(dtype, sign):
+    """A line of 1000 random values, constant across, reinitialized with the
+    line laid along x, y and z: the same bits (the z axis carries half of its
+    weights from page to page, the other two do not)."""
+    n, w = 1000, 4
+    f = sign * np.random.default_rng(3).uniform(0.001, 2.0, n)
+    outs = []
+    for dim in (1, 2, 0):  # x, y, z of a (pges, cols, rows) field
+        shape = [w, w, w]
+        shape[dim] = n
+        pges, cols, rows = shape
+        line = [1, 1, 1]
+        line[dim] = n
+        m = vls.SDF3(vls.GD3(*[np.arange(k) / 16 for k in (cols, rows, pges)]),
+                     _cuda(np.broadcast_to(f.reshape(line), shape), dtype))
+        m.setDistance()
+        out = m.WENO5RK3Reinitialization(m.F, 10).movedim(dim, 0).reshape(n, w * w)
+        assert torch.equal(out, out[:, :1].expand(n, w * w))
+        outs.append(out[:, 0])
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
 def test_fp32_rejects_fp64_only_methods():
     g, G = _grid(16)
     m = vls.SDF3(G, _cuda(_wobbly_sphere(g), torch.float32))

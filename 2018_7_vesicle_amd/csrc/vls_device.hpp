@@ -760,22 +760,32 @@ __device__ __forceinline__ Eno2Spacing eno2_spacing(double ds)
 {
     return Eno2Spacing{ds, recip(ds), recip(2.0 * (ds * ds))};
 }
+// A quotient over a distance.  At a crossing it is as small as the node's value
+// (that can be subnormal, its reciprocal infinite and the quotient still the
+// slope), so it takes the division itself: measured at 64^3, 6.1 us a stage with
+// the division or a reciprocal, 6.2 with a branch between them.  The spacing
+// brings its reciprocal.
+__device__ __forceinline__ double per_dist(double a, double r) { return a / r; }
+__device__ __forceinline__ double per_dist(double a, const RecipT<double>& r) { return quot_ieee(a, r); }
+__device__ __forceinline__ double dist_val(double r) { return r; }
+__device__ __forceinline__ double dist_val(const RecipT<double>& r) { return r.b; }
 // eno2_pair, and eno2_field_pair below, bit for bit, from the five middle values
 // v4, v1, v0, v2, v3 of a line: vr, vl the values at the distances r, l on either
 // side (the neighbours at the spacing, the interface values at a crossing).
 // The divisions by the spacing's constants share their reciprocals (4
 // instructions each instead of 11), and the products by 2 are exact, so the
 // second differences are fused.
+template <class D>
 __device__ __forceinline__ void eno2_pair_at(double& sR, double& sL, double v4, double v1, double v0, double v2,
-                                             double v3, double vr, double vl, const RecipT<double>& r,
-                                             const RecipT<double>& l, const Eno2Spacing& e)
+                                             double v3, double vr, double vl, const D& r, const D& l,
+                                             const Eno2Spacing& e)
 {
 #pragma clang fp contract(off)
     const double p2 = fma(-2.0, v0, v1) + v2;
     const double p2r = fma(-2.0, v2, v0) + v3;
-    sR = quot_ieee(vr - v0, r) - r.b * quot_ieee(min_mod(p2, p2r), e.h2);
+    sR = per_dist(vr - v0, r) - dist_val(r) * quot_ieee(min_mod(p2, p2r), e.h2);
     const double p2l = fma(-2.0, v1, v0) + v4;
-    sL = quot_ieee(v0 - vl, l) + l.b * quot_ieee(min_mod(p2, p2l), e.h2);
+    sL = per_dist(v0 - vl, l) + dist_val(l) * quot_ieee(min_mod(p2, p2l), e.h2);
 }
 // at a point without a subcell distance on the axis
 __device__ __forceinline__ void eno2_bulk_pair(double& sR, double& sL, double v4, double v1, double v0, double v2,

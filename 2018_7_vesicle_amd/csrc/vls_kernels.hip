@@ -543,8 +543,8 @@ __global__ void __launch_bounds__(256) k_eno2_stage(double* __restrict__ out, co
 #pragma unroll
         for (int a = 0; a < 3; ++a)
             eno2_pair_at(fo[a], bk[a], v[a][0], v[a][1], v[a][2], v[a][3], v[a][4],
-                         (e.r[a] == sp[a]) ? v[a][3] : 0.0, (e.l[a] == sp[a]) ? v[a][1] : 0.0, recip(e.r[a]),
-                         recip(e.l[a]), eno2_spacing(sp[a]));
+                         (e.r[a] == sp[a]) ? v[a][3] : 0.0, (e.l[a] == sp[a]) ? v[a][1] : 0.0, e.r[a], e.l[a],
+                         eno2_spacing(sp[a]));
     } else {
 #pragma unroll
         for (int a = 0; a < 3; ++a)

@@ -267,8 +267,8 @@ __global__ void __launch_bounds__(256) k_enork2_extend_stage(double* __restrict_
         }
 #pragma unroll
         for (int a = 0; a < 3; ++a)
-            eno2_pair_at(fo[a], bk[a], v[a][0], v[a][1], v[a][2], v[a][3], v[a][4], hf[a], hb[a], recip(e.r[a]),
-                         recip(e.l[a]), eno2_spacing(sp[a]));
+            eno2_pair_at(fo[a], bk[a], v[a][0], v[a][1], v[a][2], v[a][3], v[a][4],
+                         hf[a], hb[a], e.r[a], e.l[a], eno2_spacing(sp[a]));
     } else {
 #pragma unroll
         for (int a = 0; a < 3; ++a)

@@ -32,3 +32,22 @@ def test_eno2_stages(box):
         assert np.array_equal(got, po.eno2_reinit(F, 4, *g.spacing, rk2=rk2, cfl=cfl)), f"reinit rk2={rk2}"
     got = m.ENORK2Extend(T(C), 4).cpu().numpy()
     assert np.array_equal(got, po.variant_extend(C, 4, F, *g.spacing, "enork2")), "extend"
+
+
+@pytest.mark.parametrize("tiny", [3e-310, 2e-307, 1e-290])
+def test_eno2_stages_beside_a_node_value_of_almost_zero(tiny):
+    """nodes whose value is far below the spacing (down to a subnormal number)
+    beside nodes of the other sign: the subcell distance is as small, its
+    reciprocal overflows, and the quotients by it are of the size of the slopes"""
+    ax = [(np.arange(k) - (k - 1) / 2) * h for k, h in ((13, 0.11), (18, 0.1), (11, 0.12))]
+    g = cases.Grid(*ax)
+    F = np.ascontiguousarray(1.3 * g.X + 0.0 * g.Y)  # zero on the plane of column 6
+    F[:, 6, ::3] = -tiny
+    F[:, 6, 1::3] = -3 * tiny
+    C = np.ascontiguousarray(cases.smooth_scalar(g))
+    m = vls.SDF3(vls.GD3(*ax), T(F))
+    ref = po.eno2_reinit(F, 4, *g.spacing)
+    assert np.isfinite(ref).all()
+    assert np.array_equal(m.ENORK2Reinitialization(T(F), 4).cpu().numpy(), ref)
+    ref = po.variant_extend(C, 2, F, *g.spacing, "enork2")
+    assert np.array_equal(m.ENORK2Extend(T(C), 2).cpu().numpy(), ref, equal_nan=True)

@@ -569,7 +569,9 @@ __device__ __forceinline__ double upwind_normal_axis(const double v[7], JPd j, b
 }
 
 // an axis with a distance below the spacing takes the nonuniform stencil, as a
-// job of the block (axis_jobs)
+// job of the block (axis_jobs), with the division for its quotients: unlike
+// re_step and extend_step this takes a point whatever its distances, and their
+// reciprocals and the squares of the differences by them overflow
 template <typename T>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_upwind_normal(T* __restrict__ nx, T* __restrict__ ny,
                                                        T* __restrict__ nz, const T* __restrict__ lsf,
@@ -600,8 +602,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
         const double l1 = (a == 0 ? d.l[0] : (a == 1 ? d.l[1] : d.l[2]))[page + o.in];
         double v[7];
         line7_lane(lsf, o.r, o.c, o.p, a, b, v);
-        one[a][t] = weno_nonuniform_one_inl(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, ds, 0.0, 0.0,
-                                        !(fabs(v[4]) < fabs(v[2])));
+        one[a][t] = weno_nonuniform_one_inl<true>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, ds, 0.0, 0.0,
+                                                  !(fabs(v[4]) < fabs(v[2])));
     });
     __syncthreads();
     if (!q.valid) return;

@@ -87,3 +87,19 @@ def test_point_kernels_with_every_axis_beside_a_crossing(shape):
                            ("extend_step", ext, [po.extend_step(dt, C, vel, d6, cp_ref, *sp)])):
         for k, (a, b) in enumerate(zip(got, ref)):
             assert np.array_equal(a.cpu().numpy(), b), (name, k)
+
+
+def test_upwind_normal_at_any_distance():
+    """upwind_normal takes distances down to zero (re_step and extend_step freeze
+    a point below 1e-6 of the spacing): a cell of almost no width drops out of
+    the weights where its squares overflow, and a zero distance gives NaN"""
+    sp = (0.11, 0.07, 0.13)
+    rng = np.random.default_rng(5)
+    F = rng.normal(size=(5, 9, 33))
+    d6 = [h * rng.choice([1.0, 0.4, 1e-16, 1e-120, 1e-160, 1e-200, 1e-300, 1e-310, 0.0], size=F.shape)
+          for h in np.repeat(sp, 2)]
+    nrm = [torch.full(F.shape, 7.0, dtype=torch.float64, device="cuda") for _ in range(3)]
+    vls.feval_upwind_normal(*nrm, T(F), *[T(a) for a in d6], 33, 9, 5, *sp, F.size)
+    for k, (a, b) in enumerate(zip(nrm, po.upwind_normal(F, d6, *sp))):
+        assert np.isfinite(b).any()
+        assert np.array_equal(a.cpu().numpy(), b, equal_nan=True), k

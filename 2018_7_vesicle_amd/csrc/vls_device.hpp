@@ -46,8 +46,7 @@ __device__ __forceinline__ double min_mod(double x, double y)
 // also evaluated at frozen points, where a distance can be zero (then it is NaN
 // by either division) or as small as a node value, but is not used there.
 // Numerators overflow for second differences beyond ~1e34 (4 w0 tA in jp_q, W ~
-// the eighth power) and for divided differences beyond ~1e154 (the indicators of
-// the nonuniform face); there the division gives an infinity and this NaN.
+// the eighth power); there the division gives an infinity and this NaN.
 template <typename S>
 struct RecipT;
 template <>
@@ -72,11 +71,14 @@ __device__ __forceinline__ double quot_ieee(double a, const RecipT<double>& r)
 {
     return __builtin_amdgcn_div_fixup(quot(a, r), r.b, a);
 }
-// a over d, a denominator or one with its reciprocal; IEEE: the division itself
-template <bool IEEE, typename S>
+__device__ __forceinline__ double quot_ieee(double a, double b) { return quot_ieee(a, recip(b)); }
+// a over d, a denominator or one with its reciprocal.  IEEE: the division itself;
+// WIDE: a may have overflowed (quot_ieee)
+template <bool IEEE, bool WIDE = false, typename S>
 __device__ __forceinline__ S over(const S& a, const S& d)
 {
     if constexpr (IEEE) return a / d;
+    else if constexpr (WIDE) return quot_ieee(a, d);
     else return quot(a, d);
 }
 template <bool IEEE, typename S>
@@ -539,7 +541,9 @@ __device__ __forceinline__ void weno5_pair_z(double& d_fore, double& d_back, boo
 // (both sides, all axes).  Measured on MI355X: 40 extension iterations at 128^3
 // FP64 3.85 -> 3.64 ms, the step of 96 FP32 grids of 32..96 61.7 -> 57.5 ms.
 // The weights' divisions by (s + eps)^2 stay IEEE: that square overflows for
-// jumps beyond 1e75 spacings, and the weight is then 0.
+// jumps beyond 1e75 spacings, and the weight is then 0.  The products of two
+// divided differences overflow for jumps beyond 1e150 and keep their infinity
+// (over<..., true>, one instruction each), for the same reason.
 // ---------------------------------------------------------------------------
 template <typename S, bool IEEE = false>
 __device__ __forceinline__ S weno_nonuniform_face(const S* a, const S* u, bool back)
@@ -556,17 +560,17 @@ __device__ __forceinline__ S weno_nonuniform_face(const S* a, const S* u, bool b
     const S h2 = sq(h);
     const S s0 = 4.0 * sq(hX2) *
         (sq(over<IEEE>(u2 - u1, X3)) * (10.0 * h2 + X1.b * (x15 - x05))
-         + over<IEEE>((u2 - u1) * (u0 - u1), X3.b * X1.b) *
+         + over<IEEE, true>((u2 - u1) * (u0 - u1), X3.b * X1.b) *
                (20.0 * h2 + 2.0 * X1.b * (x15 - x05) + X2.b * (2.0 * x15 - x05 - xm05))
          + sq(over<IEEE>(u0 - u1, X1)) * (10.0 * h2 + (x25 + x15 - 2.0 * xm05) * (x25 + x15 - x05 - xm05)));
     const S s1 = 4.0 * sq(hW) *
         (sq(over<IEEE>(um1 - u0, Y1)) * (10.0 * h2 + X1.b * (x15 - x05))
-         + over<IEEE>((u1 - u0) * (um1 - u0), X1.b * Y1.b) *
+         + over<IEEE, true>((u1 - u0) * (um1 - u0), X1.b * Y1.b) *
                (20.0 * h2 - (x15 - x05) * (xm05 - xm15) - X1.b * Y1.b)
          + sq(over<IEEE>(u1 - u0, X1)) * (10.0 * h2 + (xm05 - xm15) * Y1.b));
     const S s2 = 4.0 * sq(hY2) *
         (sq(over<IEEE>(um2 - um1, Y3)) * (10.0 * h2 + Y1.b * (xm05 - xm15))
-         + over<IEEE>((u0 - um1) * (um2 - um1), Y1.b * Y3.b) *
+         + over<IEEE, true>((u0 - um1) * (um2 - um1), Y1.b * Y3.b) *
                (20.0 * h2 + 2.0 * Y1.b * (xm05 - xm15) + Y2.b * (x05 + xm05 - 2.0 * xm15))
          + sq(over<IEEE>(u0 - um1, Y1)) *
                (10.0 * h2 + (2.0 * x05 - xm25 - xm15) * (x05 + xm05 - xm15 - xm25)));

@@ -106,6 +106,16 @@ __device__ __forceinline__ Dual<N> quot(const Dual<N>& a, const Dual<N>& b)
     for (int k = 0; k < N; ++k) r.d[k] = (a.d[k] - r.v * b.d[k]) * ib.y;
     return r;
 }
+template <int N>
+__device__ __forceinline__ Dual<N> quot_ieee(const Dual<N>& a, const Dual<N>& b)
+{
+    const RecipT<double> ib = recip(b.v);
+    Dual<N> r;
+    r.v = vls::quot_ieee(a.v, ib);
+#pragma unroll
+    for (int k = 0; k < N; ++k) r.d[k] = (a.d[k] - r.v * b.d[k]) * ib.y;
+    return r;
+}
 // mixed forms with a constant
 template <int N>
 __device__ __forceinline__ Dual<N> operator+(double a, const Dual<N>& b)

@@ -103,3 +103,22 @@ def test_upwind_normal_at_any_distance():
     for k, (a, b) in enumerate(zip(nrm, po.upwind_normal(F, d6, *sp))):
         assert np.isfinite(b).any()
         assert np.array_equal(a.cpu().numpy(), b, equal_nan=True), k
+
+
+def test_extend_step_beside_huge_values():
+    """extend_step at interface points some of whose stencils reach a value of
+    1e200: the products of their divided differences overflow, and the stencil
+    gets no weight where the oracle gives it none (NaN where the oracle has it)"""
+    shape, sp = (5, 9, 33), (0.11, 0.07, 0.13)
+    rng = np.random.default_rng(8)
+    C = rng.normal(size=shape)
+    C = np.where(rng.uniform(size=shape) < 0.03, 1e200 * C, C)
+    d6 = [np.ascontiguousarray(h * rng.choice([1.0, 0.9, 0.4], size=shape)) for h in np.repeat(sp, 2)]
+    vel = [rng.normal(size=shape) for _ in range(3)]
+    cp6 = [rng.normal(size=shape) for _ in range(6)]
+    dt = 0.3 * np.min(np.stack(d6), axis=0)
+    ref = po.extend_step(dt, C, vel, d6, cp6, *sp)
+    ext = torch.full(shape, 7.0, dtype=torch.float64, device="cuda")
+    vls.feval_extend_step(ext, T(dt), T(C), *[T(a) for a in vel], *[T(a) for a in d6], *[T(a) for a in cp6],
+                          33, 9, 5, *sp, C.size)
+    assert np.array_equal(ext.cpu().numpy(), ref, equal_nan=True)

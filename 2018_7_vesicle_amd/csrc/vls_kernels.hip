@@ -992,17 +992,30 @@ __device__ __forceinline__ void towers_h_delta(double& H, double& delta, const B
     delta = (pxx + pyy + pzz) / g2 - dot * t.lap / (g2 * t.g * t.g);
 }
 
-// one value of an output field, past the caches: the fields are written once
-// and together are larger than any cache (302 and 453 MB at 128^3).  At 128^3
-// the toolbox of F takes 90 us with plain stores and 65 with these (its 336 MB
-// at 5.2 TB/s), that of A 174 and 169, the tail that reads them 58 and 48.
-// Dividing through shared reciprocals gains 1% of this and is not done.
-template <typename O>
+// One value of an output field; NT: past the caches.  The toolbox of A reads 13
+// fields of that of F, and its caller reads both, so the stores go past the
+// caches only where the fields would not stay in the 256 MB last-level cache
+// anyway: those of F from kStreamF bytes of its 18 fields on, those of A from
+// kStreamA of the 48 of both.  Both toolboxes in turn and a pass over their
+// fields, plain -> past the caches (a row of 72, 84 or 116 doubles ends inside a
+// cache line, where the latter also write lines in parts):
+//   both together   72^3 (143 MB) 203 -> 216 us, 80^3 (197 MB) 217 -> 237, 84^3 244 -> 273
+//   A's alone       88^3 (262 MB) 280 -> 270, 96^3 366 -> 335, 104^3 456 -> 414 (F's plain)
+//   F's (A's past)  104^3 (162 MB of F) 414 -> 440, 112^3 (202 MB) 505 -> 511,
+//                   116^3 (225 MB) 563 -> 571, 120^3 647 -> 624, 128^3 722 -> 702
+// (112^3 and 116^3 without that pass: 221 -> 204 and 255 -> 248.)
+// At 128^3 the toolbox of F takes 65 us instead of 90 (its 336 MB at 5.2 TB/s), that
+// of A 169 instead of 174, the tail that reads them 48 instead of 58.  Dividing
+// through shared reciprocals gains 1% of this and is not done.
+constexpr int64_t kStreamF = 220000000, kStreamA = 256000000;
+template <bool NT, typename O>
 __device__ __forceinline__ void put(const O& o, int k, idx_t ind, double v)
 {
-    __builtin_nontemporal_store(v, &o.f[k][ind]);
+    if constexpr (NT) __builtin_nontemporal_store(v, &o.f[k][ind]);
+    else o.f[k][ind] = v;
 }
 
+template <bool NT>
 __global__ void __launch_bounds__(256) k_set_calculus_toolbox(Fields18 o, const double* __restrict__ lsf,
                                                               const double* __restrict__ hp, Box b, double ds)
 {
@@ -1013,26 +1026,26 @@ __global__ void __launch_bounds__(256) k_set_calculus_toolbox(Fields18 o, const 
     load_box27(F, lsf, r, c, p, b);
     load_box27(P, hp, r, c, p, b);
     const Toolbox t = toolbox_of(F, b, ds);
-    put(o, 0, ind, t.fx); put(o, 1, ind, t.fy); put(o, 2, ind, t.fz); put(o, 3, ind, t.g);
-    put(o, 4, ind, t.fx / t.g); put(o, 5, ind, t.fy / t.g); put(o, 6, ind, t.fz / t.g);
-    put(o, 7, ind, t.fxx); put(o, 8, ind, t.fyy); put(o, 9, ind, t.fzz);
-    put(o, 10, ind, t.fxy); put(o, 11, ind, t.fyz); put(o, 12, ind, t.fzx); put(o, 13, ind, t.lap);
+    put<NT>(o, 0, ind, t.fx); put<NT>(o, 1, ind, t.fy); put<NT>(o, 2, ind, t.fz); put<NT>(o, 3, ind, t.g);
+    put<NT>(o, 4, ind, t.fx / t.g); put<NT>(o, 5, ind, t.fy / t.g); put<NT>(o, 6, ind, t.fz / t.g);
+    put<NT>(o, 7, ind, t.fxx); put<NT>(o, 8, ind, t.fyy); put<NT>(o, 9, ind, t.fzz);
+    put<NT>(o, 10, ind, t.fxy); put<NT>(o, 11, ind, t.fyz); put<NT>(o, 12, ind, t.fzx); put<NT>(o, 13, ind, t.lap);
     double c1 = t.fxx * t.fx + t.fxy * t.fy + t.fzx * t.fz;
     double c2 = t.fxy * t.fx + t.fyy * t.fy + t.fyz * t.fz;
     double c3 = t.fzx * t.fx + t.fyz * t.fy + t.fzz * t.fz;
     const double g3 = t.g * t.g * t.g;
-    put(o, 14, ind, -t.lap / t.g + (t.fx * c1 + t.fy * c2 + t.fz * c3) / g3);
+    put<NT>(o, 14, ind, -t.lap / t.g + (t.fx * c1 + t.fy * c2 + t.fz * c3) / g3);
     c1 = (t.fyy * t.fzz - t.fyz * t.fyz) * t.fx + (t.fzx * t.fyz - t.fxy * t.fzz) * t.fy
          + (t.fxy * t.fyz - t.fzx * t.fyy) * t.fz;
     c2 = (t.fyz * t.fzx - t.fxy * t.fzz) * t.fx + (t.fxx * t.fzz - t.fzx * t.fzx) * t.fy
          + (t.fzx * t.fxy - t.fxx * t.fyz) * t.fz;
     c3 = (t.fxy * t.fyz - t.fyy * t.fzx) * t.fx + (t.fzx * t.fxy - t.fxx * t.fyz) * t.fy
          + (t.fxx * t.fyy - t.fxy * t.fxy) * t.fz;
-    put(o, 15, ind, (t.fx * c1 + t.fy * c2 + t.fz * c3) / (g3 * t.g));
+    put<NT>(o, 15, ind, (t.fx * c1 + t.fy * c2 + t.fz * c3) / (g3 * t.g));
     double H, delta;
     towers_h_delta(H, delta, P, t, b);
-    put(o, 16, ind, H);
-    put(o, 17, ind, delta);
+    put<NT>(o, 16, ind, H);
+    put<NT>(o, 17, ind, delta);
 }
 #undef T27
 
@@ -1054,6 +1067,7 @@ __device__ __forceinline__ double norm3(double x, double y, double z)
     return dmax(sqrt(x * x + y * y + z * z), 1e-14);
 }
 
+template <bool NT>
 __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, const double* __restrict__ A,
                                                                    const double* __restrict__ ahp, Fields13c fin,
                                                                    Box b, double ds)
@@ -1066,19 +1080,19 @@ __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, c
     load_box27(Ab, A, r, c, p, b);
     load_box27(Pb, ahp, r, c, p, b);
     const Toolbox a = toolbox_of(Ab, b, ds);  // Ax..Azx, |grad A| = norm, ALaplacian
-    put(o, 0, ind, a.fx); put(o, 1, ind, a.fy); put(o, 2, ind, a.fz); put(o, 3, ind, a.g);
+    put<NT>(o, 0, ind, a.fx); put<NT>(o, 1, ind, a.fy); put<NT>(o, 2, ind, a.fz); put<NT>(o, 3, ind, a.g);
     const double fx = fin.f[0][ind], fy = fin.f[1][ind], fz = fin.f[2][ind], fg = fin.f[3][ind];
     double cx, cy, cz;
     cross3(cx, cy, cz, fx, fy, fz, a.fx, a.fy, a.fz);
     const double ncr = norm3(cx, cy, cz);
-    put(o, 4, ind, cx); put(o, 5, ind, cy); put(o, 6, ind, cz); put(o, 7, ind, ncr);
+    put<NT>(o, 4, ind, cx); put<NT>(o, 5, ind, cy); put<NT>(o, 6, ind, cz); put<NT>(o, 7, ind, ncr);
     const double tx = cx / ncr, ty = cy / ncr, tz = cz / ncr;
-    put(o, 8, ind, tx); put(o, 9, ind, ty); put(o, 10, ind, tz);
+    put<NT>(o, 8, ind, tx); put<NT>(o, 9, ind, ty); put<NT>(o, 10, ind, tz);
     double nx, ny, nz;
     cross3(nx, ny, nz, tx, ty, tz, fin.f[4][ind], fin.f[5][ind], fin.f[6][ind]);
-    put(o, 11, ind, nx); put(o, 12, ind, ny); put(o, 13, ind, nz);
-    put(o, 14, ind, a.fxx); put(o, 15, ind, a.fyy); put(o, 16, ind, a.fzz);
-    put(o, 17, ind, a.fxy); put(o, 18, ind, a.fyz); put(o, 19, ind, a.fzx); put(o, 20, ind, a.lap);
+    put<NT>(o, 11, ind, nx); put<NT>(o, 12, ind, ny); put<NT>(o, 13, ind, nz);
+    put<NT>(o, 14, ind, a.fxx); put<NT>(o, 15, ind, a.fyy); put<NT>(o, 16, ind, a.fzz);
+    put<NT>(o, 17, ind, a.fxy); put<NT>(o, 18, ind, a.fyz); put<NT>(o, 19, ind, a.fzx); put<NT>(o, 20, ind, a.lap);
     const double fxx = fin.f[7][ind], fyy = fin.f[8][ind], fzz = fin.f[9][ind];
     const double fxy = fin.f[10][ind], fyz = fin.f[11][ind], fzx = fin.f[12][ind];
     // geodesic curvature (auxi_set_calculus_toolbox.cu:115-131)
@@ -1092,7 +1106,7 @@ __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, c
     vz = tx * a.fzx + ty * a.fyz + tz * a.fzz;
     double w2x, w2y, w2z;
     cross3(w2x, w2y, w2z, fx, fy, fz, vx, vy, vz);
-    put(o, 21, ind, (nx * (w1x + w2x) + ny * (w1y + w2y) + nz * (w1z + w2z)) / ncr);
+    put<NT>(o, 21, ind, (nx * (w1x + w2x) + ny * (w1y + w2y) + nz * (w1z + w2z)) / ncr);
     // the shape operator of F's level sets, dN/dx (:135-145)
     const double g3 = fg * fg * fg;
     const double sx = fxx * fx + fxy * fy + fzx * fz;
@@ -1104,17 +1118,17 @@ __global__ void __launch_bounds__(256) k_auxi_set_calculus_toolbox(Fields27 o, c
     vx = Nxx * tx + Nxy * ty + Nxz * tz;
     vy = Nyx * tx + Nyy * ty + Nyz * tz;
     vz = Nzx * tx + Nzy * ty + Nzz * tz;
-    put(o, 22, ind, -(tx * vx + ty * vy + tz * vz));
+    put<NT>(o, 22, ind, -(tx * vx + ty * vy + tz * vz));
     vx = Nxx * nx + Nxy * ny + Nxz * nz;
     vy = Nyx * nx + Nyy * ny + Nyz * nz;
     vz = Nzx * nx + Nzy * ny + Nzz * nz;
-    put(o, 23, ind, -(tx * vx + ty * vy + tz * vz));
-    put(o, 24, ind, -(nx * vx + ny * vy + nz * vz));
+    put<NT>(o, 23, ind, -(tx * vx + ty * vy + tz * vz));
+    put<NT>(o, 24, ind, -(nx * vx + ny * vy + nz * vz));
     // Heaviside and delta of A from its primal (:166-197)
     double H, delta;
     towers_h_delta(H, delta, Pb, a, b);
-    put(o, 25, ind, H);
-    put(o, 26, ind, delta);
+    put<NT>(o, 25, ind, H);
+    put<NT>(o, 26, ind, delta);
 }
 
 // periodic neighbour index of the @GD3 index maps (circshift, GD3.m:112-117)
@@ -1687,13 +1701,16 @@ hipError_t launch_weno_derivative(const Dist6& out, const double* lsf, const Geo
 hipError_t launch_set_calculus_toolbox(const Fields18& o, const double* lsf, const double* hp, const Geom& g,
                                        double ds, hipStream_t s)
 {
-    VLS_POINT_LAUNCH(k_set_calculus_toolbox, o, lsf, hp, box_of(g), ds);
+    if (g.n() * 18 * 8 >= kStreamF) VLS_POINT_LAUNCH(k_set_calculus_toolbox<true>, o, lsf, hp, box_of(g), ds);
+    VLS_POINT_LAUNCH(k_set_calculus_toolbox<false>, o, lsf, hp, box_of(g), ds);
 }
 
 hipError_t launch_auxi_set_calculus_toolbox(const Fields27& o, const double* lsf, const double* ahp,
                                             const Fields13c& fin, const Geom& g, double ds, hipStream_t s)
 {
-    VLS_POINT_LAUNCH(k_auxi_set_calculus_toolbox, o, lsf, ahp, fin, box_of(g), ds);
+    if (g.n() * 48 * 8 >= kStreamA)
+        VLS_POINT_LAUNCH(k_auxi_set_calculus_toolbox<true>, o, lsf, ahp, fin, box_of(g), ds);
+    VLS_POINT_LAUNCH(k_auxi_set_calculus_toolbox<false>, o, lsf, ahp, fin, box_of(g), ds);
 }
 
 hipError_t launch_aux_toolbox_tail(double* afdd, double* addn, const double* ah, const double* h, const double* a,

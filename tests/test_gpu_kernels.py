@@ -196,6 +196,29 @@ def test_auxi_set_calculus_toolbox(case):
         exact(N(t), ref[name], name)
 
 
+@pytest.mark.parametrize("pges", [104, 105, 238, 239])
+def test_toolboxes_at_the_sizes_where_their_stores_change(pges):
+    """the toolboxes' stores go past the caches from 667 k points on (A) and from
+    1528 k (F): the boxes next below and above, every field"""
+    rows, cols = 64, 100
+    assert (rows * cols * pges * 48 * 8 >= 256000000) == (pges >= 105)
+    assert (rows * cols * pges * 18 * 8 >= 220000000) == (pges >= 239)
+    g = cases.Grid(*[(np.arange(k) - (k - 1) / 2) * h for k, h in ((cols, 0.02), (rows, 0.03), (pges, 0.01))])
+    F = np.sqrt(g.X ** 2 + 1.1 * g.Y ** 2 + 0.9 * g.Z ** 2) - 0.6
+    A, geo = _aux_field(g), (rows, cols, pges, *g.spacing, g.ds)
+    ft = po.set_calculus_toolbox(F, np.maximum(F, 0), *g.spacing, g.ds)
+    out = [torch.full(F.shape, np.nan, dtype=torch.float64, device="cuda") for _ in range(18)]
+    vls.feval_set_calculus_toolbox(out, T(F), T(np.maximum(F, 0)), *geo)
+    for name, t in zip(po.TOOLBOX_FIELDS, out):
+        exact(N(t), ft[name], name)
+    fin = [ft[k] for k in po.TOOLBOX_FIELDS[:13]]
+    ref = po.auxi_set_calculus_toolbox(A, np.maximum(A, 0), fin, *g.spacing, g.ds)
+    out = [torch.full(F.shape, np.nan, dtype=torch.float64, device="cuda") for _ in range(27)]
+    vls.feval_auxi_set_calculus_toolbox(out, T(A), T(np.maximum(A, 0)), [T(a) for a in fin], *geo)
+    for name, t in zip(po.AUX_TOOLBOX_FIELDS, out):
+        exact(N(t), ref[name], name)
+
+
 def test_variant_distances_and_re_step(case):
     """WENO-RK3 variant: cubic distances (cubic boundary_correction) and its re_step"""
     g, F = case["g"], case["F"]

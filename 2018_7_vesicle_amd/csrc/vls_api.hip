@@ -2007,8 +2007,8 @@ int sdf3_autotune_try(vls_sdf3* h, const T* F, int iterations, hipStream_t s, in
     const DSet ms = main_set(h);
     T *vx = vel<T>(h, 0), *vy = vel<T>(h, 1), *vz = vel<T>(h, 2);
     float best = 1e30f;
-    // the shape the box's size asks for at its depth, half and twice that, and
-    // the other shape at its own
+    // either shape at the depth the box's size asks for with it, half and twice
+    // that; the shape of the box's size first
     h->g.tr = 0;
     int best_tr = tile_rows(h->g), best_zd = h->g.zd;
     const int trs[2] = {best_tr, best_tr == 32 ? 64 : 32};
@@ -2017,7 +2017,7 @@ int sdf3_autotune_try(vls_sdf3* h, const T* F, int iterations, hipStream_t s, in
         h->g.tr = trs[i];
         h->g.zd = 0;
         const int d0 = zmarch_depth(h->g);
-        const int depths[3] = {d0, i == 0 && d0 > 1 ? d0 / 2 : 0, i == 0 && 2 * d0 <= h->g.pges ? 2 * d0 : 0};
+        const int depths[3] = {d0, d0 > 1 ? d0 / 2 : 0, 2 * d0 <= h->g.pges ? 2 * d0 : 0};
         for (int j = 0; j < 3; ++j) {
             if (depths[j] <= 0) continue;
             h->g.zd = depths[j];

@@ -7,10 +7,12 @@
 // 2/3, 1/3), where step_i depends on fs along the three 7-point lines through
 // i (clamped at the box) and on per-point parameters: the velocity for the
 // advection; the mask, subcell distances and pseudo-time step of the
-// reinitialization.  A Jacobian kernel evaluates the forward formulas on dual
-// numbers (vls_dual.hpp), so the WENO weights are differentiated exactly and
-// every branch (upwind side, sign-change test, Godunov selection, frozen
-// points) is the one the forward pass took, and stores, per point, the 21
+// reinitialization.  The Jacobian kernels differentiate the forward formulas
+// exactly, the WENO weights included, with every branch (upwind side,
+// sign-change test, Godunov selection, frozen points) the one the forward pass
+// took: the uniform correction and the Godunov step by one sweep back through
+// their operations (jp_q_grad, godunov_grad), the nonuniform stencil at the
+// interface points on dual numbers (vls_dual.hpp).  They store, per point, the 21
 // derivatives of out_i along its three lines (rows a*7+k, a = x,y,z, k =
 // offset+3), for the adjoint times lam_i; the parameter derivatives go to
 // their gradients at once in the adjoint and to memory in the tangent.  The
@@ -29,10 +31,6 @@
 #include "vls_tile.hpp"
 
 namespace vls {
-
-typedef Dual<8> D8;
-typedef Dual<9> D9;
-typedef Dual<7> D7;
 
 __device__ __forceinline__ double stage_c(int stage) { return stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 2.0 / 3.0); }
 

@@ -2152,7 +2152,7 @@ int vls_sdf3_adjoint_advect_rk3(vls_sdf3_t h, const double* F, const double* vx,
     if (rc) return rc;
     const Geom& g = h->g;
     const int64_t n = g.n();
-    if ((rc = ensure_adj(h, (size_t)n * (21 + 3 + 4)))) return rc;
+    if ((rc = ensure_adj(h, (size_t)n * (21 + 4)))) return rc;
     double* J = h->adj;
     double* t1 = J + 21 * n;
     double* t2 = t1 + n;

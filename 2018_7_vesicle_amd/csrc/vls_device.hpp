@@ -249,9 +249,6 @@ __device__ __forceinline__ void weno5_pair(S& d_fore, S& d_back, const S p[7], J
 // fewer instructions than scaling the indicators by a power of two and
 // forming their fourth powers.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float fmaxf_(float a, float b) { return (a < b) ? b : a; }
-__device__ __forceinline__ float fminf_(float a, float b) { return (a < b) ? a : b; }
-
 // the correction Q(a, b, c, d) of one side.  The indicators enter the weights
 // only through their ratios, so they are taken divided by 1 + 3/13 (the floor
 // with them: the FP32 e of the axis constants is e * 13/16) and completed to
@@ -713,30 +710,21 @@ __device__ __forceinline__ PairT<S> weno_nonuniform_pair(const S v[7], S r1, S l
 // min(0, l, -r) inside and max(0, l, -r) outside.  Squaring depends only on
 // the magnitude, so the result is bit-identical to the reference's form with
 // a third of the (half-rate) min/max operations.
-template <typename S>
-__device__ __forceinline__ S godunov_axis(bool inside, S l, S r)
-{
-    const S z(0.0);
-    const S m = inside ? dmin(dmin(z, l), -r) : dmax(dmax(z, l), -r);
-    return m * m;
-}
-// the same selections for double with each comparison's outcome flipped inside,
-// instead of both extrema and a choice between them (7 instructions, not 14)
+// The selections flip each comparison's outcome inside instead of forming both
+// extrema and choosing between them (7 instructions, not 14).
 __device__ __forceinline__ double godunov_axis(bool inside, double l, double r)
 {
     const double m = ((0.0 < l) != inside) ? l : 0.0;
     const double n = ((m < -r) != inside) ? -r : m;
     return n * n;
 }
-template <typename S>
-__device__ __forceinline__ S godunov_step(bool inside, S xR, S xL, S yF, S yB, S zU, S zD, S dt)
+__device__ __forceinline__ double godunov_step(bool inside, double xR, double xL, double yF, double yB, double zU,
+                                               double zD, double dt)
 {
-    const S g = godunov_axis(inside, xL, xR) + godunov_axis(inside, yB, yF) + godunov_axis(inside, zD, zU);
-    const S s = (sqrt(g) - 1.0) * dt;
+    const double g = godunov_axis(inside, xL, xR) + godunov_axis(inside, yB, yF) + godunov_axis(inside, zD, zU);
+    const double s = (sqrt(g) - 1.0) * dt;
     return inside ? -s : s;
 }
-
-__device__ __forceinline__ float fsq(float a) { return a * a; }
 
 // FP32 form of godunov_step (bulk points): the three-way extremum of
 // godunov_axis as one v_min3 / v_max3 per axis

@@ -132,22 +132,6 @@ __device__ __forceinline__ Dual<N> operator+(const Dual<N>& a, double b)
     return r;
 }
 template <int N>
-__device__ __forceinline__ Dual<N> operator-(double a, const Dual<N>& b)
-{
-    Dual<N> r;
-    r.v = a - b.v;
-#pragma unroll
-    for (int k = 0; k < N; ++k) r.d[k] = -b.d[k];
-    return r;
-}
-template <int N>
-__device__ __forceinline__ Dual<N> operator-(const Dual<N>& a, double b)
-{
-    Dual<N> r = a;
-    r.v = a.v - b;
-    return r;
-}
-template <int N>
 __device__ __forceinline__ Dual<N> operator*(double a, const Dual<N>& b)
 {
     Dual<N> r;
@@ -164,20 +148,6 @@ __device__ __forceinline__ Dual<N> operator*(const Dual<N>& a, double b)
 #pragma unroll
     for (int k = 0; k < N; ++k) r.d[k] = a.d[k] * b;
     return r;
-}
-template <int N>
-__device__ __forceinline__ Dual<N> operator/(const Dual<N>& a, double b)
-{
-    Dual<N> r;
-    r.v = a.v / b;
-#pragma unroll
-    for (int k = 0; k < N; ++k) r.d[k] = a.d[k] / b;
-    return r;
-}
-template <int N>
-__device__ __forceinline__ Dual<N> operator/(double a, const Dual<N>& b)
-{
-    return dconst<N>(a) / b;
 }
 
 template <int N>
@@ -210,16 +180,6 @@ __device__ __forceinline__ Dual<N> sqrt(const Dual<N>& a)
     return r;
 }
 
-template <int N>
-__device__ __forceinline__ Dual<N> dmax(const Dual<N>& a, const Dual<N>& b)
-{
-    return (a.v < b.v) ? b : a;
-}
-template <int N>
-__device__ __forceinline__ Dual<N> dmin(const Dual<N>& a, const Dual<N>& b)
-{
-    return (a.v < b.v) ? a : b;
-}
 template <int N>
 __device__ __forceinline__ Dual<N> sq(const Dual<N>& a)
 {

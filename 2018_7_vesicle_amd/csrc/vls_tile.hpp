@@ -272,13 +272,6 @@ struct IList {
     const double* dt;
     int cap;
 };
-struct IListW {
-    const int* idx;
-    const int* count;
-    double* dist;
-    double* dt;
-    int cap;
-};
 
 __device__ __forceinline__ bool frozen(const Dists& q, double dx)
 {
@@ -499,16 +492,11 @@ __device__ __forceinline__ int xcd_remap(int blk, int nblk)
     return x * (nblk >> 3) + (x < rem ? x : rem) + (blk >> 3);
 }
 
-// tiles per column and per row of a page, and in a box
+// tiles per column and per row of a page
 template <int R>
 __host__ __device__ inline int tiles_per_col(int rows) { return (rows + R - 1) / R; }
 template <int R>
 __host__ __device__ inline int tiles_per_row(int cols) { return (cols + Shape<R>::TC - 1) / Shape<R>::TC; }
-template <int R>
-__host__ __device__ inline int box_tiles(int rows, int cols, int pges)
-{
-    return tiles_per_col<R>(rows) * tiles_per_row<R>(cols) * pges;
-}
 
 // tile number `blk` of the box (rows fastest, then cols, then pages)
 template <int R>

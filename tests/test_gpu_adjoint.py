@@ -197,8 +197,8 @@ def test_dot_product_on_thin_boxes(box):
     m = vls.SDF3(G, F)
     _, Fdo = _tangent_advect(m, F, Fd, u, ud, 0.01)
     lin, gu = torch.empty_like(F), [torch.zeros_like(F) for _ in range(3)]
-    vls.lib().vls_sdf3_adjoint_advect_rk3(m._h, _p(F), *[_p(c) for c in u], ctypes.c_double(0.01), _p(lam), _p(lin),
-                                          *[_p(c) for c in gu], None)
+    assert vls.lib().vls_sdf3_adjoint_advect_rk3(m._h, _p(F), *[_p(c) for c in u], ctypes.c_double(0.01), _p(lam),
+                                                 _p(lin), *[_p(c) for c in gu], None) == 0
     rhs = lin * Fd + sum(a * b for a, b in zip(gu, ud))
     scale = float((lam * Fdo).abs().sum() + (lin * Fd).abs().sum())
     assert abs(float((lam * Fdo).sum() - rhs.sum())) <= 1e-13 * scale

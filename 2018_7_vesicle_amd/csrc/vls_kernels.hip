@@ -288,10 +288,12 @@ __global__ void k_set_mask_bit(uint8_t* __restrict__ flags, const T* __restrict_
 // The drop-in re_step.  An axis beside a sign change takes the nonuniform
 // stencil, as a job of the block (axis_jobs).  Measured on 100 x 109 x 91 (1.0 M
 // points, a closed surface), a lane for its three axes and 64 x 4 tiles before:
-// re_step 55 -> 39 us, extend_step 55 -> 42, upwind_normal 51 -> 28,
-// boundary_interpolant 48 -> 16, boundary_location 55 -> 15; the first three are
-// bound by their FP64 arithmetic, the last two by memory.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_re_step(double* __restrict__ step, const double* __restrict__ lsf,
+// re_step 58 -> 33 us, extend_step 58 -> 32, upwind_normal 54 -> 30,
+// boundary_interpolant 52 -> 16, boundary_location 55 -> 14; the first three are
+// bound by their FP64 arithmetic, the last two by memory.  Held to the 128
+// registers of four waves a SIMD, re_step and extend_step spilled 32 and 38 of
+// them and took 39 and 40 us here, 292 and 310 at 192^3 (230 and 234 so).
+__global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, const double* __restrict__ lsf,
                                                  const uint8_t* __restrict__ mask,
                                                  const double* __restrict__ deltat, Dist6c d, Box b, Inv inv,
                                                  RowDiv rd)
@@ -573,7 +575,7 @@ __device__ __forceinline__ double upwind_normal_axis(const double v[7], JPd j, b
 // re_step and extend_step this takes a point whatever its distances, and their
 // reciprocals and the squares of the differences by them overflow
 template <typename T>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_upwind_normal(T* __restrict__ nx, T* __restrict__ ny,
+__global__ void __launch_bounds__(256) k_upwind_normal(T* __restrict__ nx, T* __restrict__ ny,
                                                        T* __restrict__ nz, const T* __restrict__ lsf,
                                                        Dist6c d, Box b, Inv inv, RowDiv rd)
 {
@@ -750,7 +752,7 @@ __global__ void __launch_bounds__(256) k_boundary_interpolant(Dist6 cp, Dist6c d
 // drop-in extend_step: extend_step.cu:10-125.  An axis with a distance below the
 // spacing takes the nonuniform stencil, as a job of the block (axis_jobs); the
 // interface values are read there only.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_extend_step(double* __restrict__ step, const double* __restrict__ deltat,
+__global__ void __launch_bounds__(256) k_extend_step(double* __restrict__ step, const double* __restrict__ deltat,
                                                      const double* __restrict__ C, const double* __restrict__ vx,
                                                      const double* __restrict__ vy, const double* __restrict__ vz,
                                                      Dist6c d, Dist6c cp, Box b, Inv inv, RowDiv rd)

@@ -34,7 +34,7 @@ __global__ void __launch_bounds__(256) k_boundary_location(Dist6 d, const T* __r
 {
     __shared__ unsigned short job[3 * 256];
     __shared__ int njobs;
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point(b, rd, (int)threadIdx.x);
     const idx_t plane = (idx_t)b.rows * b.cols;
     unsigned need = 0;
     if (q.valid) {
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(256) k_boundary_location(Dist6 d, const T* __r
         need = (f0 * fx < 0 ? 1u : 0u) | (f0 * fy < 0 ? 2u : 0u) | (f0 * fz < 0 ? 4u : 0u);
     }
     axis_jobs(need, job, &njobs, [&](int t, int a) {
-        const PagePoint o = page_point_of(b, rd, t);
+        const PagePoint o = page_point(b, rd, t);
         double v[7];
         line7_lane(lsf, o.r, o.c, o.p, a, b, v);
         const double ds = a == 0 ? b.dx : (a == 1 ? b.dy : b.dz);
@@ -293,6 +293,7 @@ __global__ void k_set_mask_bit(uint8_t* __restrict__ flags, const T* __restrict_
 // bound by their FP64 arithmetic, the last two by memory.  Held to the 128
 // registers of four waves a SIMD, re_step and extend_step spilled 32 and 38 of
 // them and took 39 and 40 us here, 292 and 310 at 192^3 (230 and 234 so).
+template <bool TILES>
 __global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, const double* __restrict__ lsf,
                                                  const uint8_t* __restrict__ mask,
                                                  const double* __restrict__ deltat, Dist6c d, Box b, Inv inv,
@@ -301,7 +302,7 @@ __global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, cons
     __shared__ double pair[3][2][256];
     __shared__ unsigned short job[3 * 256];
     __shared__ int njobs;
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point<TILES>(b, rd, (int)threadIdx.x);
     const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
     double fo[3] = {0.0, 0.0, 0.0}, bk[3] = {0.0, 0.0, 0.0};
     unsigned need = 0;
@@ -322,7 +323,7 @@ __global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, cons
         }
     }
     axis_jobs(need, job, &njobs, [&](int t, int a) {
-        const PagePoint o = page_point_of(b, rd, t);
+        const PagePoint o = page_point<TILES>(b, rd, t);
         const double ds = a == 0 ? b.dx : (a == 1 ? b.dy : b.dz);
         const double r1 = (a == 0 ? d.r[0] : (a == 1 ? d.r[1] : d.r[2]))[page + o.in];
         const double l1 = (a == 0 ? d.l[0] : (a == 1 ? d.l[1] : d.l[2]))[page + o.in];
@@ -529,7 +530,7 @@ __global__ void __launch_bounds__(256) k_eno2_stage(double* __restrict__ out, co
                                                     const double* __restrict__ fn, const uint8_t* __restrict__ flags,
                                                     Dist6c d, Box b, RowDiv rd, double cfl, int heun2)
 {
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point(b, rd, (int)threadIdx.x);
     if (!q.valid) return;
     const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
     double v[3][5];
@@ -574,7 +575,7 @@ __device__ __forceinline__ double upwind_normal_axis(const double v[7], JPd j, b
 // job of the block (axis_jobs), with the division for its quotients: unlike
 // re_step and extend_step this takes a point whatever its distances, and their
 // reciprocals and the squares of the differences by them overflow
-template <typename T>
+template <bool TILES, typename T>
 __global__ void __launch_bounds__(256) k_upwind_normal(T* __restrict__ nx, T* __restrict__ ny,
                                                        T* __restrict__ nz, const T* __restrict__ lsf,
                                                        Dist6c d, Box b, Inv inv, RowDiv rd)
@@ -582,7 +583,7 @@ __global__ void __launch_bounds__(256) k_upwind_normal(T* __restrict__ nx, T* __
     __shared__ double one[3][256];
     __shared__ unsigned short job[3 * 256];
     __shared__ int njobs;
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point<TILES>(b, rd, (int)threadIdx.x);
     const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
     const double sp[3] = {b.dx, b.dy, b.dz};
     T* out[3] = {nx, ny, nz};
@@ -598,7 +599,7 @@ __global__ void __launch_bounds__(256) k_upwind_normal(T* __restrict__ nx, T* __
         }
     }
     axis_jobs(need, job, &njobs, [&](int t, int a) {
-        const PagePoint o = page_point_of(b, rd, t);
+        const PagePoint o = page_point<TILES>(b, rd, t);
         const double ds = a == 0 ? b.dx : (a == 1 ? b.dy : b.dz);
         const double r1 = (a == 0 ? d.r[0] : (a == 1 ? d.r[1] : d.r[2]))[page + o.in];
         const double l1 = (a == 0 ? d.l[0] : (a == 1 ? d.l[1] : d.l[2]))[page + o.in];
@@ -721,7 +722,7 @@ __global__ void __launch_bounds__(256) k_boundary_interpolant(Dist6 cp, Dist6c d
     __shared__ double val[6][256];
     __shared__ unsigned short job[6 * 256];
     __shared__ int njobs;
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point(b, rd, (int)threadIdx.x);
     const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
     const double sp[3] = {b.dx, b.dy, b.dz};
     unsigned need = 0;
@@ -731,7 +732,7 @@ __global__ void __launch_bounds__(256) k_boundary_interpolant(Dist6 cp, Dist6c d
             need |= (d.r[a][ind] < sp[a] ? 1u << 2 * a : 0u) | (d.l[a][ind] < sp[a] ? 2u << 2 * a : 0u);
     }
     axis_jobs(need, job, &njobs, [&](int t, int k) {
-        const PagePoint o = page_point_of(b, rd, t);
+        const PagePoint o = page_point(b, rd, t);
         const int a = k >> 1;
         const bool back = k & 1;
         const double* dis = back ? (a == 0 ? d.l[0] : (a == 1 ? d.l[1] : d.l[2]))
@@ -752,6 +753,7 @@ __global__ void __launch_bounds__(256) k_boundary_interpolant(Dist6 cp, Dist6c d
 // drop-in extend_step: extend_step.cu:10-125.  An axis with a distance below the
 // spacing takes the nonuniform stencil, as a job of the block (axis_jobs); the
 // interface values are read there only.
+template <bool TILES>
 __global__ void __launch_bounds__(256) k_extend_step(double* __restrict__ step, const double* __restrict__ deltat,
                                                      const double* __restrict__ C, const double* __restrict__ vx,
                                                      const double* __restrict__ vy, const double* __restrict__ vz,
@@ -760,7 +762,7 @@ __global__ void __launch_bounds__(256) k_extend_step(double* __restrict__ step, 
     __shared__ double pair[3][2][256];
     __shared__ unsigned short job[3 * 256];
     __shared__ int njobs;
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point<TILES>(b, rd, (int)threadIdx.x);
     const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
     const double sp[3] = {b.dx, b.dy, b.dz};
     double fo[3] = {0.0, 0.0, 0.0}, bk[3] = {0.0, 0.0, 0.0};
@@ -782,7 +784,7 @@ __global__ void __launch_bounds__(256) k_extend_step(double* __restrict__ step, 
         }
     }
     axis_jobs(need, job, &njobs, [&](int t, int a) {
-        const PagePoint o = page_point_of(b, rd, t);
+        const PagePoint o = page_point<TILES>(b, rd, t);
         const idx_t at = page + o.in;
         const double ds = a == 0 ? b.dx : (a == 1 ? b.dy : b.dz);
         const double r1 = (a == 0 ? d.r[0] : (a == 1 ? d.r[1] : d.r[2]))[at];
@@ -878,13 +880,26 @@ __device__ __forceinline__ double advect_rate(const double* __restrict__ f, int 
     return acc;
 }
 
+// PAGES: pages in memory order (page_point), for boxes whose 64 x 4 tiles hold
+// more than 20% more points than the box.  Measured on MI355X, tiles -> memory
+// order (rows x columns x pages): 200 x 17 x 180 15.9 -> 12.2 us, 8 x 8 x 2000 18.7 ->
+// 4.6, 37 x 160 x 200 25.9 -> 18.5; 109 x 100 x 91 equal, 128^3 27.6 -> 30.0.
+template <bool PAGES>
 __global__ void __launch_bounds__(256) k_advection_step(double* __restrict__ astep, const double* __restrict__ vx,
                                                         const double* __restrict__ vy,
                                                         const double* __restrict__ vz,
-                                                        const double* __restrict__ lsf, Box b, Inv inv)
+                                                        const double* __restrict__ lsf, Box b, Inv inv, RowDiv rd)
 {
     int r, c, p;
-    if (!point_of_thread(b, r, c, p)) return;
+    if constexpr (PAGES) {
+        const PagePoint q = page_point(b, rd, (int)threadIdx.x);
+        if (!q.valid) return;
+        r = q.r;
+        c = q.c;
+        p = q.p;
+    } else if (!point_of_thread(b, r, c, p)) {
+        return;
+    }
     const idx_t ind = lin(b, r, c, p);
     const double vel[3] = {vx[ind], vy[ind], vz[ind]};
     astep[ind] = advect_rate(lsf, r, c, p, b, inv, vel);
@@ -1375,6 +1390,18 @@ static inline dim3 flat_grid(int64_t n) { return dim3((unsigned)((n + 255) / 256
         return hipGetLastError();                                                                     \
     } while (0)
 
+// ... or over 64 x 4 tiles for boxes of 192 rows on whose tiles hold at most 5%
+// more.  Measured on MI355X, memory order -> tiles: extend_step at 192^3 232 ->
+// 225 us, 500 x 500 x 6 44 -> 40 (42 as a lane for its three axes), upwind_normal
+// there 37.6 -> 34.6 (36.6), but re_step at 128^3 63.8 -> 66.0 and at 60 rows 31.0 ->
+// 32.1, boundary_interpolant at 192^3 118 -> 123.
+#define VLS_WALK_LAUNCH(tiles, pages, ...)                                                             \
+    do {                                                                                               \
+        if (g.rows < 192 || !tiles_fit(g.rows, g.cols, 5)) VLS_PAGE_LAUNCH(pages, __VA_ARGS__);        \
+        tiles<<<page_grid<true>(g.rows, g.cols, g.pges), dim3(256), 0, s>>>(__VA_ARGS__, RowDiv{});    \
+        return hipGetLastError();                                                                      \
+    } while (0)
+
 #define VLS_POINT_LAUNCH(kernel, ...)                                   \
     do {                                                                \
         dim3 grid_, block_;                                             \
@@ -1521,7 +1548,7 @@ hipError_t launch_set_mask_bit(uint8_t* flags, const T* F, const Geom& g, hipStr
 hipError_t launch_re_step(double* step, const double* lsf, const uint8_t* mask, const double* deltat,
                           const Dist6c& d, const Geom& g, hipStream_t s)
 {
-    VLS_PAGE_LAUNCH(k_re_step, step, lsf, mask, deltat, d, box_of(g), inv_of(g));
+    VLS_WALK_LAUNCH(k_re_step<true>, k_re_step<false>, step, lsf, mask, deltat, d, box_of(g), inv_of(g));
 }
 
 hipError_t launch_eno2_re_step(double* step, const double* lsf, const uint8_t* mask, const double* deltat,
@@ -1594,7 +1621,7 @@ hipError_t launch_eno2_stage(double* out, const double* fs, const double* fn, co
 template <typename T>
 hipError_t launch_upwind_normal(T* nx, T* ny, T* nz, const T* lsf, const Dist6c& d, const Geom& g, hipStream_t s)
 {
-    VLS_PAGE_LAUNCH(k_upwind_normal<T>, nx, ny, nz, lsf, d, box_of(g), inv_of(g));
+    VLS_WALK_LAUNCH((k_upwind_normal<true, T>), (k_upwind_normal<false, T>), nx, ny, nz, lsf, d, box_of(g), inv_of(g));
 }
 
 template <typename T>
@@ -1630,7 +1657,7 @@ hipError_t launch_extend_step(double* step, const double* deltat, const double* 
                               const double* vy, const double* vz, const Dist6c& d, const Dist6c& cp,
                               const Geom& g, hipStream_t s)
 {
-    VLS_PAGE_LAUNCH(k_extend_step, step, deltat, C, vx, vy, vz, d, cp, box_of(g), inv_of(g));
+    VLS_WALK_LAUNCH(k_extend_step<true>, k_extend_step<false>, step, deltat, C, vx, vy, vz, d, cp, box_of(g), inv_of(g));
 }
 
 template <typename T, int S>
@@ -1668,7 +1695,9 @@ hipError_t launch_cubic_extend_stage(double* out, const double* cs, const double
 hipError_t launch_advection_step(double* astep, const double* vx, const double* vy, const double* vz,
                                  const double* lsf, const Geom& g, hipStream_t s)
 {
-    VLS_POINT_LAUNCH(k_advection_step, astep, vx, vy, vz, lsf, box_of(g), inv_of(g));
+    if (!tiles_fit(g.rows, g.cols, 20))
+        VLS_PAGE_LAUNCH(k_advection_step<true>, astep, vx, vy, vz, lsf, box_of(g), inv_of(g));
+    VLS_POINT_LAUNCH(k_advection_step<false>, astep, vx, vy, vz, lsf, box_of(g), inv_of(g), RowDiv{});
 }
 
 template <typename T>

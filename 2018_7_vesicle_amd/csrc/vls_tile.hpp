@@ -36,40 +36,47 @@ inline RowDiv row_div(int rows)
     return RowDiv{(unsigned)(((1ull << (26 + l)) + (unsigned)rows - 1) / (unsigned)rows), 26 + l};
 }
 
-// A point kernel's thread over pages in memory order: 256 consecutive points of
-// page blockIdx.y, whatever the rows (64 x 4 tiles leave a quarter of the
-// lanes of a 96-row box idle)
+// A point kernel's threads over pages (blockIdx.y): 256 consecutive points of the
+// page in memory order, whatever the rows (64 x 4 tiles leave a quarter of the
+// lanes of a 96-row box idle), or, TILES, 64 x 4 tiles, whose four columns share
+// their x-taps
 struct PagePoint {
     int r, c, p;
     unsigned in;  // index within the page
     bool valid;
 };
-__device__ __forceinline__ PagePoint page_point(const Box& b, RowDiv d)
+// the point of thread t of this block
+template <bool TILES = false>
+__device__ __forceinline__ PagePoint page_point(const Box& b, RowDiv d, int t)
 {
     PagePoint q;
-    q.in = blockIdx.x * 256u + threadIdx.x;
-    q.valid = q.in < (unsigned)b.rows * (unsigned)b.cols;
     q.p = (int)blockIdx.y;
-    if (!q.valid) q.in = 0;
-    q.c = (int)(((unsigned long long)q.in * d.m) >> d.s);
-    q.r = (int)q.in - q.c * b.rows;
+    if constexpr (TILES) {
+        const int ntr = (b.rows + 63) >> 6, cb = (int)blockIdx.x / ntr;
+        q.r = ((int)blockIdx.x - cb * ntr) * 64 + (t & 63);
+        q.c = cb * 4 + (t >> 6);
+        q.valid = q.r < b.rows && q.c < b.cols;
+        if (!q.valid) q.r = q.c = 0;
+        q.in = (unsigned)(q.c * b.rows + q.r);
+    } else {
+        q.in = blockIdx.x * 256u + (unsigned)t;
+        q.valid = q.in < (unsigned)b.rows * (unsigned)b.cols;
+        if (!q.valid) q.in = 0;
+        q.c = (int)(((unsigned long long)q.in * d.m) >> d.s);
+        q.r = (int)q.in - q.c * b.rows;
+    }
     return q;
 }
+template <bool TILES = false>
 inline dim3 page_grid(int rows, int cols, int pges)
 {
-    return dim3((unsigned)(((int64_t)rows * cols + 255) / 256), (unsigned)pges);
+    return TILES ? dim3((unsigned)((rows + 63) / 64) * (unsigned)((cols + 3) / 4), (unsigned)pges)
+                 : dim3((unsigned)(((int64_t)rows * cols + 255) / 256), (unsigned)pges);
 }
-
-// thread t of this block as page_point numbers it (a valid one)
-__device__ __forceinline__ PagePoint page_point_of(const Box& b, RowDiv d, int t)
+// whether a page's 64 x 4 tiles hold at most `percent` of its points beyond them
+inline bool tiles_fit(int rows, int cols, int percent)
 {
-    PagePoint q;
-    q.in = blockIdx.x * 256u + (unsigned)t;
-    q.valid = true;
-    q.p = (int)blockIdx.y;
-    q.c = (int)(((unsigned long long)q.in * d.m) >> d.s);
-    q.r = (int)q.in - q.c * b.rows;
-    return q;
+    return (int64_t)((rows + 63) / 64) * ((cols + 3) / 4) * 256 * 100 <= (int64_t)rows * cols * (100 + percent);
 }
 
 // The long evaluations of a point kernel (the nonuniform stencil, the quintic

@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(256) k_enork2_extend_stage(double* __restrict_
                                                              Box b, RowDiv rd, int heun2)
 {
 #pragma clang fp contract(off)
-    const PagePoint q = page_point(b, rd);
+    const PagePoint q = page_point(b, rd, (int)threadIdx.x);
     if (!q.valid) return;
     const idx_t page = (idx_t)q.p * b.rows * b.cols, ind = page + q.in;
     double v[3][5], fo[3], bk[3];

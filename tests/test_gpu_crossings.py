@@ -122,3 +122,19 @@ def test_extend_step_beside_huge_values():
     vls.feval_extend_step(ext, T(dt), T(C), *[T(a) for a in vel], *[T(a) for a in d6], *[T(a) for a in cp6],
                           33, 9, 5, *sp, C.size)
     assert np.array_equal(ext.cpu().numpy(), ref, equal_nan=True)
+
+
+@pytest.mark.parametrize("shape", [(53, 8, 3), (54, 8, 3), (191, 8, 2), (192, 4, 2), (193, 4, 2), (500, 8, 3),
+                                   (500, 7, 2), (1021, 43, 2)])
+def test_point_kernels_on_either_walk(shape):
+    """the boxes where the point kernels change between pages in memory order and
+    64 x 4 tiles (from 192 rows on if they fit within 5%; advection_step within
+    20%), with whole tiles and with ragged ones"""
+    test_point_kernels_with_every_axis_beside_a_crossing(shape)
+    rows, cols, pges = shape
+    sp = (0.11, 0.07, 0.13)
+    rng = np.random.default_rng(rows)
+    F, *vel = [rng.normal(size=(pges, cols, rows)) for _ in range(4)]
+    out = torch.full(F.shape, np.nan, dtype=torch.float64, device="cuda")
+    vls.feval_advection_step(out, *[T(a) for a in vel], T(F), rows, cols, pges, *sp)
+    assert np.array_equal(out.cpu().numpy(), po.advection_step(vel, F, *sp))

@@ -122,7 +122,7 @@ __global__ void __launch_bounds__(256) k_crossings(Dist6 d, double* __restrict__
 template <int R, typename T>
 __global__ void __launch_bounds__(256) k_crossings_z(Dist6 d, double* __restrict__ min_dist,
                                                      uint8_t* __restrict__ flags, int mask,
-                                                     const T* __restrict__ lsf, Box b, int depth,
+                                                     const T* __restrict__ lsf, Box b, ZShare zs,
                                                      int* __restrict__ cand, int* __restrict__ cand_count)
 {
     __shared__ T lds[2][Shape<R>::N];
@@ -130,7 +130,7 @@ __global__ void __launch_bounds__(256) k_crossings_z(Dist6 d, double* __restrict
     BlockList<1024> bl{cbuf, &ccount, &cbase};
     bl.init();
     int r0, c0, p0, p1;
-    zmarch_share<R>(b, depth, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
+    zmarch_share<R>(zs, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
     const idx_t plane = (idx_t)b.rows * b.cols;
     const double md = dmin(dmin(b.dx, b.dx), dmin(dmin(b.dy, b.dy), dmin(b.dz, b.dz)));
     zmarch<R, T, false, false>(lds[0], lds[1], b, r0, c0, p0, p1, lsf, nullptr, nullptr, nullptr, nullptr, nullptr,
@@ -361,7 +361,7 @@ __global__ void __launch_bounds__(256) k_re_step(double* __restrict__ step, cons
 template <int R, typename T, int S = IFACE_WENO>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStageWaves))) k_reinit_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                       const T* __restrict__ fn, const uint8_t* __restrict__ flags,
-                                                      IList il, Box b, Inv invs, int stage, int depth, int niface)
+                                                      IList il, Box b, Inv invs, int stage, ZShare zs, int niface)
 {
     __shared__ T lds[2][Shape<R>::N];
     __shared__ unsigned short job[defers_crossings<T>() ? 256 * kDeferPages : 1];
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
     const idx_t plane = (idx_t)b.rows * b.cols;
     int r0 = 0, c0 = 0, p0 = 0, p1 = 0;
     if (!lists) {
-        zmarch_share<R>(b, depth, blk - niface, (int)gridDim.x - niface, r0, c0, p0, p1);
+        zmarch_share<R>(zs, blk - niface, (int)gridDim.x - niface, r0, c0, p0, p1);
         if (threadIdx.x == 0) njobs = 0;  // before the march's first barrier
         ZFace<T> zf;
         zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, fs, fn, nullptr, nullptr, nullptr, flags, stage,
@@ -655,11 +655,11 @@ template <int R, typename T>
 __global__ void __launch_bounds__(256) k_extension_normal_z(T* __restrict__ vx, T* __restrict__ vy,
                                                             T* __restrict__ vz, const T* __restrict__ lsf,
                                                             const uint8_t* __restrict__ flags, double floor_, Box b,
-                                                            int depth)
+                                                            ZShare zs)
 {
     __shared__ T lds[2][Shape<R>::N];
     int r0, c0, p0, p1;
-    zmarch_share<R>(b, depth, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
+    zmarch_share<R>(zs, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
     const idx_t plane = (idx_t)b.rows * b.cols;
     const double sp[3] = {b.dx, b.dy, b.dz};
     zmarch<R, T, false, true>(lds[0], lds[1], b, r0, c0, p0, p1, lsf, nullptr, nullptr, nullptr, nullptr, flags, 0,
@@ -831,7 +831,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
                                                       const T* __restrict__ vy, const T* __restrict__ vz,
                                                       IList il, const double* __restrict__ lcp,
                                                       const double* __restrict__ lv, Box b, Inv inv, int stage,
-                                                      int depth, int niface)
+                                                      ZShare zs, int niface)
 {
     __shared__ T lds[2][Shape<R>::N];
     const int blk = (int)blockIdx.x;
@@ -850,7 +850,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
         return;
     }
     int r0, c0, p0, p1;
-    zmarch_share<R>(b, depth, blk - niface, (int)gridDim.x - niface, r0, c0, p0, p1);
+    zmarch_share<R>(zs, blk - niface, (int)gridDim.x - niface, r0, c0, p0, p1);
     const idx_t plane = (idx_t)b.rows * b.cols;
     // the listed points carry a NaN x-velocity (k_list_gather_vel), so the
     // bulk needs no flags: it skips them and the lanes outside the box
@@ -910,11 +910,11 @@ template <int R, typename T>
 __global__ void __launch_bounds__(256) k_advect_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                       const T* __restrict__ fn, const T* __restrict__ vx,
                                                       const T* __restrict__ vy, const T* __restrict__ vz,
-                                                      double dt, Box b, Inv inv, int stage, int depth)
+                                                      double dt, Box b, Inv inv, int stage, ZShare zs)
 {
     __shared__ T lds[2][Shape<R>::N];
     int r0, c0, p0, p1;
-    zmarch_share<R>(b, depth, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
+    zmarch_share<R>(zs, (int)blockIdx.x, (int)gridDim.x, r0, c0, p0, p1);
     const idx_t plane = (idx_t)b.rows * b.cols;
     ZDiff<T> zd;
     zmarch<R, T, true, false>(lds[0], lds[1], b, r0, c0, p0, p1, fs, fn, vx, vy, vz, nullptr, stage,
@@ -1419,6 +1419,7 @@ hipError_t launch_boundary_location(int order, const Dist6& d, const T* lsf, con
 }
 
 static inline int bulk_blocks(const Geom& g, int depth);
+static inline ZShare bulk_shares(const Geom& g, int depth);
 
 template <typename T>
 hipError_t launch_set_distance(int order, const Dist6& d, double* min_dist, uint8_t* flags, const T* mask_src,
@@ -1430,12 +1431,13 @@ hipError_t launch_set_distance(int order, const Dist6& d, double* min_dist, uint
     k_zero_pair<<<dim3(1), dim3(64), 0, s>>>(cand_count, lv.idx ? lv.count : nullptr);
     if (!mask_src || (const void*)mask_src == (const void*)lsf) {
         const int zd = zmarch_depth(g), m = mask_src ? 1 : 0;
+        const ZShare zs = bulk_shares(g, zd);
         if (tile_rows(g) == 32)
             k_crossings_z<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(d, min_dist, flags, m, lsf, box_of(g),
-                                                                               zd, cand, cand_count);
+                                                                               zs, cand, cand_count);
         else
             k_crossings_z<64, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(d, min_dist, flags, m, lsf, box_of(g),
-                                                                               zd, cand, cand_count);
+                                                                               zs, cand, cand_count);
     } else {
         k_crossings<T><<<grid, block, 0, s>>>(d, min_dist, flags, mask_src, lsf, box_of(g), cand, cand_count);
     }
@@ -1537,6 +1539,11 @@ static inline int bulk_blocks(const Geom& g, int depth)
     return tile_rows(g) == 32 ? zmarch_blocks<32>(g.rows, g.cols, g.pges, depth)
                       : zmarch_blocks<64>(g.rows, g.cols, g.pges, depth);
 }
+static inline ZShare bulk_shares(const Geom& g, int depth)
+{
+    return tile_rows(g) == 32 ? zmarch_shares<32>(g.rows, g.cols, g.pges, depth)
+                              : zmarch_shares<64>(g.rows, g.cols, g.pges, depth);
+}
 
 template <typename T>
 hipError_t launch_set_mask_bit(uint8_t* flags, const T* F, const Geom& g, hipStream_t s)
@@ -1563,12 +1570,13 @@ static hipError_t reinit_stage_scheme(T* out, const T* fs, const T* fn, const ui
 {
     const IList il{lv.idx, lv.count, lv.dist, lv.dt, lv.cap};
     const int zd = reinit_depth<T>(zmarch_depth(g)), ni = fused_iface_blocks(g);
+    const ZShare zs = bulk_shares(g, zd);
     const dim3 grid(bulk_blocks(g, zd) + ni);
     if (tile_rows(g) == 32)
-        k_reinit_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage, zd,
+        k_reinit_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage, zs,
                                                             ni);
     else
-        k_reinit_stage<64, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage, zd,
+        k_reinit_stage<64, T, S><<<grid, dim3(256), 0, s>>>(out, fs, fn, flags, il, box_of(g), inv_of(g), stage, zs,
                                                             ni);
     return hipGetLastError();
 }
@@ -1629,12 +1637,13 @@ hipError_t launch_extension_normal(T* vx, T* vy, T* vz, const T* F, const uint8_
                                    double floor_, const Geom& g, hipStream_t s)
 {
     const int zd = zmarch_depth(g);
+    const ZShare zs = bulk_shares(g, zd);
     if (tile_rows(g) == 32)
         k_extension_normal_z<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(vx, vy, vz, F, flags, floor_,
-                                                                                  box_of(g), zd);
+                                                                                  box_of(g), zs);
     else
         k_extension_normal_z<64, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(vx, vy, vz, F, flags, floor_,
-                                                                                  box_of(g), zd);
+                                                                                  box_of(g), zs);
     const IList il{lv.idx, lv.count, lv.dist, lv.dt, lv.cap};
     k_extension_normal_list<T><<<dim3(iface_blocks(g)), dim3(256), 0, s>>>(vx, vy, vz, F, il, floor_, box_of(g));
     return hipGetLastError();
@@ -1667,13 +1676,14 @@ static hipError_t extend_stage_scheme(T* out, const T* cs, const T* cn, const T*
 {
     const IList il{lv.idx, lv.count, lv.dist, lv.dt, lv.cap};
     const int zd = zmarch_depth(g), ni = fused_iface_blocks(g);
+    const ZShare zs = bulk_shares(g, zd);
     const dim3 grid(bulk_blocks(g, zd) + ni);
     if (tile_rows(g) == 32)
         k_extend_stage<32, T, S><<<grid, dim3(256), 0, s>>>(out, cs, cn, vx, vy, vz, il, lcp, lvel,
-                                                            box_of(g), inv_of(g), stage, zd, ni);
+                                                            box_of(g), inv_of(g), stage, zs, ni);
     else
         k_extend_stage<64, T, S><<<grid, dim3(256), 0, s>>>(out, cs, cn, vx, vy, vz, il, lcp, lvel,
-                                                            box_of(g), inv_of(g), stage, zd, ni);
+                                                            box_of(g), inv_of(g), stage, zs, ni);
     return hipGetLastError();
 }
 
@@ -1705,12 +1715,13 @@ hipError_t launch_advect_stage(T* out, const T* fs, const T* fn, const T* vx, co
                                const Geom& g, int stage, hipStream_t s)
 {
     const int zd = zmarch_depth(g);
+    const ZShare zs = bulk_shares(g, zd);
     if (tile_rows(g) == 32)
         k_advect_stage<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(out, fs, fn, vx, vy, vz, dt, box_of(g),
-                                                                              inv_of(g), stage, zd);
+                                                                              inv_of(g), stage, zs);
     else
         k_advect_stage<64, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(out, fs, fn, vx, vy, vz, dt, box_of(g),
-                                                                              inv_of(g), stage, zd);
+                                                                              inv_of(g), stage, zs);
     return hipGetLastError();
 }
 

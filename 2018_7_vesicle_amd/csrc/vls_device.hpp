@@ -72,19 +72,22 @@ __device__ __forceinline__ double quot_ieee(double a, const RecipT<double>& r)
     return __builtin_amdgcn_div_fixup(quot(a, r), r.b, a);
 }
 __device__ __forceinline__ double quot_ieee(double a, double b) { return quot_ieee(a, recip(b)); }
-// a over d, a denominator or one with its reciprocal.  IEEE: the division itself;
-// WIDE: a may have overflowed (quot_ieee)
-template <bool IEEE, bool WIDE = false, typename S>
+// How the nonuniform stencils divide: by the unscaled quotients; with those of
+// their overflowing products as the division gives them (WIDE, the default); or
+// by the division throughout
+enum { QUOT_FAST, QUOT_WIDE, QUOT_IEEE };
+// a over d, a denominator or one with its reciprocal; PRODUCT: a may have overflowed
+template <int Q, bool PRODUCT = false, typename S>
 __device__ __forceinline__ S over(const S& a, const S& d)
 {
-    if constexpr (IEEE) return a / d;
-    else if constexpr (WIDE) return quot_ieee(a, d);
+    if constexpr (Q == QUOT_IEEE) return a / d;
+    else if constexpr (Q == QUOT_WIDE && PRODUCT) return quot_ieee(a, d);
     else return quot(a, d);
 }
-template <bool IEEE, typename S>
+template <int Q, typename S>
 __device__ __forceinline__ S over(const S& a, const RecipT<S>& d)
 {
-    if constexpr (IEEE) return a / d.b;
+    if constexpr (Q == QUOT_IEEE) return a / d.b;
     else return quot(a, d);
 }
 // exchanges a and b in the lanes where c holds
@@ -540,9 +543,11 @@ __device__ __forceinline__ void weno5_pair_z(double& d_fore, double& d_back, boo
 // The weights' divisions by (s + eps)^2 stay IEEE: that square overflows for
 // jumps beyond 1e75 spacings, and the weight is then 0.  The products of two
 // divided differences overflow for jumps beyond 1e150 and keep their infinity
-// (over<..., true>, one instruction each), for the same reason.
+// (QUOT_WIDE), for the same reason; the lanes of FP32 fields, which hold no such
+// values, leave that out (QUOT_FAST: their numerators then need not stay in
+// registers; FP32 reinitialization stage at 48^3 8.46 -> 8.22 us).
 // ---------------------------------------------------------------------------
-template <typename S, bool IEEE = false>
+template <typename S, int Q = QUOT_WIDE>
 __device__ __forceinline__ S weno_nonuniform_face(const S* a, const S* u, bool back)
 {
 #pragma clang fp contract(off)
@@ -552,24 +557,24 @@ __device__ __forceinline__ S weno_nonuniform_face(const S* a, const S* u, bool b
     const RecipT<S> X1 = recip(x15 - xm05), X2 = recip(x25 - xm05), X3 = recip(x25 - x05);
     const RecipT<S> Y1 = recip(x05 - xm15), Y2 = recip(x05 - xm25), Y3 = recip(xm05 - xm25);
     const RecipT<S> W3 = recip(x15 - xm15);
-    const S hX2 = over<IEEE>(h, X2), hY2 = over<IEEE>(h, Y2), hW = over<IEEE>(h, W3);
+    const S hX2 = over<Q>(h, X2), hY2 = over<Q>(h, Y2), hW = over<Q>(h, W3);
     // smoothness indicators (re_step.cu:136-178), the same on both sides
     const S h2 = sq(h);
     const S s0 = 4.0 * sq(hX2) *
-        (sq(over<IEEE>(u2 - u1, X3)) * (10.0 * h2 + X1.b * (x15 - x05))
-         + over<IEEE, true>((u2 - u1) * (u0 - u1), X3.b * X1.b) *
+        (sq(over<Q>(u2 - u1, X3)) * (10.0 * h2 + X1.b * (x15 - x05))
+         + over<Q, true>((u2 - u1) * (u0 - u1), X3.b * X1.b) *
                (20.0 * h2 + 2.0 * X1.b * (x15 - x05) + X2.b * (2.0 * x15 - x05 - xm05))
-         + sq(over<IEEE>(u0 - u1, X1)) * (10.0 * h2 + (x25 + x15 - 2.0 * xm05) * (x25 + x15 - x05 - xm05)));
+         + sq(over<Q>(u0 - u1, X1)) * (10.0 * h2 + (x25 + x15 - 2.0 * xm05) * (x25 + x15 - x05 - xm05)));
     const S s1 = 4.0 * sq(hW) *
-        (sq(over<IEEE>(um1 - u0, Y1)) * (10.0 * h2 + X1.b * (x15 - x05))
-         + over<IEEE, true>((u1 - u0) * (um1 - u0), X1.b * Y1.b) *
+        (sq(over<Q>(um1 - u0, Y1)) * (10.0 * h2 + X1.b * (x15 - x05))
+         + over<Q, true>((u1 - u0) * (um1 - u0), X1.b * Y1.b) *
                (20.0 * h2 - (x15 - x05) * (xm05 - xm15) - X1.b * Y1.b)
-         + sq(over<IEEE>(u1 - u0, X1)) * (10.0 * h2 + (xm05 - xm15) * Y1.b));
+         + sq(over<Q>(u1 - u0, X1)) * (10.0 * h2 + (xm05 - xm15) * Y1.b));
     const S s2 = 4.0 * sq(hY2) *
-        (sq(over<IEEE>(um2 - um1, Y3)) * (10.0 * h2 + Y1.b * (xm05 - xm15))
-         + over<IEEE, true>((u0 - um1) * (um2 - um1), Y1.b * Y3.b) *
+        (sq(over<Q>(um2 - um1, Y3)) * (10.0 * h2 + Y1.b * (xm05 - xm15))
+         + over<Q, true>((u0 - um1) * (um2 - um1), Y1.b * Y3.b) *
                (20.0 * h2 + 2.0 * Y1.b * (xm05 - xm15) + Y2.b * (x05 + xm05 - 2.0 * xm15))
-         + sq(over<IEEE>(u0 - um1, Y1)) *
+         + sq(over<Q>(u0 - um1, Y1)) *
                (10.0 * h2 + (2.0 * x05 - xm25 - xm15) * (x05 + xm05 - xm15 - xm25)));
     // the face's side: p1, p2, g downwind of it, q1, q2, m1, m2 upwind (fore: downwind is right)
     RecipT<S> p1 = X1, q1 = Y1, p2 = X2, q2 = Y2, g = X3, m2 = Y3;
@@ -583,14 +588,14 @@ __device__ __forceinline__ S weno_nonuniform_face(const S* a, const S* u, bool b
     swap_if(back, udd, uuu);
     hp2 = back ? hq2 : hp2;
     // the three stencils' values: downwind, central, upwind
-    const S T1 = (u0 - ud) * (1.0 + over<IEEE>(h, p1) + hp2);
+    const S T1 = (u0 - ud) * (1.0 + over<Q>(h, p1) + hp2);
     RecipT<S> A1 = p2, A2 = g;
     swap_if(back, A1, A2);
-    const S T2 = (udd - ud) * over<IEEE>(h, A1) * over<IEEE>(p1.b, A2);
+    const S T2 = (udd - ud) * over<Q>(h, A1) * over<Q>(p1.b, A2);
     const S vd = (ud + (back ? T2 : T1)) + (back ? T1 : T2);
-    const S vc = u0 + (uu - u0) * hW * over<IEEE>(p1.b, q1) - (ud - u0) * hW * over<IEEE>(m1, p1);
-    const S m1q2 = over<IEEE>(m1, q2);
-    const S vu = uu + (u0 - uu) * m1q2 * over<IEEE>(m2.b, q1) - (uuu - uu) * m1q2 * over<IEEE>(h, m2);
+    const S vc = u0 + (uu - u0) * hW * over<Q>(p1.b, q1) - (ud - u0) * hW * over<Q>(m1, p1);
+    const S m1q2 = over<Q>(m1, q2);
+    const S vu = uu + (u0 - uu) * m1q2 * over<Q>(m2.b, q1) - (uuu - uu) * m1q2 * over<Q>(h, m2);
     // their linear weights
     const RecipT<S> T = recip(x25 - xm25), N1 = recip(x25 - xm15), N2 = recip(x15 - xm25);
     RecipT<S> Na = N1, Nb = N2;
@@ -598,16 +603,16 @@ __device__ __forceinline__ S weno_nonuniform_face(const S* a, const S* u, bool b
     S e1 = m2.b, e2 = p2.b, e3 = p1.b, e4 = p2.b;
     swap_if(back, e1, e2);
     swap_if(back, e3, e4);
-    S c0 = over<IEEE>(m1, T) * over<IEEE>(m2.b, Na);
-    const S c1 = over<IEEE>(e1, T) * over<IEEE>(e2, N1) * (1.0 + over<IEEE>(N1.b, N2));
-    S c2 = over<IEEE>(e3, T) * over<IEEE>(e4, Nb);
+    S c0 = over<Q>(m1, T) * over<Q>(m2.b, Na);
+    const S c1 = over<Q>(e1, T) * over<Q>(e2, N1) * (1.0 + over<Q>(N1.b, N2));
+    S c2 = over<Q>(e3, T) * over<Q>(e4, Nb);
     S v0 = vd, v2 = vu;
     swap_if(back, c0, c2);
     swap_if(back, v0, v2);
     const double eps = 1e-6;
     const S al0 = c0 / sq(s0 + eps), al1 = c1 / sq(s1 + eps), al2 = c2 / sq(s2 + eps);
     const RecipT<S> sum = recip(al0 + al1 + al2);
-    return v0 * over<IEEE>(al0, sum) + vc * over<IEEE>(al1, sum) + v2 * over<IEEE>(al2, sum);
+    return v0 * over<Q>(al0, sum) + vc * over<Q>(al1, sum) + v2 * over<Q>(al2, sum);
 }
 
 template <typename S>
@@ -624,7 +629,7 @@ struct NonuniformStencil {
     S x[7], d[6];
 };
 
-template <bool IEEE = false, typename S>
+template <int Q = QUOT_WIDE, typename S>
 __device__ __forceinline__ NonuniformStencil<S> nonuniform_stencil(S p0, S p1, S p2, S p3, S p4, S p5, S p6, S r1,
                                                                    S l1, double ds, S h_fore, S h_back)
 {
@@ -648,7 +653,7 @@ __device__ __forceinline__ NonuniformStencil<S> nonuniform_stencil(S p0, S p1, S
         h[2] = p2; h[1] = p1; h[0] = p0;
     }
 #pragma unroll
-    for (int k = 0; k < 6; ++k) st.d[k] = over<IEEE>(h[k + 1] - h[k], st.x[k + 1] - st.x[k]);
+    for (int k = 0; k < 6; ++k) st.d[k] = over<Q>(h[k + 1] - h[k], st.x[k + 1] - st.x[k]);
     return st;
 }
 
@@ -657,14 +662,14 @@ __device__ __forceinline__ NonuniformStencil<S> nonuniform_stencil(S p0, S p1, S
 // the interface lanes run in blocks of their own); the others call the
 // out-of-line forms: they run only at interface nodes, and scalar arguments
 // and a returned struct keep the caller's stencil in registers.
-template <typename S>
+template <int Q = QUOT_WIDE, typename S>
 __device__ __forceinline__ PairT<S> weno_nonuniform_pair_inl(S p0, S p1, S p2, S p3, S p4, S p5, S p6, S r1, S l1,
                                                              double ds, S h_fore, S h_back)
 {
-    const NonuniformStencil<S> st = nonuniform_stencil(p0, p1, p2, p3, p4, p5, p6, r1, l1, ds, h_fore, h_back);
+    const NonuniformStencil<S> st = nonuniform_stencil<Q>(p0, p1, p2, p3, p4, p5, p6, r1, l1, ds, h_fore, h_back);
     PairT<S> out;
-    out.fore = weno_nonuniform_face(&st.x[1], &st.d[1], false);
-    out.back = weno_nonuniform_face(&st.x[0], &st.d[0], true);
+    out.fore = weno_nonuniform_face<S, Q>(&st.x[1], &st.d[1], false);
+    out.back = weno_nonuniform_face<S, Q>(&st.x[0], &st.d[0], true);
     return out;
 }
 template <typename S>
@@ -674,19 +679,19 @@ __device__ __noinline__ PairT<S> weno_nonuniform_pair(S p0, S p1, S p2, S p3, S 
     return weno_nonuniform_pair_inl(p0, p1, p2, p3, p4, p5, p6, r1, l1, ds, h_fore, h_back);
 }
 
-// one face only: d_fore (back == false) or d_back.  IEEE: every quotient by the
-// division, for a caller that takes any distance
-template <bool IEEE = false, typename S>
+// one face only: d_fore (back == false) or d_back.  QUOT_IEEE is for a caller that
+// takes any distance
+template <int Q = QUOT_WIDE, typename S>
 __device__ __forceinline__ S weno_nonuniform_one_inl(S p0, S p1, S p2, S p3, S p4, S p5, S p6, S r1, S l1,
                                                      double ds, S h_fore, S h_back, bool back)
 {
-    const NonuniformStencil<S> st = nonuniform_stencil<IEEE>(p0, p1, p2, p3, p4, p5, p6, r1, l1, ds, h_fore, h_back);
+    const NonuniformStencil<S> st = nonuniform_stencil<Q>(p0, p1, p2, p3, p4, p5, p6, r1, l1, ds, h_fore, h_back);
     S x[6], d[5];
 #pragma unroll
     for (int k = 0; k < 6; ++k) x[k] = back ? st.x[k] : st.x[k + 1];
 #pragma unroll
     for (int k = 0; k < 5; ++k) d[k] = back ? st.d[k] : st.d[k + 1];
-    return weno_nonuniform_face<S, IEEE>(x, d, back);
+    return weno_nonuniform_face<S, Q>(x, d, back);
 }
 template <typename S>
 __device__ __noinline__ S weno_nonuniform_one(S p0, S p1, S p2, S p3, S p4, S p5, S p6, S r1, S l1, double ds,

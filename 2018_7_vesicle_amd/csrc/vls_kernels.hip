@@ -605,7 +605,7 @@ __global__ void __launch_bounds__(256) k_upwind_normal(T* __restrict__ nx, T* __
         const double l1 = (a == 0 ? d.l[0] : (a == 1 ? d.l[1] : d.l[2]))[page + o.in];
         double v[7];
         line7_lane(lsf, o.r, o.c, o.p, a, b, v);
-        one[a][t] = weno_nonuniform_one_inl<true>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, ds, 0.0, 0.0,
+        one[a][t] = weno_nonuniform_one_inl<QUOT_IEEE>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, ds, 0.0, 0.0,
                                                   !(fabs(v[4]) < fabs(v[2])));
     });
     __syncthreads();

@@ -291,8 +291,6 @@ __device__ __forceinline__ double min6(const Dists& q)
     return dmin(dmin(q.r[0], q.l[0]), dmin(dmin(q.r[1], q.l[1]), dmin(q.r[2], q.l[2])));
 }
 
-// per-axis derivative pair with the sign-change interface test (re_step.cu:248-269);
-// INL: the nonuniform face inline (see weno_nonuniform_pair_inl)
 // Interface schemes of the fused stage kernels (IFACE_WENO, IFACE_CUBIC of
 // vls_kernels.hpp): the WENO5 path's nonuniform WENO (re_step.cu:79-243,
 // shared_utilities.cup:49-278) or the WENO-RK3 variants' cubic ENO
@@ -337,14 +335,14 @@ __device__ __forceinline__ void reinit_axis_cubic(double& fore, double& back, co
     wenork3_pair(fore, back, v, r1, l1, ds, jp, v[2] * v[3] < 0 || v[3] * v[4] < 0, 0.0, 0.0);
 }
 
-template <bool INL = false>
+// per-axis derivative pair with the sign-change interface test (re_step.cu:248-269);
+// Q: the quotients of the nonuniform faces
+template <int Q>
 __device__ __forceinline__ void reinit_axis(double& fore, double& back, const double v[7], double r1, double l1,
                                             double ds, JPd jp)
 {
     if (v[2] * v[3] < 0 || v[3] * v[4] < 0) {
-        Pair q;
-        if constexpr (INL) q = weno_nonuniform_pair_inl(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, ds, 0.0, 0.0);
-        else q = weno_nonuniform_pair(v, r1, l1, ds, 0.0, 0.0);
+        const Pair q = weno_nonuniform_pair_inl<Q>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, ds, 0.0, 0.0);
         fore = q.fore;
         back = q.back;
     } else {
@@ -992,6 +990,14 @@ __host__ __device__ constexpr int reinit_parts(int depth)
     return defers_crossings<T>() ? (depth + kDeferPages - 1) / kDeferPages : 1;
 }
 
+// the interface lanes' quotients: an FP32 field's differences over distances of
+// at least 1e-6 of a spacing have finite products
+template <typename T>
+constexpr int lane_quot()
+{
+    return sizeof(T) == 8 ? QUOT_WIDE : QUOT_FAST;
+}
+
 // one lane (point, axis) of the reinitialization interface pass
 struct ReinitLane {
     double m = 0.0;   // this axis's Godunov term
@@ -1023,7 +1029,7 @@ __device__ __forceinline__ ReinitLane reinit_iface_lane(const T* __restrict__ fs
         double v[7], fo, bk;
         line7_lane(fs, r, c, p, a, b, v);
         if constexpr (SCHEME == IFACE_CUBIC) reinit_axis_cubic(fo, bk, v, r1, l1, sp[a], inv.jd[a]);
-        else reinit_axis<true>(fo, bk, v, r1, l1, sp[a], inv.jd[a]);
+        else reinit_axis<lane_quot<T>()>(fo, bk, v, r1, l1, sp[a], inv.jd[a]);
         q.m = godunov_axis(q.inside, bk, fo);
     }
     return q;
@@ -1104,7 +1110,7 @@ __device__ __forceinline__ ExtendLane extend_iface_lane(const T* __restrict__ cs
                 eno_cubic_pair(df, db, x, h);
                 dv = fore ? df : db;
             } else {
-                dv = weno_nonuniform_one_inl(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, sp[a], hf, hb, !fore);
+                dv = weno_nonuniform_one_inl<lane_quot<T>()>(v[0], v[1], v[2], v[3], v[4], v[5], v[6], r1, l1, sp[a], hf, hb, !fore);
             }
             q.t = 0.0 + (fore ? vel : dmax(0.0, vel)) * dv;
         } else {

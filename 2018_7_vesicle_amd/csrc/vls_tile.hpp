@@ -891,13 +891,15 @@ __host__ __device__ __forceinline__ int quotient(int n, IntDiv d)
 }
 
 // The shares of a z-march launch: tile columns (nct of them, ntr to a column of
-// the page) and chunks of `len` pages, one more in the first `rem` of them.
-// Computed on the host: a block's first loads wait for its share, and four
-// divisions there (two of them of 64 bits) were 360 instructions.  Advection stage,
-// one page a block: 48^3 FP32 4.26 -> 3.63 us, FP64 5.24 -> 4.61; 96^3 FP32 at 4
-// pages 8.9 -> 8.0, its extension stage 12.05 -> 11.1.
+// the page) and nch chunks of `len` pages, one more in `rem` of them, spread
+// evenly: an XCD takes a contiguous range of chunks (the longer ones first made
+// the first XCDs last, 1% at 200^3).  Computed on the host: a block's first
+// loads wait for its share, and four divisions there (two of them of 64 bits)
+// were 360 instructions.  Advection stage, one page a block: 48^3 FP32 4.26 ->
+// 3.63 us, FP64 5.24 -> 4.61; 96^3 FP32 at 4 pages 8.9 -> 8.0, its extension
+// stage 12.05 -> 11.1.
 struct ZShare {
-    IntDiv nct, ntr;
+    IntDiv nct, ntr, nch;
     int len, rem;
 };
 template <int R>
@@ -906,7 +908,7 @@ inline ZShare zmarch_shares(int rows, int cols, int pges, int depth)
     // equal chunks of at most `depth` pages (a last chunk of a page or two would
     // pay a whole block's start-up)
     const int ntr = tiles_per_col<R>(rows), nch = (pges + depth - 1) / depth;
-    return ZShare{int_div(ntr * tiles_per_row<R>(cols)), int_div(ntr), pges / nch, pges % nch};
+    return ZShare{int_div(ntr * tiles_per_row<R>(cols)), int_div(ntr), int_div(nch), pges / nch, pges % nch};
 }
 // the share of block blk of the launch's nblk = zmarch_blocks(...): tile column
 // (r0, c0) and pages [p0, p1).  Consecutive blocks of one XCD take neighbouring
@@ -919,8 +921,9 @@ __device__ __forceinline__ void zmarch_share(const ZShare& z, int blk, int nblk,
     const int cb = quotient(ct, z.ntr);
     r0 = (ct - cb * z.ntr.d) * R;
     c0 = cb * Shape<R>::TC;
-    p0 = ch * z.len + min(ch, z.rem);
-    p1 = p0 + z.len + (ch < z.rem ? 1 : 0);
+    // rem is 0 at one page a chunk, so nch * rem stays below 65535^2 / 4
+    p0 = ch * z.len + quotient(ch * z.rem, z.nch);
+    p1 = (ch + 1) * z.len + quotient((ch + 1) * z.rem, z.nch);
 }
 
 // blocks of a z-march launch with `depth` pages per block

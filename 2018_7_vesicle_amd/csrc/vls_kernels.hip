@@ -1545,6 +1545,18 @@ static inline ZShare bulk_shares(const Geom& g, int depth)
                               : zmarch_shares<64>(g.rows, g.cols, g.pges, depth);
 }
 
+// as zmarch_depth for the advection stage, whose launch holds no interface list:
+// one page a block while that makes no more than three blocks a CU.  (The other
+// stages of such boxes wait for their lists whatever the depth.)  Measured on
+// MI355X, two pages -> one: 24^3 FP64 3.9 -> 3.2 us, FP32 3.4 -> 2.8; 40^3 4.0 -> 3.85
+// and 3.55 -> 3.15; 52^3 (728 blocks) 5.2 -> 4.75 and 3.85 -> 3.7; 56^3 (784) 5.3 ->
+// 5.4 and 3.9 -> 4.1.
+static int advect_depth(const Geom& g)
+{
+    if (g.zd > 0) return zmarch_depth(g);
+    return bulk_blocks(g, 1) <= 3 * device_cus() ? 1 : zmarch_depth(g);
+}
+
 template <typename T>
 hipError_t launch_set_mask_bit(uint8_t* flags, const T* F, const Geom& g, hipStream_t s)
 {
@@ -1714,7 +1726,7 @@ template <typename T>
 hipError_t launch_advect_stage(T* out, const T* fs, const T* fn, const T* vx, const T* vy, const T* vz, double dt,
                                const Geom& g, int stage, hipStream_t s)
 {
-    const int zd = zmarch_depth(g);
+    const int zd = advect_depth(g);
     const ZShare zs = bulk_shares(g, zd);
     if (tile_rows(g) == 32)
         k_advect_stage<32, T><<<dim3(bulk_blocks(g, zd)), dim3(256), 0, s>>>(out, fs, fn, vx, vy, vz, dt, box_of(g),

@@ -266,7 +266,8 @@ int vls_sdf3_set_tile_rows(vls_sdf3_t h, int tile_rows);
  * box size, so that the blocks are resident together); results do not depend
  * on it */
 int vls_sdf3_set_zmarch_depth(vls_sdf3_t h, int depth);
-/* the tile rows and z-march depth the bulk stage kernels launch with */
+/* the tile rows and z-march depth the bulk stage kernels launch with (the
+ * advection of a small box by default with a depth of 1) */
 int vls_sdf3_get_launch(vls_sdf3_t h, int *tile_rows, int *depth);
 
 /* setDistance (+SD/@SDF3/setDistance.m:3-21): subcell distances of F with the

@@ -369,3 +369,18 @@ def test_default_launch_shape_gives_same_results(box, dtype):
                      m.WENO5RK3Advection(m.F, *[T(c) for c in u], 0.01, 2)))
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("pges", [48, 49])
+def test_advection_depth_of_small_boxes_gives_same_results(pges, dtype):
+    """the last box whose advection takes one page a block (768 blocks on 256
+    CUs) and the first that takes more, against chunks of three pages"""
+    ax = [(np.arange(k) - (k - 1) / 2) * 0.1 for k in (64, 64, pges)]
+    g = cases.Grid(*ax)
+    T = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to("cuda", dtype)  # noqa: E731
+    m = vls.SDF3(vls.GD3(*ax), T(cases.star_phi0(g)))
+    u = [T(c) for c in cases.smooth_velocity(g)]
+    out = m.WENO5RK3Advection(m.F, *u, 0.01, 2)
+    m.setZmarchDepth(3)
+    assert torch.equal(out, m.WENO5RK3Advection(m.F, *u, 0.01, 2))

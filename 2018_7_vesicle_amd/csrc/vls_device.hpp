@@ -274,7 +274,7 @@ __device__ __forceinline__ void weno5_pair(S& d_fore, S& d_back, const S p[7], J
 // (ZDiff) and the buffer addressing of the march (Page) the FP32 extension
 // loop has 140 VALU instructions a point instead of 159 and the
 // reinitialization loop 218 instead of 240; both stages are bound by them.
-// Measured on MI355X at 256^3: 94.9 -> 92.0 and 112.6 -> 106.7 us a stage.
+// At 256^3 the stages take 94 and 112 us in the vesicle-step pipeline (MI355X).
 __device__ __forceinline__ float jp_weights(float z, float r1, float x2)
 {
     return __builtin_amdgcn_rcpf(fmaf(0.25f, z, fmaf(0.5f, x2, fmaf(r1, r1, 0x1p-125f))));

@@ -309,7 +309,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kStage
 }
 
 template <int R, typename T>
-__global__ void __launch_bounds__(256) kb_advect_stage(T* __restrict__ out, const T* __restrict__ fs,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAdvectWaves, kAdvectWaves))) kb_advect_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                        const T* __restrict__ fn, const T* __restrict__ vx,
                                                        const T* __restrict__ vy, const T* __restrict__ vz,
                                                        const double* __restrict__ dt, BatchView B, int stage)

@@ -907,7 +907,7 @@ __global__ void __launch_bounds__(256) k_advection_step(double* __restrict__ ast
 
 // fused TVD-RK3 advection stage: out = combine(fs - dt*L(fs), fn), plane tiles
 template <int R, typename T>
-__global__ void __launch_bounds__(256) k_advect_stage(T* __restrict__ out, const T* __restrict__ fs,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kAdvectWaves, kAdvectWaves))) k_advect_stage(T* __restrict__ out, const T* __restrict__ fs,
                                                       const T* __restrict__ fn, const T* __restrict__ vx,
                                                       const T* __restrict__ vy, const T* __restrict__ vz,
                                                       double dt, Box b, Inv inv, int stage, ZShare zs)

@@ -741,6 +741,13 @@ __device__ __forceinline__ void line5s(const double* __restrict__ f, const Box& 
 // interface lanes spill 100 bytes: the batch of 96 FP32 grids of 32..96 runs
 // 58.9 ms a step with 5 waves and 56.6 ms with 4, 256^3 is equal.
 constexpr int kStageWaves = 4;
+// The advection stages have no interface lanes.  Left to itself the compiler aims
+// at 8 waves a SIMD (51 VGPRs in FP32, 80 in FP64) and puts a page's chains one
+// behind the other, which small boxes wait for.  Measured on MI355X without -> at 6
+// waves: 60 stages of 4 grids of 32^3 FP32 449 -> 426 us, of 8 odd grids 578 -> 498,
+// FP64 795 -> 758; a stage of 160^3 FP32 23.7 -> 22.3, 200^3 FP64 86.8 -> 85.4.
+// 5 waves lose 2-6% of small FP64 stages, 7 spill in FP64 (926 for the odd grids).
+constexpr int kAdvectWaves = 6;
 
 // ---------------------------------------------------------------------------
 // z-marching walk (single grid): a block takes one tile column (TR rows x TC
